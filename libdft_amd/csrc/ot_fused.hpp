@@ -358,20 +358,41 @@ struct MidProg {
 #endif
 template <typename T, int N> using MidCfg = ColCfg<T, N, DFT_XMID_EM, DFT_XMID_COLS>;
 // minimum resident blocks per CU asked of the register allocator (0: none)
-#ifndef DFT_XMID_ORDER
-#define DFT_XMID_ORDER 0
-#endif
 #ifndef DFT_XMID_MINB
 #define DFT_XMID_MINB 0
 #endif
 template <typename T> constexpr int mid_minb() { return sizeof(T) == 4 ? DFT_XMID_MINB : 0; }
 
 // Blocks of the x-middle pass: ny * ntile tiles of COLS consecutive kz < P-1
-// at one ky, then ceil(ny / COLS) tiles of the Nyquist column kz = P-1 over
-// COLS consecutive ky.
+// at one ky, and ceil(ny / COLS) tiles of the Nyquist column kz = P-1 over COLS
+// consecutive ky.  A Nyquist tile touches one value per row, a cache line per
+// lane, and takes several times as long as the others: these tiles go first,
+// dealt over the XCDs by the plain block order, so that they overlap the rest
+// instead of ending the launch alone (last, at 256^3 FP32: single-term outputs
+// 305 us, accumulating 141, derivative program 216; first: 252, 105, 184).
 template <int COLS> __host__ __device__ inline int mid_tiles(int P) { return (P - 1 + COLS - 1) / COLS; }
 template <int COLS> __host__ __device__ inline int mid_blocks(int ny, int P) {
   return ny * mid_tiles<COLS>(P) + (ny + COLS - 1) / COLS;
+}
+// Output m (of nl) and column of lane `col` of this block, for a grid of
+// mid_blocks * nl blocks.  Past the Nyquist tiles, consecutive logical blocks
+// (the outputs of a tile, the tiles of one ky) are on one XCD, back to back.
+struct MidCol {
+  int m, o, kz;
+  bool act;  // out-of-range lanes read an in-range column and store nothing
+};
+template <int COLS> __device__ __forceinline__ MidCol mid_col(int ny, int P, int nl, int col) {
+  const int nyq = (ny + COLS - 1) / COLS * nl, ntile = mid_tiles<COLS>(P);
+  int i = blockIdx.x;
+  if (i < nyq) {
+    const int t = i / nl, r = t * COLS + col;
+    return {i - t * nl, r < ny ? r : ny - 1, P - 1, r < ny};
+  }
+  i -= nyq;
+  const int n = gridDim.x - nyq;
+  const int L = (n & 7) == 0 ? (i & 7) * (n >> 3) + (i >> 3) : i, b = L / nl;
+  const int o = b / ntile, c = (b - o * ntile) * COLS + col;
+  return {L - b * nl, o, c < P - 1 ? c : P - 2, c < P - 1};
 }
 
 // Spectra are [nx][ny][PP] (P values per row) after the y pass; the x line
@@ -388,26 +409,10 @@ __global__ void __launch_bounds__((MidCfg<T, N>::BS), mid_minb<T>()) k_xmid(cons
   constexpr int E = G::E, TPL = G::TPL, COLS = G::COLS, LP = G::LP;
   __shared__ C s_x[G::S > 1 ? COLS * LP : 1];
   __shared__ C s_tw[rf::tw_len<T, N>()];
-  // DFT_XMID_ORDER 0: consecutive tiles (one ky) on one XCD, back to back
-  // (shared L2 lines); 1: ky fastest, so that the blocks in flight spread over
-  // whole x-planes
-  const int b = DFT_XMID_ORDER == 0 ? rf::xcd_block() : (int)blockIdx.x;
   const int col = threadIdx.x % COLS, t = threadIdx.x / COLS;
-  const int ntile = mid_tiles<COLS>(P);
-  int o, kz;
-  bool act;
-  if (b < ny * ntile) {
-    const int tile = DFT_XMID_ORDER == 0 ? b % ntile : b / ny;
-    o = DFT_XMID_ORDER == 0 ? b / ntile : b % ny;
-    const int c = tile * COLS + col;
-    act = c < P - 1;
-    kz = act ? c : P - 2;  // out-of-range lanes read an in-range column and store nothing
-  } else {
-    const int r = (b - ny * ntile) * COLS + col;
-    act = r < ny;
-    o = act ? r : ny - 1;
-    kz = P - 1;
-  }
+  const MidCol mc = mid_col<COLS>(ny, P, 1, col);
+  const int o = mc.o, kz = mc.kz;
+  const bool act = mc.act;
   const uint32_t es = (uint32_t)ny * PP;
   const uint32_t e0 = (uint32_t)o * PP + kz + t * es;  // element index of point t
   const uint32_t obC = e0 * (uint32_t)sizeof(C), obR = e0 * (uint32_t)sizeof(T);
@@ -551,23 +556,10 @@ __global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DF
   __shared__ C s_x[G::S > 1 ? COLS * LP : 1];
   __shared__ C s_tw[rf::tw_len<T, N>()];
   // outputs m0 .. m0 + nl - 1 of the program
-  const int L = rf::xcd_block();
-  const int b = L / nl, m = m0 + (L - b * nl);
   const int col = threadIdx.x % COLS, t = threadIdx.x / COLS;
-  const int ntile = mid_tiles<COLS>(P);
-  int o, kz;
-  bool act;
-  if (b < ny * ntile) {
-    o = b / ntile;
-    const int c = (b - o * ntile) * COLS + col;
-    act = c < P - 1;
-    kz = act ? c : P - 2;  // out-of-range lanes read an in-range column and store nothing
-  } else {
-    const int r = (b - ny * ntile) * COLS + col;
-    act = r < ny;
-    o = act ? r : ny - 1;
-    kz = P - 1;
-  }
+  const MidCol mc = mid_col<COLS>(ny, P, nl, col);
+  const int o = mc.o, kz = mc.kz, m = m0 + mc.m;
+  const bool act = mc.act;
   const uint32_t es = (uint32_t)ny * PP;
   const uint32_t e0 = (uint32_t)o * PP + kz + t * es;  // element index of point t
   const uint32_t obC = e0 * (uint32_t)sizeof(C), obR = e0 * (uint32_t)sizeof(T);
