@@ -369,18 +369,17 @@ template <typename T> __global__ void k_scale_psi(cplx<T> *psi, const double *f,
 // Fused x pass of the propagator: forward x FFT, kinetic phase
 // exp(-i k^2 dt / 2M), inverse x FFT.  Field is [nx][ny][nz] complex.
 // The phase factorises as X(kx) YZ(ky, kz); both factors are evaluated in FP64
-// (X once per block, in LDS), multiplied in FP64, and in FP32 applied as the
-// rounded value plus its residual, so that its modulus is exact: a phase of
-// the same mode is applied every step, and a rounded one would change that
-// mode's amplitude by the same factor every time.
+// (X once per block, in LDS) and applied in FP64 between the FP64 stages of
+// rfft_apply, so that its modulus is exact and one rounding separates the
+// coefficients before it from those after it.
 // Geometry: at least DFT_XKIN_COLS columns per block (N = 512 keeps the
 // column default).
 #ifndef DFT_XKIN_COLS
 #define DFT_XKIN_COLS 8
 #endif
-// waves per SIMD asked of the register allocator (0: no request): at 3 the
-// FP32 pass fits 168 VGPRs with 28 bytes per lane of spills and runs 70 -> 58 us
-// at 256^3 (178 VGPRs and 2 waves without); more waves do not fit its LDS.
+// waves per SIMD asked of the register allocator (0: no request); more waves do
+// not fit the LDS.  256^3 FP32: 66 us, 156 VGPRs (with FP32 stages around the
+// phase, which took 168 VGPRs and spilled: 69 us).
 #ifndef DFT_XKIN_MINB
 #define DFT_XKIN_MINB 3
 #endif
@@ -421,27 +420,16 @@ __global__ void __launch_bounds__((KinCfg<T, N>::BS), sizeof(T) == 4 ? DFT_XKIN_
     const double m = exp(K * dti);
     s_kx[e] = make_double2(m * c, -m * s);
   }
-  __syncthreads();
-  rf::rfft<T, N, G::EM, -1, rf::BlockSync>(v, s_x + col * LP, s_tw, t);
   const double my = (double)(o < ny / 2 ? o : o - ny) - oy;
   const double mz = (double)(cc < nz / 2 ? cc : cc - nz) - oz;
   const double Kyz = cy * (my * my) + cz * (mz * mz);
   double sy, cyz;
   sincos(Kyz * dtr, &sy, &cyz);
   const double myz = exp(Kyz * dti);
-  const double yr = myz * cyz, yi = -myz * sy;
-#pragma unroll
-  for (int i = 0; i < E; ++i) {
-    const double2 x = s_kx[t + TPL * i];
-    const double pr = x.x * yr - x.y * yi, pi = x.x * yi + x.y * yr;
-    if constexpr (sizeof(T) == 4) {
-      const float hr = (float)pr, hi = (float)pi;
-      v[i] = cmul_hl_phase(v[i], make_float2(hr, hi), make_float2((float)(pr - hr), (float)(pi - hi)));
-    } else {
-      v[i] = cmul(v[i], cmk<C>(pr, pi));
-    }
-  }
-  rf::rfft<T, N, G::EM, +1, rf::BlockSync>(v, s_x + col * LP, s_tw, t);
+  const double2 yz = make_double2(myz * cyz, -myz * sy);
+  __syncthreads();
+  rf::rfft_apply<T, N, G::EM, rf::BlockSync>(v, s_x + col * LP, s_tw, t,
+                                             [&](int e, double2 u) { return cmul(u, cmul(s_kx[e], yz)); });
   if (act) {
 #pragma unroll
     for (int i = 0; i < E; ++i) gst<C>((char *)psi + (size_t)i * st, ob, v[i]);
