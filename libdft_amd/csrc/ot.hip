@@ -1193,6 +1193,12 @@ template <typename T, int N> void launch_zA(bool BF, const cplx<T> *psi, T *rho,
 #define DFT_XMID_KIND 3
 #endif
 
+// Whether summed outputs without derivative terms take k_xconv (any number of kernels).
+template <typename T> constexpr bool xconv_sums(int nx) {
+  return ((DFT_XMID_KIND == 1 || DFT_XMID_KIND == 2) && sizeof(T) == 4) ||
+         (DFT_XMID_KIND == 3 && (sizeof(T) == 4 || nx <= 256));
+}
+
 template <typename T, int N, int NK, bool DV>
 void launch_xmid1(const fused::MidProg *pg, int ny, int P, int PP, const cplx<T> *tw, hipStream_t s) {
   using Cfg = fused::MidCfg<T, N>;
@@ -1239,8 +1245,7 @@ void launch_xmid(const fused::MidProg *pg, const fused::MidProg &hp, int ny, int
   DFT_PROF_BEGIN(s);
   bool one = true;
   for (int m = 0; m < hp.nout; ++m) one = one && hp.o[m].nterms == 1;
-  if constexpr (((DFT_XMID_KIND == 1 || DFT_XMID_KIND == 2) && sizeof(T) == 4) ||
-                (DFT_XMID_KIND == 3 && (sizeof(T) == 4 || N <= 256))) {
+  if constexpr (xconv_sums<T>(N)) {
     // per-output blocks unless the program shares inputs between
     // multi-term outputs with derivative symbols (J_d and T1 = F sum_d D_d G_d)
     if (one || !deriv || DFT_XMID_KIND == 2) {
@@ -1415,6 +1420,13 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
 
   // ---- stage A: psi -> {rho, q_d, q4, [rho~]}, forward z and y
   const bool HB = BF && pw.bfhd;
+  // Re V_BF holds C = U*q4 linearly, -m/2 c_bf C, unless it is clamped or multiplied
+  // by the switch's d(G rho)/d rho: then C joins the linear terms that stage C sums
+  // in k space and its inverse transform is saved (256^3: 2135 -> 2122 us per FP32
+  // step, 4204 -> 4090 FP64).  On small grids the longer chain of the summing
+  // pass costs as much as is saved (128^3 FP32: 722 and 724 us; 32x32x64: 92.0 and
+  // 92.8).
+  const bool csum = BF && !HB && !pw.clamp_bf && n > ((int64_t)1 << 21) && xconv_sums<T>(d->nx);
   const int nA = BF ? (HB ? 6 : 5) : 1;
   fused::Ptrs8 oA{};
   for (int i = 0; i < nA; ++i) oA.p[i] = d->slot[SP0 + i];
@@ -1441,7 +1453,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     if (KC) add(0, K_F);
     if (BF) {
       add(HB ? 5 : 0, K_U);
-      for (int i = 1; i <= 4; ++i) add(i, K_U);
+      for (int i = 1; i <= (csum ? 3 : 4); ++i) add(i, K_U);
     }
     setk(pg);
     nB = pg.nout;
@@ -1524,16 +1536,21 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
   // ---- stage C: linear terms summed in k space, z^-1, accumulate or start the step
   {
     fused::MidProg pg = new_prog();
-    pg.nin = KC ? 3 : 2;
+    pg.nin = 2;
     pg.in[0] = d->slot[SP0];
     pg.in[1] = d->slot[Q4];
-    pg.in[2] = d->slot[SH];
     pg.nout = 1;
     pg.multi = 0;
-    pg.o[0].nterms = KC ? 3 : 2;
     pg.o[0].t[0] = mterm(0, K_LJ, -1, h3N);
     pg.o[0].t[1] = mterm(1, K_SA, -1, h3N);
-    pg.o[0].t[2] = mterm(2, K_F, -1, h3N * otf->kc_coef23 * otf->alpha_s / (2.0 * otf->mass));
+    auto add = [&](void *in, int kern, double scale) {
+      pg.in[pg.nin] = in;
+      pg.o[0].t[pg.nin] = mterm(pg.nin, kern, -1, scale);
+      ++pg.nin;
+    };
+    if (KC) add(d->slot[SH], K_F, h3N * otf->kc_coef23 * otf->alpha_s / (2.0 * otf->mass));
+    if (csum) add(d->slot[SP4], K_U, -0.5 * h3N * otf->mass * otf->c_bfpot);
+    pg.o[0].nterms = pg.nin;
     pg.o[0].out = d->slot[TMP4];
     setk(pg);
     DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(mid_prog(d, 2, pg, s), pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));

@@ -336,10 +336,10 @@ struct MidTerm {
 };
 struct MidOut {
   int nterms, pad;
-  MidTerm t[3];
+  MidTerm t[4];
   void *out;
 };
-constexpr int kMidMaxIn = 6, kMidMaxOut = 8, kMidMaxKern = 3;
+constexpr int kMidMaxIn = 6, kMidMaxOut = 8, kMidMaxKern = 4;
 struct MidProg {
   int nin, nout, multi, nkern;
   const void *in[kMidMaxIn];
@@ -718,7 +718,7 @@ __device__ __forceinline__ void c2r_pipe(rf::Regs<T, N, pair_em<N>()> &v, fft::R
   rf::rfft<T, N, pair_em<N>(), +1, PairSync<N>>(v, X, tw, t);
 }
 struct ZABArgs {
-  Ptrs8 in;       // rhobar, [rhot], [A, Bx, By, Bz, C]
+  Ptrs8 in;       // rhobar, [rhot], [A, Bx, By, Bz, C] (C null: its term is summed in k space, see fused_impl)
   Ptrs8 out;      // Q, [G_x, G_y, G_z]
   const void *rho, *psi;
   void *rhot, *vre, *vim, *wx, *wy, *wz;
@@ -799,7 +799,8 @@ __device__ __forceinline__ void zAB_body(ZABArgs a, int64_t npairs, int P, PW<T>
         for (int i = 0; i < E; ++i)
 #pragma unroll
           for (int w = 0; w < 2; ++w) vg(w, i, vds[w][i], gis[w][i]);
-      c2r(a.in.p[IA + 1 + D], a.in.p[IA + 2 + D]);
+      const void *next = D < 2 || a.in.p[IA + 4] ? a.in.p[D < 2 ? IA + 2 + D : IA + 4] : (DO_LOCAL ? a.in.p[0] : nullptr);
+      c2r(a.in.p[IA + 1 + D], next);
       if constexpr ((PF & 1) == 0) qq = q.here();
       T Wv[2][E];
 #pragma unroll
@@ -833,12 +834,14 @@ __device__ __forceinline__ void zAB_body(ZABArgs a, int64_t npairs, int P, PW<T>
     axis(std::integral_constant<int, 0>{});
     axis(std::integral_constant<int, 1>{});
     axis(std::integral_constant<int, 2>{});
-    c2r(a.in.p[IA + 4], DO_LOCAL ? a.in.p[0] : nullptr);
+    const void *C_ = a.in.p[IA + 4];
+    if (C_) c2r(C_, DO_LOCAL ? a.in.p[0] : nullptr);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
-        T re = tr[w][i] + part(v[i], w);
+        T re = tr[w][i];
+        if (C_) re += part(v[i], w);
         if constexpr (HB) re = re * dg[w][i];
         re = re * ((T)-0.5 * pw.mass);
         if (pw.clamp_bf) re = clampv(re, pw.bfmax);

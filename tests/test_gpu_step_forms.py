@@ -1,0 +1,74 @@
+"""Forms that the fused step chooses between, against the FP64 device path's
+unfused potential or the oracle at the sizes where the choice changes."""
+import numpy as np
+import pytest
+
+import libdft_amd as L
+from oracle import pyoracle as po
+from tests import inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", [L.GRID_FP64, L.GRID_FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("cbf", [1.0, 0.5], ids=["cbf1", "cbf05"])
+@pytest.mark.parametrize("shape", [(128, 128, 128), (256, 128, 128), (64, 512, 128)], ids=lambda s: "x".join(map(str, s)))
+def test_potential_forms_agree(shape, cbf, prec):
+    """dft_ot_potential (U*q4 summed in k space above 2^21 points, transformed by
+    itself up to there) against dft_ot_potential2 on the same density and
+    velocities, which always transforms it: FP64 to rounding, FP32 to 2e-5 of the
+    largest value (the bound of the potential tests)."""
+    step = 0.8
+    lib = L.lib()
+    w = L.Wave(shape, step, prec)
+    f = L.Functional(9, w, 2, 4)
+    f.p.c_bfpot = cbf
+    w.set(inputs.smooth_modulated(shape, step, f.p.rho0, 0.3))
+    a, b = L.CField(shape, step, prec), L.CField(shape, step, prec)
+    f.potential(a)
+    rho, v = L.RField(shape, step, prec), [L.RField(shape, step, prec) for _ in range(3)]
+    lib.grid_wf_density(w.h, rho.h)
+    lib.grid_wf_velocity(w.h, v[0].h, v[1].h, v[2].h, L.DFT_EPS)
+    lib.dft_ot_potential2(f.h, b.h, rho.h, v[0].h, v[1].h, v[2].h)
+    got, want = a.get(), b.get()
+    for g, x in ((got.real, want.real), (got.imag, want.imag)):
+        assert np.abs(g - x).max() <= (1e-12 if prec == L.GRID_FP64 else 2e-5) * np.abs(want).max()
+    for x in (a, b, rho, *v, f, w):
+        x.free()
+
+
+@pytest.mark.parametrize("prec", [L.GRID_FP64, L.GRID_FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("shape", [(4, 8, 16), (8, 4, 64), (16, 16, 8), (32, 8, 4), (64, 4, 16), (128, 8, 8), (256, 4, 8),
+                                   (512, 8, 4)], ids=lambda s: "x".join(map(str, s)))
+def test_propagation_every_x_length(shape, prec):
+    """grid_wf_propagate at every length of the x axis (the kinetic pass and its
+    mirrored inverse) against the oracle, in real and imaginary time."""
+    step = 0.7
+    psi = inputs.smooth_modulated(shape, step, 3e-3, 0.3)
+    x = inputs.splitmix64_uniform(int(np.prod(shape)) * 2, 7).reshape(shape + (2,))
+    psi = psi * (1 + 0.1 * (x[..., 0] + 1j * x[..., 1]))
+    V = 1e-4 * (x[..., 1] + 0.3j * x[..., 0])
+    for dt in (150.0, -90j):
+        w, p = L.Wave(shape, step, prec), L.CField(shape, step, prec)
+        w.set(psi), p.set(V)
+        L.lib().grid_wf_propagate(w.h, p.h, L.Complex.of(dt))
+        want = po.propagate(psi, V, dt, step)
+        assert np.abs(w.get() - want).max() <= (1e-12 if prec == L.GRID_FP64 else 5e-6) * np.abs(want).max()
+        w.free(), p.free()
+
+
+@pytest.mark.parametrize("model", [0, 1, 9], ids=["plain", "kc", "full"])
+@pytest.mark.parametrize("shape", [(8, 4, 16), (16, 8, 4), (64, 16, 32), (32, 64, 128)], ids=lambda s: "x".join(map(str, s)))
+def test_potential_nyquist_tiles(shape, model):
+    """The x-middle's Nyquist tiles where ny is below, at and above a tile's columns,
+    and grids whose tile count is no multiple of 8, against the oracle (FP64)."""
+    step = 1.1
+    o = po.OracleOT(model, shape, step, 2, 4)
+    psi = inputs.smooth_modulated(shape, step, o.p.rho0, 0.3)
+    w = L.Wave(shape, step, L.GRID_FP64)
+    w.set(psi)
+    f, p = L.Functional(model, w, 2, 4), L.CField(shape, step, L.GRID_FP64)
+    f.potential(p)
+    want = o.potential(psi)
+    assert np.abs(p.get() - want).max() <= 1e-10 * np.abs(want).max()
+    p.free(), f.free(), w.free()
