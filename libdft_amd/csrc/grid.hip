@@ -28,6 +28,10 @@ void *dmalloc(size_t bytes) {
   void *p = nullptr;
   if (bytes == 0) bytes = 16;
   hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess && trim_workspaces()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, bytes);
+  }
   if (e != hipSuccess) {
     fprintf(stderr, "libdft: hipMalloc(%zu) failed: %s\n", bytes, hipGetErrorString(e));
     return nullptr;

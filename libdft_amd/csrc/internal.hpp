@@ -9,6 +9,9 @@ namespace dft {
 hipStream_t lib_stream();
 void *dmalloc(size_t bytes);
 void dfree(void *p);
+// Gives back the work spaces that functionals keep between calls and nobody is
+// using; true if any was.
+bool trim_workspaces();
 
 // ------------------------------------------------------------------ FFT ----
 template <typename T> struct Plan3D {

@@ -17,8 +17,10 @@
 // reference.  The derivative kernels dF_d are never stored: their spectra
 // are F^ * i sin(k_d h)/h, the symbol of the periodic central difference
 // the reference applies to F before transforming (src/ot.c:196).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "ideal_gas.hpp"
@@ -898,6 +900,8 @@ struct dft_ot_device {
   double *norm_part;         // per-block sums |psi|^2 and the factor of a renormalising step
   double *igtab;             // pow(k, s) table of the ideal Bose gas (thermal models), or null
   double ig_g1;              // and its g_{3/2}(1)
+  void *adj;                 // AdjWork of the reverse passes, kept between calls (or null)
+  bool adj_busy;             // a call is working with it
   // x-middle programs of the fused schedule in device memory, and the host
   // copies they were uploaded from (re-uploaded only when one changes)
   fused::MidProg *mid_dev;
@@ -1803,9 +1807,12 @@ template <typename T> bool build_kernels(dft_ot_functional *otf, int min_sub, in
   return true;
 }
 
+void free_adj(dft_ot_device *d);
+
 void free_device(dft_ot_device *d) {
   if (!d) return;
   DFT_HIP_CHECK(hipStreamSynchronize(lib_stream()));
+  free_adj(d);
   for (int i = 0; i < NSLOT; ++i) dfree(d->slot[i]);
   for (int i = 0; i < 4; ++i) dfree(d->kern[i]);
   dfree(d->phase);
@@ -1892,7 +1899,9 @@ bool check_r(dft_ot_functional *otf, rgrid *g, const char *fn) {
 
 // -------------------------------------------------------- adjoint sweep --
 // Work space of the reverse pass: real fields, complex fields and half spectra,
-// and for backflow models the fields of the backflow transpose.
+// for backflow models the fields of the backflow transpose, and the sweep's
+// adjoint state, running state and well; one allocation.  `states` holds a
+// sweep's checkpoints and segment.
 template <typename T> struct AdjWork {
   int64_t n = 0, nh = 0;
   bool bf = false;
@@ -1900,33 +1909,114 @@ template <typename T> struct AdjWork {
   T *b[20] = {};
   cplx<T> *c[4] = {};
   cplx<T> *spec[10] = {};
+  cplx<T> *psib = nullptr, *cur = nullptr;
+  T *well = nullptr;
   double *pa = nullptr, *pw = nullptr;
+  void *slab = nullptr;
+  cplx<T> *states = nullptr;
+  int64_t nstates = 0;
+  size_t slab_bytes = 0;
+  size_t bytes() const { return slab_bytes + sizeof(cplx<T>) * (size_t)n * nstates; }
   bool alloc(int64_t n_, int64_t nh_, bool with_bf) {
     n = n_;
     nh = nh_;
     bf = with_bf;
-    for (auto &x : r)
-      if (!(x = (T *)dmalloc(sizeof(T) * n))) return false;
-    if (bf)
-      for (auto &x : b)
-        if (!(x = (T *)dmalloc(sizeof(T) * n))) return false;
-    for (auto &x : c)
-      if (!(x = (cplx<T> *)dmalloc(sizeof(cplx<T>) * n))) return false;
-    for (auto &x : spec)
-      if (!(x = (cplx<T> *)dmalloc(sizeof(cplx<T>) * nh))) return false;
-    pa = (double *)dmalloc(sizeof(double) * red_blocks(n));
-    pw = (double *)dmalloc(sizeof(double) * red_blocks(n));
-    return pa && pw;
+    size_t off = 0;
+    // two rounds: sizes, then pointers
+    for (int round = 0; round < 2; ++round) {
+      auto take = [&](auto &p, size_t elems) {
+        using P = std::remove_reference_t<decltype(p)>;
+        if (round) p = (P)((char *)slab + off);
+        off += (sizeof(*p) * elems + 255) & ~(size_t)255;
+      };
+      off = 0;
+      for (auto &x : r) take(x, n);
+      if (bf)
+        for (auto &x : b) take(x, n);
+      for (auto &x : c) take(x, n);
+      for (auto &x : spec) take(x, nh);
+      take(psib, n);
+      take(cur, n);
+      take(well, n);
+      take(pa, red_blocks(n));
+      take(pw, red_blocks(n));
+      if (!round && !(slab = dmalloc(slab_bytes = off))) return false;
+    }
+    return true;
+  }
+  bool alloc_states(int64_t k) {
+    if (k <= nstates) return true;
+    dfree(states);
+    nstates = 0;
+    if (!(states = (cplx<T> *)dmalloc(sizeof(cplx<T>) * n * k))) return false;
+    nstates = k;
+    return true;
   }
   void release() {
-    for (auto &x : r) dfree(x);
-    for (auto &x : b) dfree(x);
-    for (auto &x : c) dfree(x);
-    for (auto &x : spec) dfree(x);
-    dfree(pa);
-    dfree(pw);
+    dfree(slab);
+    dfree(states);
+    *this = AdjWork<T>();
   }
 };
+
+// The work space stays with its functional between calls (a reverse pass of a
+// 128^3 potential takes 1.3 ms, the allocations and frees of its ~55 fields took
+// 15 ms): up to kAdjKeep bytes, given back by dft_ot_free and when an allocation
+// of the library fails (trim_workspaces).  A call that finds it taken by another
+// thread works with one of its own.
+constexpr size_t kAdjKeep = (size_t)16 << 30;
+std::mutex g_adj_mu;                    // guards dft_ot_device::adj, adj_busy and g_adj_devs
+std::vector<dft_ot_device *> g_adj_devs;  // functionals that keep a work space
+
+template <typename T> void drop_adj(dft_ot_device *d) {  // g_adj_mu held
+  ((AdjWork<T> *)d->adj)->release();
+  delete (AdjWork<T> *)d->adj;
+  d->adj = nullptr;
+  g_adj_devs.erase(std::find(g_adj_devs.begin(), g_adj_devs.end(), d));
+}
+
+template <typename T> struct AdjLease {
+  dft_ot_device *d;
+  AdjWork<T> *w;
+  bool ok;
+  AdjLease(dft_ot_device *d_, bool bf) : d(d_), w(nullptr) {
+    {
+      std::lock_guard<std::mutex> lk(g_adj_mu);
+      if (d->adj && !d->adj_busy) {
+        w = (AdjWork<T> *)d->adj;
+        d->adj_busy = true;
+      }
+    }
+    ok = w != nullptr;
+    if (!ok) {
+      w = new AdjWork<T>();
+      ok = w->alloc(d->n, (int64_t)d->nx * d->ny * d->PP, bf);
+    }
+  }
+  AdjLease(const AdjLease &) = delete;
+  ~AdjLease() {
+    DFT_HIP_CHECK(hipStreamSynchronize(lib_stream()));
+    std::lock_guard<std::mutex> lk(g_adj_mu);
+    const bool keep = ok && w->bytes() <= kAdjKeep;
+    if (d->adj == w) {
+      d->adj_busy = false;
+      if (!keep) drop_adj<T>(d);
+    } else if (keep && !d->adj) {
+      d->adj = w;
+      g_adj_devs.push_back(d);
+    } else {
+      w->release();
+      delete w;
+    }
+  }
+};
+
+void free_adj(dft_ot_device *d) {
+  std::lock_guard<std::mutex> lk(g_adj_mu);
+  if (!d->adj) return;
+  if (d->prec == GRID_FP32) drop_adj<float>(d);
+  else drop_adj<double>(d);
+}
 
 // Real fields of the work space.
 enum { AQB, ALV, AHP, ARP, ARBB, AT1B, APB, AJB = APB + 3, AGB = AJB + 3, ARSB = AGB + 3, AGBAR, ACONV = AGBAR + 3,
@@ -2180,23 +2270,17 @@ int adjoint_sweep(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu, do
   const int64_t n = d->n;
   const size_t bytes = sizeof(cplx<T>) * n;
   const int64_t ncp = (K + every - 1) / every;
-  std::vector<cplx<T> *> cp(ncp, nullptr), seg(every, nullptr);
-  bool ok = true;
-  for (auto &x : cp) ok = ok && (x = (cplx<T> *)dmalloc(bytes)) != nullptr;
-  for (auto &x : seg) ok = ok && (x = (cplx<T> *)dmalloc(bytes)) != nullptr;
-  wf *cur = grid_wf_clone(gwf, (char *)"adjoint state");
-  rgrid *vext = rgrid_clone(otf->density, (char *)"adjoint well");
-  auto cleanup = [&]() {
-    DFT_HIP_CHECK(hipStreamSynchronize(s));
-    for (auto x : cp) dfree(x);
-    for (auto x : seg) dfree(x);
-    if (cur) grid_wf_free(cur);
-    if (vext) rgrid_free(vext);
-  };
-  if (!ok || !cur || !vext) {
-    cleanup();
-    return -1;
-  }
+  if (!w.alloc_states(ncp + every)) return -1;
+  auto cp = [&](int64_t i) { return w.states + i * n; };
+  auto seg = [&](int64_t i) { return w.states + (ncp + i) * n; };
+  // the running state and the well, on the work space's fields
+  cgrid cg = *gwf->grid;
+  cg.dev = w.cur;
+  wf cw = *gwf, *cur = &cw;
+  cw.grid = &cg;
+  cw.cworkspace = nullptr;
+  rgrid vg = *otf->density, *vext = &vg;
+  vg.dev = w.well;
   hipLaunchKernelGGL(k_well<T>, dim3(grid_for(n)), dim3(kBlock), 0, s, (T *)vext->dev, wl, n);
   DFT_LAUNCH_CHECK();
   REAL_COMPLEX dt;
@@ -2208,7 +2292,7 @@ int adjoint_sweep(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu, do
   DFT_HIP_CHECK(hipMemcpyAsync(cur->grid->dev, gwf->grid->dev, bytes, hipMemcpyDeviceToDevice, s));
   for (int64_t it = 0; it < K; ++it) {
     if (it % every == 0) {
-      DFT_HIP_CHECK(hipMemcpyAsync(cp[it / every], cur->grid->dev, bytes, hipMemcpyDeviceToDevice, s));
+      DFT_HIP_CHECK(hipMemcpyAsync(cp(it / every), cur->grid->dev, bytes, hipMemcpyDeviceToDevice, s));
       if (g_verbose) {
         DFT_HIP_CHECK(hipStreamSynchronize(s));
         fprintf(stderr, "libdft: adjoint forward step %lld / %lld\n", (long long)it, (long long)K);
@@ -2220,16 +2304,15 @@ int adjoint_sweep(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu, do
   // reverse sweep, segment by segment
   for (int64_t j = ncp - 1; j >= 0; --j) {
     const int64_t n0 = j * every, n1 = std::min(K, n0 + every);
-    DFT_HIP_CHECK(hipMemcpyAsync(cur->grid->dev, cp[j], bytes, hipMemcpyDeviceToDevice, s));
+    DFT_HIP_CHECK(hipMemcpyAsync(cur->grid->dev, cp(j), bytes, hipMemcpyDeviceToDevice, s));
     for (int64_t it = n0; it < n1; ++it) {
-      DFT_HIP_CHECK(hipMemcpyAsync(seg[it - n0], cur->grid->dev, bytes, hipMemcpyDeviceToDevice, s));
+      DFT_HIP_CHECK(hipMemcpyAsync(seg(it - n0), cur->grid->dev, bytes, hipMemcpyDeviceToDevice, s));
       if (it + 1 < n1) dft_ot_propagate(otf, cur, vext, mu, dt);
     }
     for (int64_t it = n1 - 1; it >= n0; --it)
-      adj_step<T>(otf, seg[it - n0], psib, mass, wl, mu, dtr, dti, k0, w, th);
+      adj_step<T>(otf, seg(it - n0), psib, mass, wl, mu, dtr, dti, k0, w, th);
     if (g_verbose) fprintf(stderr, "libdft: adjoint reverse segment %lld / %lld done\n", (long long)(ncp - j), (long long)ncp);
   }
-  cleanup();
   return 0;
 }
 
@@ -2241,9 +2324,10 @@ int adjoint_well_impl(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu
   hipStream_t s = lib_stream();
   const int64_t n = d->n;
   const bool BF = (otf->model & DFT_OT_BACKFLOW) != 0;
-  AdjWork<T> w;
-  cplx<T> *psib = nullptr;
-  bool ok = w.alloc(n, (int64_t)d->nx * d->ny * d->PP, BF) && (psib = (cplx<T> *)dmalloc(sizeof(cplx<T>) * n));
+  AdjLease<T> lease(d, BF);
+  AdjWork<T> &w = *lease.w;
+  cplx<T> *psib = w.psib;
+  const bool ok = lease.ok;
   double th[2] = {0.0, 0.0};
   auto seed = [&](wf *cur, cplx<T> *pb, double t2[2]) {
     // the gradient of the total energy with respect to psi_K
@@ -2275,9 +2359,6 @@ int adjoint_well_impl(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu
   if (rc) fprintf(stderr, "libdft: dft_ot_adjoint_well: out of device memory\n");
   grad[0] = th[0];
   grad[1] = th[1];
-  DFT_HIP_CHECK(hipStreamSynchronize(s));
-  dfree(psib);
-  w.release();
   return rc;
 }
 
@@ -2358,10 +2439,10 @@ int adjoint_cavity_impl(dft_ot_functional *otf, wf *gwf, double rho0, double R0,
   hipLaunchKernelGGL(k_cavity<T>, dim3(grid_for(n)), dim3(kBlock), 0, s, (cplx<T> *)gwf->grid->dev, geo, rho0, R0, wd,
                      n);
   DFT_LAUNCH_CHECK();
-  AdjWork<T> w;
-  cplx<T> *psib = nullptr;
-  bool ok = w.alloc(n, (int64_t)d->nx * d->ny * d->PP, (otf->model & DFT_OT_BACKFLOW) != 0) &&
-            (psib = (cplx<T> *)dmalloc(sizeof(cplx<T>) * n));
+  AdjLease<T> lease(d, (otf->model & DFT_OT_BACKFLOW) != 0);
+  AdjWork<T> &w = *lease.w;
+  cplx<T> *psib = w.psib;
+  const bool ok = lease.ok;
   double th[2] = {0.0, 0.0}, explicit_term = 0.0;
   auto seed = [&](wf *cur, cplx<T> *pb, double *) {
     const cplx<T> *psiK = (const cplx<T> *)cur->grid->dev;
@@ -2386,26 +2467,21 @@ int adjoint_cavity_impl(dft_ot_functional *otf, wf *gwf, double rho0, double R0,
     DFT_LAUNCH_CHECK();
     *grad = sum_partials(w.pa, red_blocks(n), s) + explicit_term;
   }
-  DFT_HIP_CHECK(hipStreamSynchronize(s));
-  dfree(psib);
-  w.release();
   return rc;
 }
 
 // Standalone reverse pass of V_OT at the density of gwf (for tests): rho_bar = (dV/drho)^T v_bar.
 template <typename T> bool potential_vjp_impl(dft_ot_functional *otf, T *rho_bar, const T *v_bar, wf *gwf) {
   dft_ot_device *d = otf->device;
-  AdjWork<T> w;
-  if (!w.alloc(d->n, (int64_t)d->nx * d->ny * d->PP, false)) {
+  AdjLease<T> lease(d, false);
+  AdjWork<T> &w = *lease.w;
+  if (!lease.ok) {
     fprintf(stderr, "libdft: dft_ot_potential_vjp: out of device memory\n");
-    w.release();
     return false;
   }
   Well none{0.0, 1.0, 0.0, 0.0, 0.0, d->step, d->nx, d->ny, d->nz};
   adj_potential<T>(otf, (const cplx<T> *)gwf->grid->dev, gwf->mass, none, 0.0, w);
   vjp_ot<T>(otf, v_bar, w.r[ARHO], nullptr, nullptr, rho_bar, w);
-  DFT_HIP_CHECK(hipStreamSynchronize(lib_stream()));
-  w.release();
   return true;
 }
 
@@ -2424,10 +2500,10 @@ template <typename T> bool potential_vjp_psi_impl(dft_ot_functional *otf, cplx<T
   dft_ot_device *d = otf->device;
   hipStream_t s = lib_stream();
   const bool BF = (otf->model & DFT_OT_BACKFLOW) != 0;
-  AdjWork<T> w;
-  if (!w.alloc(d->n, (int64_t)d->nx * d->ny * d->PP, BF)) {
+  AdjLease<T> lease(d, BF);
+  AdjWork<T> &w = *lease.w;
+  if (!lease.ok) {
     fprintf(stderr, "libdft: dft_ot_potential_vjp_psi: out of device memory\n");
-    w.release();
     return false;
   }
   const cplx<T> *psi = (const cplx<T> *)gwf->grid->dev;
@@ -2439,12 +2515,23 @@ template <typename T> bool potential_vjp_psi_impl(dft_ot_functional *otf, cplx<T
   DFT_HIP_CHECK(hipMemsetAsync(psib, 0, sizeof(cplx<T>) * d->n, s));
   vjp_ot<T>(otf, w.r[AVBAR], w.r[ARHO], psib, psi, nullptr, w);
   if (BF) vjp_bf<T>(otf, w.r[AVBAR], w.b[BVBI], w.r[ARHO], psib, psi, gwf->mass, w);
-  DFT_HIP_CHECK(hipStreamSynchronize(s));
-  w.release();
   return true;
 }
 
 }  // namespace
+
+bool dft::trim_workspaces() {
+  std::lock_guard<std::mutex> lk(g_adj_mu);
+  bool any = false;
+  for (size_t i = g_adj_devs.size(); i-- > 0;) {
+    dft_ot_device *d = g_adj_devs[i];
+    if (d->adj_busy) continue;
+    if (d->prec == GRID_FP32) drop_adj<float>(d);
+    else drop_adj<double>(d);
+    any = true;
+  }
+  return any;
+}
 
 // ================================================================== C ABI ==
 extern "C" {

@@ -72,3 +72,42 @@ def test_potential_nyquist_tiles(shape, model):
     want = o.potential(psi)
     assert np.abs(p.get() - want).max() <= 1e-10 * np.abs(want).max()
     p.free(), f.free(), w.free()
+
+
+def test_reverse_pass_work_space_is_reusable():
+    """The reverse passes' kept work space: repeated and interleaved calls of two
+    functionals, a sweep with more checkpoints than the one before, and two threads
+    on functionals of their own give the results of a first call, bit for bit."""
+    import threading
+
+    def setup(shape, model, seed):
+        w = L.Wave(shape, 0.9, L.GRID_FP64)
+        f = L.Functional(model, w, 2, 4)
+        w.set(inputs.smooth_modulated(shape, 0.9, f.p.rho0, 0.3, seed))
+        vb, out = L.CField(shape, 0.9, L.GRID_FP64), L.CField(shape, 0.9, L.GRID_FP64)
+        vb.set(inputs.smooth_modulated(shape, 0.9, 1.0, 0.5, seed + 1))
+        return w, f, vb, out
+
+    def vjp(s):
+        assert L.lib().dft_ot_potential_vjp_psi(s[1].h, s[3].h, s[2].h, s[0].h) == 0
+        return s[3].get()
+
+    def sweep(s, k, every):
+        return s[1].adjoint_well(-1e-4, 4.0, (0.0, 0.0, 0.0), 0.0, 100.0, k, every)
+
+    a, b = setup((16, 16, 32), 9, 5), setup((32, 16, 16), 1, 9)
+    first = vjp(a), vjp(b), sweep(a, 3, 2), sweep(a, 7, 3), sweep(b, 3, 2)
+    again = vjp(a), vjp(b), sweep(a, 3, 2), sweep(a, 7, 3), sweep(b, 3, 2)
+    for x, y in zip(first, again):
+        assert np.array_equal(np.asarray(x, dtype=object), np.asarray(y, dtype=object)) if isinstance(x, tuple) else np.array_equal(x, y)
+    got = {}
+    ts = [threading.Thread(target=lambda k=k, s=s: got.__setitem__(k, [vjp(s) for _ in range(3)])) for k, s in enumerate((a, b))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for k in (0, 1):
+        assert all(np.array_equal(x, first[k]) for x in got[k])
+    for s in (a, b):
+        for x in (s[2], s[3], s[1], s[0]):
+            x.free()
