@@ -115,26 +115,6 @@ void launch_strided(const Plan3D<T> &p, const fft::Batch &b, int nb, int axis, i
                2.0 * nb * (double)p.nx * p.ny * cols * sizeof(cplx<T>));
 }
 
-template <typename T, int N>
-void launch_xcombine(const Plan3D<T> &p, const fft::Batch &b, const fft::CombineSet &cs, const fft::KernTab &kt,
-                     int nb, hipStream_t s) {
-  using G = rf::ColCfg<T, N>;
-  const int ntile = (p.P + G::COLS - 1) / G::COLS;
-  dim3 grid((unsigned)(p.ny * ntile), nb);
-  // traffic: each term's spectrum and kernel, plus the output
-  double per = 0;
-  for (int i = 0; i < nb; ++i) {
-    per += sizeof(cplx<T>);
-    for (int t = 0; t < cs.c[i].nterms; ++t)
-      per += sizeof(cplx<T>) + (cs.c[i].t[t].kern >= 0 ? sizeof(T) : 0);
-  }
-  DFT_PROF_BEGIN(s);
-  hipLaunchKernelGGL((fft::k_xcombine_inv<T, N>), grid, dim3(G::BS), 0, s, b, cs, kt, p.ny, p.P, p.PP, ntile,
-                     p.twx);
-  DFT_LAUNCH_CHECK();
-  DFT_PROF_END(s, "fft_x_combine_c2c", per * (double)p.nhalf());
-}
-
 template <typename T, int N, int DIR>
 void launch_zc2c(const Plan3D<T> &p, const cplx<T> *src, cplx<T> *dst, const cplx<T> *pot, double dtr, double dti,
                  T scale, double *partial, hipStream_t s) {
@@ -216,7 +196,7 @@ int64_t strang_partials(int nx, int ny, int nz, int prec) {
 }
 
 template <typename T>
-void r2c3d(const Plan3D<T> &p, int nb, const T *const *in, cplx<T> *const *out, hipStream_t s) {
+void r2c3d(const Plan3D<T> &p, int nb, const T *const *in, cplx<T> *const *out, hipStream_t s, bool xpass) {
   for (int b0 = 0; b0 < nb; b0 += fft::kMaxBatch) {
     const int cnt = nb - b0 < fft::kMaxBatch ? nb - b0 : fft::kMaxBatch;
     fft::Batch bz{}, by{};
@@ -228,32 +208,20 @@ void r2c3d(const Plan3D<T> &p, int nb, const T *const *in, cplx<T> *const *out, 
     }
     DFT_DISPATCH_N(p.nz, (launch_zr2c<T, N_>(p, bz, cnt, s)));
     DFT_DISPATCH_N(p.ny, (launch_strided<T, N_, -1>(p, by, cnt, 1, p.P, p.PP, (T)1, s)));
-    DFT_DISPATCH_N(p.nx, (launch_strided<T, N_, -1>(p, by, cnt, 0, p.P, p.PP, (T)1, s)));
+    if (xpass) DFT_DISPATCH_N(p.nx, (launch_strided<T, N_, -1>(p, by, cnt, 0, p.P, p.PP, (T)1, s)));
   }
 }
 
 template <typename T>
-void c2r3d(const Plan3D<T> &p, int nin, const cplx<T> *const *in, int nout, const fft::Combine *cmb,
-           const fft::KernTab &kt, cplx<T> *const *tmp, T *const *out, hipStream_t s) {
-  if (nin > fft::kMaxBatch) {
-    fprintf(stderr, "libdft: c2r3d: too many inputs\n");
-    abort();
-  }
-  for (int b0 = 0; b0 < nout; b0 += fft::kMaxBatch) {
-    const int cnt = nout - b0 < fft::kMaxBatch ? nout - b0 : fft::kMaxBatch;
-    fft::Batch bx{}, by{}, bz{};
-    fft::CombineSet cs{};
-    for (int i = 0; i < nin; ++i) bx.in[i] = in[i];
+void c2r_yz(const Plan3D<T> &p, int nb, cplx<T> *const *in, T *const *out, hipStream_t s) {
+  ypass<T>(p, nb, in, +1, p.P, p.PP, s);
+  for (int b0 = 0; b0 < nb; b0 += fft::kMaxBatch) {
+    const int cnt = nb - b0 < fft::kMaxBatch ? nb - b0 : fft::kMaxBatch;
+    fft::Batch bz{};
     for (int i = 0; i < cnt; ++i) {
-      bx.out[i] = tmp[b0 + i];
-      by.in[i] = tmp[b0 + i];
-      by.out[i] = tmp[b0 + i];
-      bz.in[i] = tmp[b0 + i];
+      bz.in[i] = in[b0 + i];
       bz.out[i] = out[b0 + i];
-      cs.c[i] = cmb[b0 + i];
     }
-    DFT_DISPATCH_N(p.nx, (launch_xcombine<T, N_>(p, bx, cs, kt, cnt, s)));
-    DFT_DISPATCH_N(p.ny, (launch_strided<T, N_, +1>(p, by, cnt, 1, p.P, p.PP, (T)1, s)));
     DFT_DISPATCH_N(p.nz, (launch_zc2r<T, N_>(p, bz, cnt, (T)1, s)));
   }
 }
@@ -333,9 +301,8 @@ template <typename T> void c2c_inv(const Plan3D<T> &p, const cplx<T> *in, cplx<T
 
 #define DFT_INST(T)                                                                                          \
   template struct Plan3D<T>;                                                                                 \
-  template void r2c3d<T>(const Plan3D<T> &, int, const T *const *, cplx<T> *const *, hipStream_t);           \
-  template void c2r3d<T>(const Plan3D<T> &, int, const cplx<T> *const *, int, const fft::Combine *,          \
-                         const fft::KernTab &, cplx<T> *const *, T *const *, hipStream_t);                   \
+  template void r2c3d<T>(const Plan3D<T> &, int, const T *const *, cplx<T> *const *, hipStream_t, bool);     \
+  template void c2r_yz<T>(const Plan3D<T> &, int, cplx<T> *const *, T *const *, hipStream_t);                \
   template void strang<T>(const Plan3D<T> &, cplx<T> *, const cplx<T> *, double, double, double, double *,   \
                           hipStream_t, const double *);                                                      \
   template void c2c_fwd<T>(const Plan3D<T> &, const cplx<T> *, cplx<T> *, hipStream_t);                    \

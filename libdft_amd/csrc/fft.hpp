@@ -11,10 +11,10 @@
 //    two lines.
 //  * y / x passes work on column tiles of the half spectrum
 //    [nx][ny][nz/2+1] (or of a full complex field for the propagator).
-//  * The inverse x pass can fuse a k-space combination on load:
+//  * The x pass of a convolution transforms forward, forms
 //    out(k) = sum_t s_t K_t(k) D_t(k) in_t(k), with K_t a real kernel
 //    spectrum and D_t = i sin(k_d h)/h, the symbol of the periodic central
-//    difference.
+//    difference, and transforms back (the x-middle pass of ot_fused.hpp).
 // Twiddles are computed in FP64 on the host; FP32 carries each as a rounded
 // value plus its residual.  Forward transforms are unnormalised (e^{-i}).
 #pragma once
@@ -184,19 +184,15 @@ struct Batch {
   void *out[kMaxBatch];
 };
 
-// k-space combination for the inverse x pass.
+// Output of a convolution: the inverse transform of sum_t s_t K_t(k) in_t(k).
 struct Term {
-  int in;       // index into Batch::in
-  int kern;     // index into KernTab::k, -1 = none
-  int deriv;    // 0,1,2 = multiply by i sin(k_d h)/h, -1 = none
+  int in;       // index of the input
+  int kern;     // index into KernTab::k
   double scale;
 };
 struct Combine {
   int nterms;
   Term t[4];
-};
-struct CombineSet {
-  Combine c[kMaxBatch];
 };
 struct KernTab {
   const void *k[8];    // real half-spectrum arrays [nx][ny][PP]

@@ -199,55 +199,6 @@ __global__ void __launch_bounds__((StrCfg<T, N>::BS))
   }
 }
 
-// ------------------------------- inverse x pass with fused k-space combine --
-// Spectra are [nx][ny][PP] (P values per row); x line (ky, kz) at ky*PP + kx*ny*PP + kz.
-template <typename T, int N>
-__global__ void __launch_bounds__((ColCfg<T, N>::BS))
-    k_xcombine_inv(Batch b, CombineSet cs, KernTab kt, int ny, int P, int PP, int ntile,
-                   const cplx<T> *__restrict__ g_tw) {
-  using C = cplx<T>;
-  using G = ColCfg<T, N>;
-  constexpr int E = G::E, TPL = G::TPL, COLS = G::COLS, LP = G::LP;
-  __shared__ C s_x[G::S > 1 ? COLS * LP : 1];
-  __shared__ C s_tw[rf::tw_len<T, N>()];
-  const Combine cb = cs.c[blockIdx.y];
-  void *out = b.out[blockIdx.y];
-  const int o = blockIdx.x / ntile, c0 = (blockIdx.x - o * ntile) * COLS;
-  const int col = threadIdx.x % COLS, t = threadIdx.x / COLS;
-  const bool act = c0 + col < P;
-  const int cc = act ? c0 + col : P - 1;
-  const uint32_t es = (uint32_t)ny * PP;
-  const uint32_t e0 = (uint32_t)o * PP + cc + t * es;  // element index of point t
-  rf::load_tw<T, N, G::EM, G::BS>(s_tw, g_tw);
-  const T *sx = (const T *)kt.sinx, *sy = (const T *)kt.siny, *sz = (const T *)kt.sinz;
-  C v[E];
-#pragma unroll
-  for (int i = 0; i < E; ++i) v[i] = cmk<C>(0, 0);
-  const size_t stC = (size_t)TPL * es * sizeof(C), stR = (size_t)TPL * es * sizeof(T);
-  for (int q = 0; q < cb.nterms; ++q) {
-    const Term tm = cb.t[q];
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-      const int el = t + TPL * i;
-      C a = gld<C>((const char *)b.in[tm.in] + i * stC, e0 * (uint32_t)sizeof(C));
-      T s = (T)tm.scale;
-      if (tm.kern >= 0) s *= gld<T>((const char *)kt.k[tm.kern] + i * stR, e0 * (uint32_t)sizeof(T));
-      if (tm.deriv >= 0) {
-        s *= tm.deriv == 0 ? sx[el] : (tm.deriv == 1 ? sy[o] : sz[cc]);
-        a = cmk<C>(-a.y, a.x);  // times i
-      }
-      v[i].x += s * a.x;
-      v[i].y += s * a.y;
-    }
-  }
-  __syncthreads();
-  rf::rfft<T, N, G::EM, +1, rf::BlockSync>(v, s_x + col * LP, s_tw, t);
-  if (act) {
-#pragma unroll
-    for (int i = 0; i < E; ++i) gst<C>((char *)out + i * stC, e0 * (uint32_t)sizeof(C), v[i]);
-  }
-}
-
 // ---------------------------------------- propagator passes (complex psi) --
 // Sum of an FP64 value over the block (BS threads) into partial[blockIdx.x].
 template <int BS> __device__ __forceinline__ void block_sum(double acc, double *partial) {
@@ -429,7 +380,7 @@ __global__ void __launch_bounds__((KinCfg<T, N>::BS), sizeof(T) == 4 ? DFT_XKIN_
   const double2 yz = make_double2(myz * cyz, -myz * sy);
   __syncthreads();
   rf::rfft_apply<T, N, G::EM, rf::BlockSync>(v, s_x + col * LP, s_tw, t,
-                                             [&](int e, double2 u) { return cmul(u, cmul(s_kx[e], yz)); });
+                                             [&](int i, double2 u) { return cmul(u, cmul(s_kx[t + TPL * i], yz)); });
   if (act) {
 #pragma unroll
     for (int i = 0; i < E; ++i) gst<C>((char *)psi + (size_t)i * st, ob, v[i]);

@@ -29,14 +29,13 @@ template <typename T> struct Plan3D {
 
 bool fft_size_ok(int64_t n);
 
-// Real fields -> half spectra [nx][ny][nz/2+1] (unnormalised forward transform).
+// Real fields -> half spectra [nx][ny][nz/2+1] (unnormalised forward transform);
+// without the x pass, spectra that the x-middle pass (ot.hip) takes as they are.
 template <typename T>
-void r2c3d(const Plan3D<T> &p, int nb, const T *const *in, cplx<T> *const *out, hipStream_t s);
-// Half spectra -> real fields: out_m = F^-1[ sum_t s_t K_t D_t in_t ], one combine per output.
-// tmp: nout half-spectrum scratch buffers.
+void r2c3d(const Plan3D<T> &p, int nb, const T *const *in, cplx<T> *const *out, hipStream_t s, bool xpass = true);
+// The way back from the x-middle pass: y (in place) and z passes to real fields.
 template <typename T>
-void c2r3d(const Plan3D<T> &p, int nin, const cplx<T> *const *in, int nout, const fft::Combine *cmb,
-           const fft::KernTab &kt, cplx<T> *const *tmp, T *const *out, hipStream_t s);
+void c2r_yz(const Plan3D<T> &p, int nb, cplx<T> *const *in, T *const *out, hipStream_t s);
 // One Strang step on psi; partial (may be null) receives per-block sums of |psi|^2.
 // k0 (may be null): momentum frame (kx0, ky0, kz0), kinetic symbol (k - k0)^2 / 2M.
 template <typename T>

@@ -8,7 +8,7 @@
 //   P2   local terms, Q = (c2 rhobar + c3 rhobar^2) rho, G_d = d_d rho (1 - F*rho/rho_0s),
 //        BF real part, W_d = v_d A - B_d, (d_d rho/(rho+eps)) W_d
 //   F2   r2c {Q, G_x, G_y, G_z}
-//   I2   c2r {J_d = F*G_d (3), T1 = F*sum_d d_d G_d}
+//   I2   c2r {J_d = F*G_d (3)} (unfused; fused: and T1 = F*sum_d d_d G_d = sum_d d_d J_d)
 //   P3   H = sum_d d_d rho J_d, KC terms 1 and 3, BF sum_d d_d W_d
 //   F3   r2c {H}
 //   I3   c2r {V_LJ*rho + Pi*Q + k23 c F*H}  (all linear terms summed in k space)
@@ -233,7 +233,7 @@ __global__ void k_stageB(StageBIn in, StageBOut out, PW<T> pw) {
 }
 
 struct StageCIn {
-  const void *rho, *rhot, *T1, *Jx, *Jy, *Jz, *Px, *Py, *Pz, *Wx, *Wy, *Wz;
+  const void *rho, *rhot, *Jx, *Jy, *Jz, *Wx, *Wy, *Wz;
 };
 struct StageCOut {
   void *H, *Vre, *Vim;
@@ -250,17 +250,17 @@ __global__ void k_stageC(StageCIn in, StageCOut out, PW<T> pw) {
     if constexpr (KC) {
       const T *rho = (const T *)in.rho;
       const T rst = ((const T *)in.rhot)[c] * (-pw.inv_rho0s) + (T)1;
-      const T J[3] = {((const T *)in.Jx)[c], ((const T *)in.Jy)[c], ((const T *)in.Jz)[c]};
-      const T Pd[3] = {((const T *)in.Px)[c], ((const T *)in.Py)[c], ((const T *)in.Pz)[c]};
-      T H = 0, t3 = 0;
+      const T *rt = (const T *)in.rhot, *J[3] = {(const T *)in.Jx, (const T *)in.Jy, (const T *)in.Jz};
+      T H = 0, t3 = 0, T1 = 0;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const T g = (rho[nb.p[d]] - rho[nb.m[d]]) * pw.inv2h;
-        H += g * J[d];
-        t3 += Pd[d] * J[d];
+        const T g = (rho[nb.p[d]] - rho[nb.m[d]]) * pw.inv2h, Jd = J[d][c];
+        H += g * Jd;
+        t3 += (rt[nb.p[d]] - rt[nb.m[d]]) * pw.inv2h * Jd;  // dF_d * rho = D_d (F * rho)
+        T1 += (J[d][nb.p[d]] - J[d][nb.m[d]]) * pw.inv2h;   // F * sum_d D_d G_d = sum_d D_d J_d
       }
       ((T *)out.H)[c] = H;
-      ((T *)out.Vre)[c] += ((const T *)in.T1)[c] * rst * pw.ckc - t3 * (pw.ckc * pw.k23);
+      ((T *)out.Vre)[c] += T1 * rst * pw.ckc - t3 * (pw.ckc * pw.k23);
     }
     if constexpr (BF) {
       const T *W[3] = {(const T *)in.Wx, (const T *)in.Wy, (const T *)in.Wz};
@@ -419,7 +419,7 @@ __global__ void k_grad_final(T *__restrict__ grad, const T *__restrict__ vre, co
 //   V = L*rho + c2/2 rb^2 + c3/3 rb^3 + Pi*[(c2 rb + c3 rb^2) rho]
 //       + ckc [rst T1 - k23 sum_d P_d J_d + k23 F*H].
 struct VjpA {
-  const void *vbar, *rho, *rb, *qb, *lv, *hp, *rt, *t1, *J[3], *Pd[3];
+  const void *vbar, *rho, *rb, *qb, *lv, *hp, *rt, *J[3];
   void *rp, *rbb, *t1b, *pb[3], *jb[3], *gb[3], *rsb;
 };
 
@@ -440,15 +440,19 @@ template <typename T, bool KC> __global__ void k_vjp_a(VjpA a, PW<T> pw) {
       const T ck = pw.ckc, ckk = pw.ckc * pw.k23;
       const T Hb = ckk * ((const T *)a.hp)[c];
       ((T *)a.t1b)[c] = ck * vb * rst;
-      ((T *)a.rsb)[c] = ck * vb * ((const T *)a.t1)[c];
+      const T *rt = (const T *)a.rt;
+      T t1 = 0;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
+        const T *Jf = (const T *)a.J[d];
+        t1 += (Jf[nb.p[d]] - Jf[nb.m[d]]) * pw.inv2h;
         const T g = (rho[nb.p[d]] - rho[nb.m[d]]) * pw.inv2h;
-        const T J = ((const T *)a.J[d])[c], P = ((const T *)a.Pd[d])[c];
+        const T J = Jf[c], P = (rt[nb.p[d]] - rt[nb.m[d]]) * pw.inv2h;
         ((T *)a.pb[d])[c] = -ckk * vb * J;
         ((T *)a.jb[d])[c] = -ckk * vb * P + Hb * g;
         ((T *)a.gb[d])[c] = Hb * J;
       }
+      ((T *)a.rsb)[c] = ck * vb * t1;
     }
   }
 }
@@ -902,11 +906,6 @@ struct dft_ot_device {
   double ig_g1;              // and its g_{3/2}(1)
   void *adj;                 // AdjWork of the reverse passes, kept between calls (or null)
   bool adj_busy;             // a call is working with it
-  // x-middle programs of the fused schedule in device memory, and the host
-  // copies they were uploaded from (re-uploaded only when one changes)
-  fused::MidProg *mid_dev;
-  fused::MidProg mid_host[3];
-  bool mid_valid[3];
 };
 
 namespace {
@@ -935,8 +934,8 @@ fft::Combine cmb(int nterms, const fft::Term *t) {
   for (int i = 0; i < nterms; ++i) c.t[i] = t[i];
   return c;
 }
-fft::Combine cmb1(int in, int kern, int deriv, double scale) {
-  fft::Term t{in, kern, deriv, scale};
+fft::Combine cmb1(int in, int kern, double scale) {
+  fft::Term t{in, kern, scale};
   return cmb(1, &t);
 }
 
@@ -989,6 +988,154 @@ template <typename T> PW<T> make_pw(dft_ot_functional *otf, double wf_mass, doub
     DFT_PROF_END(lib_stream(), name, (double)(nf) * (double)d->n * sizeof(T));               \
   } while (0)
 
+// x-middle implementation: 0 = all outputs of a column tile in one block
+// (k_xmid), 1 = one output per block (k_xconv) in FP32 for the programs
+// without derivative terms, 2 = k_xconv for every FP32 program, 3 = as 1 in
+// FP64 too (N <= 256)
+#ifndef DFT_XMID_KIND
+#define DFT_XMID_KIND 3
+#endif
+
+// Whether summed outputs without derivative terms take k_xconv (any number of kernels).
+template <typename T> constexpr bool xconv_sums(int nx) {
+  return ((DFT_XMID_KIND == 1 || DFT_XMID_KIND == 2) && sizeof(T) == 4) ||
+         (DFT_XMID_KIND == 3 && (sizeof(T) == 4 || nx <= 256));
+}
+
+template <typename T, int N, int NK, bool DV>
+void launch_xmid1(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T> *tw, hipStream_t s) {
+  using Cfg = fused::MidCfg<T, N>;
+  hipLaunchKernelGGL((fused::k_xmid<T, N, NK, DV>), dim3((unsigned)fused::mid_blocks<Cfg::COLS>(ny, P)),
+                     dim3(Cfg::BS), 0, s, pg, ny, P, PP, tw);
+}
+
+template <typename T, int N>
+const char *launch_xconv(const fused::MidProg &pg, bool deriv, int ny, int P, int PP,
+                         const cplx<T> *tw, hipStream_t s) {
+  // leading outputs with a single kernel term take the lean form, the rest
+  // the accumulating one
+  int n1 = 0;
+  while (n1 < pg.nout && pg.o[n1].nterms == 1 && pg.o[n1].t[0].kern >= 0 && pg.o[n1].t[0].deriv < 0) ++n1;
+  using Cfg1 = fused::XConvCfg<T, N, true>;
+  using Cfg = fused::XConvCfg<T, N, false>;
+  if (n1 > 0)
+    hipLaunchKernelGGL((fused::k_xconv<T, N, false, true>), dim3((unsigned)(fused::mid_blocks<Cfg1::COLS>(ny, P) * n1)),
+                       dim3(Cfg1::BS), 0, s, pg, 0, n1, ny, P, PP, tw);
+  if (n1 < pg.nout) {
+    const dim3 grid((unsigned)(fused::mid_blocks<Cfg::COLS>(ny, P) * (pg.nout - n1)));
+    if (deriv)
+      hipLaunchKernelGGL((fused::k_xconv<T, N, true, false>), grid, dim3(Cfg::BS), 0, s, pg, n1, pg.nout - n1, ny, P,
+                         PP, tw);
+    else
+      hipLaunchKernelGGL((fused::k_xconv<T, N, false, false>), grid, dim3(Cfg::BS), 0, s, pg, n1, pg.nout - n1, ny, P,
+                         PP, tw);
+  }
+  return n1 == pg.nout ? "ot_xconv_single" : (n1 == 0 ? "ot_xconv_multi" : "ot_xconv_mixed");
+}
+
+// x-middle pass of program pg (device copy; host copy hp).  Programs without
+// derivative terms run one output per block (k_xconv; FP64 only up to
+// N = 256); the others, and FP64 at N = 512, all outputs of a column tile per
+// block (k_xmid, instantiated per number of distinct kernels): measured at
+// 256^3 FP32, k_xconv takes 337 and 139 us for the first and last programs
+// against 427 and 158, k_xmid 266 us for the derivative program against 380.
+template <typename T, int N>
+void launch_xmid(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T> *tw,
+                 hipStream_t s, double bytes) {
+  bool deriv = false;
+  for (int m = 0; m < pg.nout; ++m)
+    for (int q = 0; q < pg.o[m].nterms; ++q) deriv = deriv || pg.o[m].t[q].deriv >= 0;
+  DFT_PROF_BEGIN(s);
+  bool one = true;
+  for (int m = 0; m < pg.nout; ++m) one = one && pg.o[m].nterms == 1;
+  if constexpr (xconv_sums<T>(N)) {
+    // per-output blocks unless the program shares inputs between
+    // multi-term outputs with derivative symbols (J_d and T1 = F sum_d D_d G_d)
+    if (one || !deriv || DFT_XMID_KIND == 2) {
+      const char *label = launch_xconv<T, N>(pg, deriv, ny, P, PP, tw, s);
+      DFT_LAUNCH_CHECK();
+      DFT_PROF_END(s, label, bytes);
+      return;
+    }
+  }
+  {
+    if (deriv && pg.nkern == 1) launch_xmid1<T, N, 1, true>(pg, ny, P, PP, tw, s);
+    else if (!deriv && pg.nkern == 1) launch_xmid1<T, N, 1, false>(pg, ny, P, PP, tw, s);
+    else if (!deriv && pg.nkern == 2) launch_xmid1<T, N, 2, false>(pg, ny, P, PP, tw, s);
+    else if (!deriv && pg.nkern == 3) launch_xmid1<T, N, 3, false>(pg, ny, P, PP, tw, s);
+    else {
+      fprintf(stderr, "libdft: x-middle program with %d kernels%s is not instantiated\n", pg.nkern,
+              deriv ? " and derivative terms" : "");
+      abort();
+    }
+  }
+  DFT_LAUNCH_CHECK();
+  DFT_PROF_END(s, "ot_xmid_fused", bytes);
+}
+
+fused::MidProg new_prog() { return fused::MidProg{}; }
+
+fused::MidTerm mterm(int in, int kern, int deriv, double scale) {
+  fused::MidTerm t{};
+  t.in = in;
+  t.kern = kern;
+  t.deriv = deriv;
+  t.scale = scale;
+  return t;
+}
+
+// Algorithmic traffic of an x-middle program: inputs and outputs, and each
+// distinct kernel spectrum once.
+template <typename T> double mid_bytes(const fused::MidProg &pg, int64_t nh) {
+  return (pg.nin + pg.nout) * (double)nh * sizeof(cplx<T>) + pg.nkern * (double)nh * sizeof(T);
+}
+
+// terms name kernels by K_*; the program lists the distinct ones and the terms their slots
+void set_kernels(fused::MidProg &pg, const fft::KernTab &kt) {
+  int slot[4] = {-1, -1, -1, -1};
+  pg.nkern = 0;
+  for (int m = 0; m < pg.nout; ++m)
+    for (int q = 0; q < pg.o[m].nterms; ++q) {
+      int &k = pg.o[m].t[q].kern;
+      if (k < 0) continue;
+      if (slot[k] < 0) {
+        slot[k] = pg.nkern;
+        pg.kern[pg.nkern++] = kt.k[k];
+      }
+      k = slot[k];
+    }
+  pg.sinx = kt.sinx;
+  pg.siny = kt.siny;
+  pg.sinz = kt.sinz;
+}
+
+// Convolutions of the unfused paths: inputs are half spectra after the z and y
+// passes (r2c3d without the x pass), outputs real fields.  The x transforms both
+// ways and the k-space combinations are one x-middle pass per output.
+template <typename T>
+void convolve(dft_ot_device *d, int nin, const cplx<T> *const *in, int nout, const fft::Combine *c,
+              cplx<T> *const *tmp, T *const *out) {
+  Plan3D<T> &p = plan_of<T>(d);
+  hipStream_t s = lib_stream();
+  fused::MidProg pg = new_prog();
+  pg.nin = nin;
+  pg.nout = nout;
+  pg.multi = -1;
+  for (int i = 0; i < nin; ++i) pg.in[i] = in[i];
+  for (int m = 0; m < nout; ++m) {
+    pg.o[m].nterms = c[m].nterms;
+    pg.o[m].out = tmp[m];
+    for (int q = 0; q < c[m].nterms; ++q) pg.o[m].t[q] = mterm(c[m].t[q].in, c[m].t[q].kern, -1, c[m].t[q].scale);
+  }
+  set_kernels(pg, kerntab<T>(d));
+  DFT_PROF_BEGIN(s);
+  const char *label = "";
+  DFT_DISPATCH_N(d->nx, (label = launch_xconv<T, N_>(pg, false, d->ny, d->P, d->PP, p.twx, s)));
+  DFT_LAUNCH_CHECK();
+  DFT_PROF_END(s, label, mid_bytes<T>(pg, (int64_t)d->nx * d->ny * d->P));
+  c2r_yz<T>(p, nout, tmp, out, s);
+}
+
 // Which parts of the potential to evaluate.
 // loc: local correlation (Pi terms), kc, bf; lj: the Lennard-Jones term
 // (-1: with loc, 0 / 1: without / with).
@@ -1007,7 +1154,6 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
   hipStream_t s = lib_stream();
   const double h3N = d->step * d->step * d->step / (double)d->n;
   const bool KC = parts.kc, BF = parts.bf, LOC = parts.loc, LJ = parts.lj < 0 ? LOC : parts.lj != 0;
-  fft::KernTab kt = kerntab<T>(d);
   PW<T> pw = make_pw<T>(otf, wf_mass, otf->div_epsilon, true);
 
   // P1
@@ -1036,7 +1182,7 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
       in.push_back(S<T>(d, SA_));
       out.push_back(CS<T>(d, SP5));
     }
-    r2c3d<T>(p, (int)in.size(), in.data(), out.data(), s);
+    r2c3d<T>(p, (int)in.size(), in.data(), out.data(), s, false);
   }
   // I1
   {
@@ -1044,30 +1190,26 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
     std::vector<fft::Combine> c;
     std::vector<T *> out;
     if (LOC) {
-      c.push_back(cmb1(0, K_SA, -1, h3N));
+      c.push_back(cmb1(0, K_SA, h3N));
       out.push_back(S<T>(d, RB));
     }
     if (KC) {
-      c.push_back(cmb1(0, K_F, -1, h3N));
+      c.push_back(cmb1(0, K_F, h3N));
       out.push_back(S<T>(d, RT));
-      for (int dd = 0; dd < 3; ++dd) {
-        c.push_back(cmb1(0, K_F, dd, h3N));
-        out.push_back(S<T>(d, PX + dd));
-      }
     }
     if (BF) {
-      c.push_back(cmb1(HB ? 5 : 0, K_U, -1, h3N));
+      c.push_back(cmb1(HB ? 5 : 0, K_U, h3N));
       out.push_back(S<T>(d, SA_));
       for (int dd = 0; dd < 3; ++dd) {
-        c.push_back(cmb1(1 + dd, K_U, -1, h3N));
+        c.push_back(cmb1(1 + dd, K_U, h3N));
         out.push_back(S<T>(d, SBX + dd));
       }
-      c.push_back(cmb1(4, K_U, -1, h3N));
+      c.push_back(cmb1(4, K_U, h3N));
       out.push_back(S<T>(d, SC));
     }
     std::vector<cplx<T> *> tmp;
     for (size_t i = 0; i < out.size(); ++i) tmp.push_back(CS<T>(d, TMP0 + (int)i));
-    if (!out.empty()) c2r3d<T>(p, HB ? 6 : 5, in, (int)out.size(), c.data(), kt, tmp.data(), out.data(), s);
+    if (!out.empty()) convolve<T>(d, HB ? 6 : 5, in, (int)out.size(), c.data(), tmp.data(), out.data());
   }
   // P2
   {
@@ -1098,23 +1240,20 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
         in.push_back(S<T>(d, QX + dd));
         out.push_back(CS<T>(d, SP1 + dd));
       }
-    if (!in.empty()) r2c3d<T>(p, (int)in.size(), in.data(), out.data(), s);
+    if (!in.empty()) r2c3d<T>(p, (int)in.size(), in.data(), out.data(), s, false);
   }
-  // I2 (J_d and T1 into the slots F2 has consumed; A = U*rho in SA_ stays for the adjoint)
+  // I2 (J_d into the slots F2 has consumed; A = U*rho in SA_ stays for the adjoint)
   if (KC) {
     const cplx<T> *in[3] = {CS<T>(d, SP1), CS<T>(d, SP2), CS<T>(d, SP3)};
-    fft::Combine c[4];
-    T *out[4] = {S<T>(d, QX), S<T>(d, QY), S<T>(d, QZ), S<T>(d, Q4)};
-    for (int dd = 0; dd < 3; ++dd) c[dd] = cmb1(dd, K_F, -1, h3N);
-    fft::Term t[3] = {{0, K_F, 0, h3N}, {1, K_F, 1, h3N}, {2, K_F, 2, h3N}};
-    c[3] = cmb(3, t);
-    cplx<T> *tmp[4] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2), CS<T>(d, TMP3)};
-    c2r3d<T>(p, 3, in, 4, c, kt, tmp, out, s);
+    fft::Combine c[3];
+    T *out[3] = {S<T>(d, QX), S<T>(d, QY), S<T>(d, QZ)};
+    for (int dd = 0; dd < 3; ++dd) c[dd] = cmb1(dd, K_F, h3N);
+    cplx<T> *tmp[3] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2)};
+    convolve<T>(d, 3, in, 3, c, tmp, out);
   }
   // P3
   if (KC || BF) {
-    StageCIn ci{rho, S<T>(d, RT), S<T>(d, Q4), S<T>(d, QX), S<T>(d, QY), S<T>(d, QZ), S<T>(d, PX),
-                S<T>(d, PY), S<T>(d, PZ), S<T>(d, WX), S<T>(d, WY), S<T>(d, WZ)};
+    StageCIn ci{rho, S<T>(d, RT), S<T>(d, QX), S<T>(d, QY), S<T>(d, QZ), S<T>(d, WX), S<T>(d, WY), S<T>(d, WZ)};
     StageCOut co{S<T>(d, TMP5), S<T>(d, VRE), S<T>(d, VIM)};
     if (KC && BF) LAUNCH_PW("ot_stage_kc_terms_bf_div", 17, (k_stageC<T, true, true>), ci, co, pw);
     else if (KC) LAUNCH_PW("ot_stage_kc_terms_bf_div", 12, (k_stageC<T, true, false>), ci, co, pw);
@@ -1125,19 +1264,19 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
     if (KC) {
       const T *in[1] = {S<T>(d, TMP5)};
       cplx<T> *out[1] = {CS<T>(d, SH)};
-      r2c3d<T>(p, 1, in, out, s);
+      r2c3d<T>(p, 1, in, out, s, false);
     }
     const cplx<T> *in[3] = {CS<T>(d, SP0), CS<T>(d, SP4), CS<T>(d, SH)};
     fft::Term t[3];
     int nt = 0;
-    if (LJ) t[nt++] = {0, K_LJ, -1, h3N};
-    if (LOC) t[nt++] = {1, K_SA, -1, h3N};
-    if (KC) t[nt++] = {2, K_F, -1, h3N * otf->kc_coef23 * otf->alpha_s / (2.0 * otf->mass)};
+    if (LJ) t[nt++] = {0, K_LJ, h3N};
+    if (LOC) t[nt++] = {1, K_SA, h3N};
+    if (KC) t[nt++] = {2, K_F, h3N * otf->kc_coef23 * otf->alpha_s / (2.0 * otf->mass)};
     fft::Combine c = cmb(nt, t);
     // (TMP1 as a real field: RB keeps rhobar for the adjoint pass)
     T *out[1] = {S<T>(d, TMP1)};
     cplx<T> *tmp[1] = {CS<T>(d, TMP0)};
-    c2r3d<T>(p, 3, in, 1, &c, kt, tmp, out, s);
+    convolve<T>(d, 3, in, 1, &c, tmp, out);
   }
   // ideal Bose gas of the thermal models, with the whole potential (dft_ot_potential,
   // dft_ot_potential2: src/ot.c:402-407, 505-510)
@@ -1187,91 +1326,6 @@ template <typename T, int N> void launch_zA(bool BF, const cplx<T> *psi, T *rho,
   else hipLaunchKernelGGL((fused::k_zA<T, N, false>), grid, dim3(fused::PairBS<T, N>), 0, s, psi, rho, o, npairs, P, pw, tw);
   DFT_LAUNCH_CHECK();
   DFT_PROF_END(s, "ot_zA_density_r2c", bytes);
-}
-
-// x-middle implementation: 0 = all outputs of a column tile in one block
-// (k_xmid), 1 = one output per block (k_xconv) in FP32 for the programs
-// without derivative terms, 2 = k_xconv for every FP32 program, 3 = as 1 in
-// FP64 too (N <= 256)
-#ifndef DFT_XMID_KIND
-#define DFT_XMID_KIND 3
-#endif
-
-// Whether summed outputs without derivative terms take k_xconv (any number of kernels).
-template <typename T> constexpr bool xconv_sums(int nx) {
-  return ((DFT_XMID_KIND == 1 || DFT_XMID_KIND == 2) && sizeof(T) == 4) ||
-         (DFT_XMID_KIND == 3 && (sizeof(T) == 4 || nx <= 256));
-}
-
-template <typename T, int N, int NK, bool DV>
-void launch_xmid1(const fused::MidProg *pg, int ny, int P, int PP, const cplx<T> *tw, hipStream_t s) {
-  using Cfg = fused::MidCfg<T, N>;
-  hipLaunchKernelGGL((fused::k_xmid<T, N, NK, DV>), dim3((unsigned)fused::mid_blocks<Cfg::COLS>(ny, P)),
-                     dim3(Cfg::BS), 0, s, pg, ny, P, PP, tw);
-}
-
-template <typename T, int N>
-const char *launch_xconv(const fused::MidProg *pg, const fused::MidProg &hp, bool deriv, int ny, int P, int PP,
-                         const cplx<T> *tw, hipStream_t s) {
-  // leading outputs with a single kernel term take the lean form, the rest
-  // the accumulating one
-  int n1 = 0;
-  while (n1 < hp.nout && hp.o[n1].nterms == 1 && hp.o[n1].t[0].kern >= 0 && hp.o[n1].t[0].deriv < 0) ++n1;
-  using Cfg1 = fused::XConvCfg<T, N, true>;
-  using Cfg = fused::XConvCfg<T, N, false>;
-  if (n1 > 0)
-    hipLaunchKernelGGL((fused::k_xconv<T, N, false, true>), dim3((unsigned)(fused::mid_blocks<Cfg1::COLS>(ny, P) * n1)),
-                       dim3(Cfg1::BS), 0, s, pg, 0, n1, ny, P, PP, tw);
-  if (n1 < hp.nout) {
-    const dim3 grid((unsigned)(fused::mid_blocks<Cfg::COLS>(ny, P) * (hp.nout - n1)));
-    if (deriv)
-      hipLaunchKernelGGL((fused::k_xconv<T, N, true, false>), grid, dim3(Cfg::BS), 0, s, pg, n1, hp.nout - n1, ny, P,
-                         PP, tw);
-    else
-      hipLaunchKernelGGL((fused::k_xconv<T, N, false, false>), grid, dim3(Cfg::BS), 0, s, pg, n1, hp.nout - n1, ny, P,
-                         PP, tw);
-  }
-  return n1 == hp.nout ? "ot_xconv_single" : (n1 == 0 ? "ot_xconv_multi" : "ot_xconv_mixed");
-}
-
-// x-middle pass of program pg (device copy; host copy hp).  Programs without
-// derivative terms run one output per block (k_xconv; FP64 only up to
-// N = 256); the others, and FP64 at N = 512, all outputs of a column tile per
-// block (k_xmid, instantiated per number of distinct kernels): measured at
-// 256^3 FP32, k_xconv takes 337 and 139 us for the first and last programs
-// against 427 and 158, k_xmid 266 us for the derivative program against 380.
-template <typename T, int N>
-void launch_xmid(const fused::MidProg *pg, const fused::MidProg &hp, int ny, int P, int PP, const cplx<T> *tw,
-                 hipStream_t s, double bytes) {
-  bool deriv = false;
-  for (int m = 0; m < hp.nout; ++m)
-    for (int q = 0; q < hp.o[m].nterms; ++q) deriv = deriv || hp.o[m].t[q].deriv >= 0;
-  DFT_PROF_BEGIN(s);
-  bool one = true;
-  for (int m = 0; m < hp.nout; ++m) one = one && hp.o[m].nterms == 1;
-  if constexpr (xconv_sums<T>(N)) {
-    // per-output blocks unless the program shares inputs between
-    // multi-term outputs with derivative symbols (J_d and T1 = F sum_d D_d G_d)
-    if (one || !deriv || DFT_XMID_KIND == 2) {
-      const char *label = launch_xconv<T, N>(pg, hp, deriv, ny, P, PP, tw, s);
-      DFT_LAUNCH_CHECK();
-      DFT_PROF_END(s, label, bytes);
-      return;
-    }
-  }
-  {
-    if (deriv && hp.nkern == 1) launch_xmid1<T, N, 1, true>(pg, ny, P, PP, tw, s);
-    else if (!deriv && hp.nkern == 1) launch_xmid1<T, N, 1, false>(pg, ny, P, PP, tw, s);
-    else if (!deriv && hp.nkern == 2) launch_xmid1<T, N, 2, false>(pg, ny, P, PP, tw, s);
-    else if (!deriv && hp.nkern == 3) launch_xmid1<T, N, 3, false>(pg, ny, P, PP, tw, s);
-    else {
-      fprintf(stderr, "libdft: x-middle program with %d kernels%s is not instantiated\n", hp.nkern,
-              deriv ? " and derivative terms" : "");
-      abort();
-    }
-  }
-  DFT_LAUNCH_CHECK();
-  DFT_PROF_END(s, "ot_xmid_fused", bytes);
 }
 
 // HB: the backflow density switch of HD / HD2 (k_zAB_bfhd)
@@ -1354,39 +1408,6 @@ void launch_zC(bool step, const fused::ZCArgs &a, int64_t npairs, int P, const c
   DFT_PROF_END(s, step ? "ot_zC_c2r_phase_z_fwd" : "ot_zC_c2r_accumulate", bytes);
 }
 
-// Device copy of x-middle program k (uploaded when it differs from the last one).
-const fused::MidProg *mid_prog(dft_ot_device *d, int k, const fused::MidProg &pg, hipStream_t s) {
-  if (!d->mid_valid[k] || memcmp(&d->mid_host[k], &pg, sizeof pg) != 0) {
-    DFT_HIP_CHECK(hipStreamSynchronize(s));
-    memcpy(&d->mid_host[k], &pg, sizeof pg);
-    DFT_HIP_CHECK(hipMemcpy(d->mid_dev + k, &d->mid_host[k], sizeof pg, hipMemcpyHostToDevice));
-    d->mid_valid[k] = true;
-  }
-  return d->mid_dev + k;
-}
-
-// A zero-filled program (padding included, so that programs compare bytewise).
-fused::MidProg new_prog() {
-  fused::MidProg pg;
-  memset(&pg, 0, sizeof pg);
-  return pg;
-}
-
-fused::MidTerm mterm(int in, int kern, int deriv, double scale) {
-  fused::MidTerm t{};
-  t.in = in;
-  t.kern = kern;
-  t.deriv = deriv;
-  t.scale = scale;
-  return t;
-}
-
-// Algorithmic traffic of an x-middle program: inputs and outputs, and each
-// distinct kernel spectrum once.
-template <typename T> double mid_bytes(const fused::MidProg &pg, int64_t nh) {
-  return (pg.nin + pg.nout) * (double)nh * sizeof(cplx<T>) + pg.nkern * (double)nh * sizeof(T);
-}
-
 template <typename T>
 void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *rho, cplx<T> *V, const StepIn *st) {
   dft_ot_device *d = otf->device;
@@ -1398,29 +1419,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
   const int64_t npairs = (int64_t)d->nx * d->ny / 2, nh = (int64_t)d->nx * d->ny * d->P, n = d->n;
   const int P = d->P, PP = d->PP;
   const double R = (double)n * sizeof(T), H = (double)nh * sizeof(cplx<T>);
-  fft::KernTab kt = kerntab<T>(d);
-  // terms name kernels by K_*; the program lists the distinct ones and the terms their slots
-  auto setk = [&](fused::MidProg &pg) {
-    int slot[4] = {-1, -1, -1, -1};
-    pg.nkern = 0;
-    for (int m = 0; m < pg.nout; ++m)
-      for (int q = 0; q < pg.o[m].nterms; ++q) {
-        int &k = pg.o[m].t[q].kern;
-        if (k < 0) continue;
-        if (slot[k] < 0) {
-          if (pg.nkern == fused::kMidMaxKern) {
-            fprintf(stderr, "libdft: x-middle program uses more than %d kernels\n", fused::kMidMaxKern);
-            abort();
-          }
-          slot[k] = pg.nkern;
-          pg.kern[pg.nkern++] = kt.k[k];
-        }
-        k = slot[k];
-      }
-    pg.sinx = kt.sinx;
-    pg.siny = kt.siny;
-    pg.sinz = kt.sinz;
-  };
+  const fft::KernTab kt = kerntab<T>(d);
 
   // ---- stage A: psi -> {rho, q_d, q4, [rho~]}, forward z and y
   const bool HB = BF && pw.bfhd;
@@ -1459,9 +1458,9 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
       add(HB ? 5 : 0, K_U);
       for (int i = 1; i <= (csum ? 3 : 4); ++i) add(i, K_U);
     }
-    setk(pg);
+    set_kernels(pg, kt);
     nB = pg.nout;
-    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(mid_prog(d, 0, pg, s), pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
+    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
     cplx<T> *b[8];
     for (int i = 0; i < nB; ++i) b[i] = CS<T>(d, TMP0 + i);
     ypass<T>(p, nB, b, +1, P, PP, s);
@@ -1505,8 +1504,8 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     for (int dd = 0; dd < 3; ++dd) pg.o[3].t[dd] = mterm(dd, K_F, dd, h3N);
     pg.o[3].out = d->slot[TMP3];
     pg.multi = 3;
-    setk(pg);
-    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(mid_prog(d, 1, pg, s), pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
+    set_kernels(pg, kt);
+    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
     cplx<T> *b[4] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2), CS<T>(d, TMP3)};
     ypass<T>(p, 4, b, +1, P, PP, s);
     fused::ZBCArgs a{};
@@ -1527,8 +1526,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     cplx<T> *hb[1] = {CS<T>(d, SH)};
     ypass<T>(p, 1, hb, -1, P, PP, s);
   } else if (BF) {
-    StageCIn ci{rho, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                S<T>(d, WX), S<T>(d, WY), S<T>(d, WZ)};
+    StageCIn ci{rho, nullptr, nullptr, nullptr, nullptr, S<T>(d, WX), S<T>(d, WY), S<T>(d, WZ)};
     StageCOut co{nullptr, S<T>(d, VRE), S<T>(d, VIM)};
     LAUNCH_PW("ot_stage_kc_terms_bf_div", 5, (k_stageC<T, false, true>), ci, co, pw);
   }
@@ -1556,8 +1554,8 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     if (csum) add(d->slot[SP4], K_U, -0.5 * h3N * otf->mass * otf->c_bfpot);
     pg.o[0].nterms = pg.nin;
     pg.o[0].out = d->slot[TMP4];
-    setk(pg);
-    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(mid_prog(d, 2, pg, s), pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
+    set_kernels(pg, kt);
+    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
     cplx<T> *b[1] = {CS<T>(d, TMP4)};
     ypass<T>(p, 1, b, +1, P, PP, s);
     fused::ZCArgs a{};
@@ -1594,7 +1592,6 @@ void energy_impl(dft_ot_functional *otf, T *eps, const cplx<T> *psi, double wf_m
   hipStream_t s = lib_stream();
   const double h3N = d->step * d->step * d->step / (double)d->n;
   const bool KC = parts.kc, BF = parts.bf, LOC = parts.loc;
-  fft::KernTab kt = kerntab<T>(d);
   PW<T> pw = make_pw<T>(otf, wf_mass, DFT_EPS, false);
   T *vx = S<T>(d, VX), *vy = S<T>(d, VY), *vz = S<T>(d, VZ);
   if (BF && !psi) {
@@ -1625,35 +1622,35 @@ void energy_impl(dft_ot_functional *otf, T *eps, const cplx<T> *psi, double wf_m
       in.push_back(S<T>(d, SA_));
       out.push_back(CS<T>(d, SP5));
     }
-    r2c3d<T>(p, (int)in.size(), in.data(), out.data(), s);
+    r2c3d<T>(p, (int)in.size(), in.data(), out.data(), s, false);
   }
   {
     const cplx<T> *in[6] = {CS<T>(d, SP0), CS<T>(d, SP1), CS<T>(d, SP2), CS<T>(d, SP3), CS<T>(d, SP4), CS<T>(d, SP5)};
     std::vector<fft::Combine> c;
     std::vector<T *> out;
     if (LOC) {
-      c.push_back(cmb1(0, K_LJ, -1, h3N));
+      c.push_back(cmb1(0, K_LJ, h3N));
       out.push_back(S<T>(d, PX));
-      c.push_back(cmb1(0, K_SA, -1, h3N));
+      c.push_back(cmb1(0, K_SA, h3N));
       out.push_back(S<T>(d, RB));
     }
     if (KC) {
-      c.push_back(cmb1(0, K_F, -1, h3N));
+      c.push_back(cmb1(0, K_F, h3N));
       out.push_back(S<T>(d, RT));
     }
     if (BF) {
-      c.push_back(cmb1(HB ? 5 : 0, K_U, -1, h3N));
+      c.push_back(cmb1(HB ? 5 : 0, K_U, h3N));
       out.push_back(S<T>(d, SA_));
       for (int dd = 0; dd < 3; ++dd) {
-        c.push_back(cmb1(1 + dd, K_U, -1, h3N));
+        c.push_back(cmb1(1 + dd, K_U, h3N));
         out.push_back(S<T>(d, SBX + dd));
       }
-      c.push_back(cmb1(4, K_U, -1, h3N));
+      c.push_back(cmb1(4, K_U, h3N));
       out.push_back(S<T>(d, SC));
     }
     std::vector<cplx<T> *> tmp;
     for (size_t i = 0; i < out.size(); ++i) tmp.push_back(CS<T>(d, TMP0 + (int)i));
-    c2r3d<T>(p, HB ? 6 : 5, in, (int)out.size(), c.data(), kt, tmp.data(), out.data(), s);
+    convolve<T>(d, HB ? 6 : 5, in, (int)out.size(), c.data(), tmp.data(), out.data());
   }
   {
     EnergyIn ei{rho, S<T>(d, PX), S<T>(d, RB), S<T>(d, RT), vx, vy, vz, S<T>(d, SA_), S<T>(d, SBX), S<T>(d, SBY),
@@ -1676,13 +1673,13 @@ void energy_impl(dft_ot_functional *otf, T *eps, const cplx<T> *psi, double wf_m
     if (KC) {
       const T *in3[3] = {S<T>(d, QX), S<T>(d, QY), S<T>(d, QZ)};
       cplx<T> *sp[3] = {CS<T>(d, SP1), CS<T>(d, SP2), CS<T>(d, SP3)};
-      r2c3d<T>(p, 3, in3, sp, s);
+      r2c3d<T>(p, 3, in3, sp, s, false);
       const cplx<T> *cin[3] = {sp[0], sp[1], sp[2]};
       fft::Combine c[3];
-      for (int dd = 0; dd < 3; ++dd) c[dd] = cmb1(dd, K_F, -1, h3N);
+      for (int dd = 0; dd < 3; ++dd) c[dd] = cmb1(dd, K_F, h3N);
       T *J[3] = {S<T>(d, SBX), S<T>(d, SBY), S<T>(d, SBZ)};
       cplx<T> *tmp[3] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2)};
-      c2r3d<T>(p, 3, cin, 3, c, kt, tmp, J, s);
+      convolve<T>(d, 3, cin, 3, c, tmp, J);
       LAUNCH_PW("ot_energy_kc", 8, (k_energyC<T>), eps, J[0], J[1], J[2], G[0], G[1], G[2], (T)(-otf->alpha_s / (4.0 * otf->mass)),
                 d->n);
     }
@@ -1700,19 +1697,18 @@ template <typename T> void gradient_impl(dft_ot_functional *otf, T *grad, const 
   hipStream_t s = lib_stream();
   const double h3N = d->step * d->step * d->step / (double)d->n;
   const bool KC = (otf->model & DFT_OT_KC) != 0;
-  fft::KernTab kt = kerntab<T>(d);
   PW<T> pw = make_pw<T>(otf, 1.0, otf->div_epsilon, false);
   {
     const T *in[1] = {rho};
     cplx<T> *out[1] = {CS<T>(d, SP0)};
-    r2c3d<T>(p, 1, in, out, s);
+    r2c3d<T>(p, 1, in, out, s, false);
   }
   {
     const cplx<T> *in[1] = {CS<T>(d, SP0)};
-    fft::Combine c[2] = {cmb1(0, K_SA, -1, h3N), cmb1(0, K_F, -1, h3N)};
+    fft::Combine c[2] = {cmb1(0, K_SA, h3N), cmb1(0, K_F, h3N)};
     T *out[2] = {S<T>(d, RB), S<T>(d, RT)};
     cplx<T> *tmp[2] = {CS<T>(d, TMP0), CS<T>(d, TMP1)};
-    c2r3d<T>(p, 1, in, KC ? 2 : 1, c, kt, tmp, out, s);
+    convolve<T>(d, 1, in, KC ? 2 : 1, c, tmp, out);
   }
   {
     StageBIn bi{rho, S<T>(d, RB), S<T>(d, RT), nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
@@ -1725,28 +1721,28 @@ template <typename T> void gradient_impl(dft_ot_functional *otf, T *grad, const 
   {
     const T *in[4] = {S<T>(d, Q4), S<T>(d, QX), S<T>(d, QY), S<T>(d, QZ)};
     cplx<T> *out[4] = {CS<T>(d, SP4), CS<T>(d, SP1), CS<T>(d, SP2), CS<T>(d, SP3)};
-    r2c3d<T>(p, KC ? 4 : 1, in, out, s);
+    r2c3d<T>(p, KC ? 4 : 1, in, out, s, false);
   }
   if (KC) {
     const cplx<T> *in[3] = {CS<T>(d, SP1), CS<T>(d, SP2), CS<T>(d, SP3)};
-    fft::Combine c[3] = {cmb1(0, K_F, -1, h3N), cmb1(1, K_F, -1, h3N), cmb1(2, K_F, -1, h3N)};
+    fft::Combine c[3] = {cmb1(0, K_F, h3N), cmb1(1, K_F, h3N), cmb1(2, K_F, h3N)};
     T *J[3] = {S<T>(d, SBX), S<T>(d, SBY), S<T>(d, SBZ)};
     cplx<T> *tmp[3] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2)};
-    c2r3d<T>(p, 3, in, 3, c, kt, tmp, J, s);
+    convolve<T>(d, 3, in, 3, c, tmp, J);
     LAUNCH_PW("ot_grad_kc", 9, (k_grad_kc<T>), rho, S<T>(d, RT), J[0], J[1], J[2], S<T>(d, SC), S<T>(d, WX),
               S<T>(d, WY), S<T>(d, WZ), pw);
     const T *hin[1] = {S<T>(d, SC)};
     cplx<T> *hout[1] = {CS<T>(d, SH)};
-    r2c3d<T>(p, 1, hin, hout, s);
+    r2c3d<T>(p, 1, hin, hout, s, false);
   }
   {
     const cplx<T> *in[3] = {CS<T>(d, SP0), CS<T>(d, SP4), CS<T>(d, SH)};
-    fft::Term t[3] = {{0, K_LJ, -1, h3N}, {1, K_SA, -1, h3N},
-                      {2, K_F, -1, h3N * otf->alpha_s / (2.0 * otf->mass) / otf->rho_0s}};
+    fft::Term t[3] = {{0, K_LJ, h3N}, {1, K_SA, h3N},
+                      {2, K_F, h3N * otf->alpha_s / (2.0 * otf->mass) / otf->rho_0s}};
     fft::Combine c = cmb(KC ? 3 : 2, t);
     T *out[1] = {S<T>(d, RB)};
     cplx<T> *tmp[1] = {CS<T>(d, TMP0)};
-    c2r3d<T>(p, 3, in, 1, &c, kt, tmp, out, s);
+    convolve<T>(d, 3, in, 1, &c, tmp, out);
   }
   LAUNCH_PW("ot_grad_final", KC ? 6 : 3, (k_grad_final<T>), grad, S<T>(d, VRE), S<T>(d, RB),
             KC ? S<T>(d, WX) : (T *)nullptr, S<T>(d, WY), S<T>(d, WZ), pw);
@@ -1819,7 +1815,6 @@ void free_device(dft_ot_device *d) {
   dfree(d->vsave);
   dfree(d->norm_part);
   dfree(d->igtab);
-  dfree(d->mid_dev);
   if (d->plan) {
     if (d->prec == GRID_FP32) {
       ((Plan3D<float> *)d->plan)->destroy();
@@ -2033,10 +2028,10 @@ void adj_conv(dft_ot_device *d, AdjWork<T> &w, int nin, const T *const *in, int 
   Plan3D<T> &p = plan_of<T>(d);
   hipStream_t s = lib_stream();
   cplx<T> *si[5] = {w.spec[0], w.spec[1], w.spec[2], w.spec[3], w.spec[4]};
-  r2c3d<T>(p, nin, in, si, s);
+  r2c3d<T>(p, nin, in, si, s, false);
   const cplx<T> *ci[5] = {w.spec[0], w.spec[1], w.spec[2], w.spec[3], w.spec[4]};
   cplx<T> *tmp[5] = {w.spec[5], w.spec[6], w.spec[7], w.spec[8], w.spec[9]};
-  c2r3d<T>(p, nin, ci, nout, c, kerntab<T>(d), tmp, out, s);
+  convolve<T>(d, nin, ci, nout, c, tmp, out);
 }
 
 // R = (dV_OT/drho)^T vbar (real parts: LJ, local, KC, HD) at the state whose
@@ -2051,7 +2046,7 @@ void vjp_ot(dft_ot_functional *otf, const T *vbar, const T *rho, cplx<T> *psib, 
   PW<T> pw = make_pw<T>(otf, 1.0, otf->div_epsilon, false);
   {
     const T *in[1] = {vbar};
-    fft::Combine c[3] = {cmb1(0, K_SA, -1, h3N), cmb1(0, K_LJ, -1, h3N), cmb1(0, K_F, -1, h3N)};
+    fft::Combine c[3] = {cmb1(0, K_SA, h3N), cmb1(0, K_LJ, h3N), cmb1(0, K_F, h3N)};
     T *out[3] = {w.r[AQB], w.r[ALV], w.r[AHP]};
     adj_conv<T>(d, w, 1, in, KC ? 3 : 2, c, out);
   }
@@ -2063,10 +2058,8 @@ void vjp_ot(dft_ot_functional *otf, const T *vbar, const T *rho, cplx<T> *psib, 
   a.lv = w.r[ALV];
   a.hp = w.r[AHP];
   a.rt = S<T>(d, RT);
-  a.t1 = S<T>(d, Q4);
   for (int k = 0; k < 3; ++k) {
     a.J[k] = S<T>(d, QX + k);
-    a.Pd[k] = S<T>(d, PX + k);
     a.pb[k] = w.r[APB + k];
     a.jb[k] = w.r[AJB + k];
     a.gb[k] = w.r[AGB + k];
@@ -2080,7 +2073,7 @@ void vjp_ot(dft_ot_functional *otf, const T *vbar, const T *rho, cplx<T> *psib, 
     LAUNCH_PW("ot_adjoint_b", 7, (k_vjp_b<T>), a, pw);
     {
       const T *in[3] = {w.r[AJB], w.r[AJB + 1], w.r[AJB + 2]};
-      fft::Combine c[3] = {cmb1(0, K_F, -1, h3N), cmb1(1, K_F, -1, h3N), cmb1(2, K_F, -1, h3N)};
+      fft::Combine c[3] = {cmb1(0, K_F, h3N), cmb1(1, K_F, h3N), cmb1(2, K_F, h3N)};
       T *out[3] = {w.r[AGBAR], w.r[AGBAR + 1], w.r[AGBAR + 2]};
       adj_conv<T>(d, w, 3, in, 3, c, out);
     }
@@ -2089,14 +2082,14 @@ void vjp_ot(dft_ot_functional *otf, const T *vbar, const T *rho, cplx<T> *psib, 
     LAUNCH_PW("ot_adjoint_c", 12, (k_vjp_c<T>), ac, pw);
     LAUNCH_PW("ot_adjoint_d", 10, (k_vjp_d<T>), a, pw);
     const T *in[2] = {w.r[ARBB], w.r[ARSB]};
-    fft::Term t[2] = {{0, K_SA, -1, h3N}, {1, K_F, -1, h3N}};
+    fft::Term t[2] = {{0, K_SA, h3N}, {1, K_F, h3N}};
     fft::Combine c = cmb(2, t);
     T *out[1] = {w.r[ACONV]};
     adj_conv<T>(d, w, 2, in, 1, &c, out);
   } else {
     LAUNCH_PW("ot_adjoint_a", 6, (k_vjp_a<T, false>), a, pw);
     const T *in[1] = {w.r[ARBB]};
-    fft::Combine c = cmb1(0, K_SA, -1, h3N);
+    fft::Combine c = cmb1(0, K_SA, h3N);
     T *out[1] = {w.r[ACONV]};
     adj_conv<T>(d, w, 1, in, 1, &c, out);
   }
@@ -2141,7 +2134,7 @@ void vjp_bf(dft_ot_functional *otf, const T *vrb, const T *vib, const T *rho, cp
   {
     const T *in[5] = {w.b[BAB], w.b[BBB], w.b[BBB + 1], w.b[BBB + 2], w.b[BTB]};
     fft::Combine c[5];
-    for (int i = 0; i < 5; ++i) c[i] = cmb1(i, K_U, -1, h3N);
+    for (int i = 0; i < 5; ++i) c[i] = cmb1(i, K_U, h3N);
     T *out[5] = {w.b[BUA], w.b[BUB], w.b[BUB + 1], w.b[BUB + 2], w.b[BUC]};
     adj_conv<T>(d, w, 5, in, 5, c, out);
   }
@@ -2671,7 +2664,6 @@ dft_ot_functional *dft_ot_alloc(INT model, wf *gwf, INT min_substeps, INT max_su
   if (ok)
     ok = (d->norm_part = (double *)dmalloc(sizeof(double) * (strang_partials(d->nx, d->ny, d->nz, d->prec) + 1))) !=
          nullptr;
-  if (ok) ok = (d->mid_dev = (fused::MidProg *)dmalloc(3 * sizeof(fused::MidProg))) != nullptr;
   if (ok && has_ig(otf)) {
     double tab[3 * ig::kTerms];
     ig::fill_table(tab);

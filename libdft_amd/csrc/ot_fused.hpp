@@ -398,12 +398,10 @@ template <int COLS> __device__ __forceinline__ MidCol mid_col(int ny, int P, int
 // Spectra are [nx][ny][PP] (P values per row) after the y pass; the x line
 // (ky = o, kz) has stride ny*PP.  Each distinct kernel spectrum is read once
 // per point into registers (NK of them) and shared by the terms that use it.
-// The program is read from device memory: indexed at run time, a by-value
-// kernel argument of this size would be copied to scratch by every thread.
+// The program is a kernel argument, indexed uniformly over the block: scalar loads.
 template <typename T, int N, int NK, bool DERIV>
-__global__ void __launch_bounds__((MidCfg<T, N>::BS), mid_minb<T>()) k_xmid(const MidProg *__restrict__ pgp, int ny, int P, int PP,
+__global__ void __launch_bounds__((MidCfg<T, N>::BS), mid_minb<T>()) k_xmid(const MidProg pg, int ny, int P, int PP,
                                                            const cplx<T> *__restrict__ g_tw) {
-  const MidProg &pg = *pgp;
   using C = cplx<T>;
   using G = MidCfg<T, N>;
   constexpr int E = G::E, TPL = G::TPL, COLS = G::COLS, LP = G::LP;
@@ -547,9 +545,8 @@ using XConvCfg = ColCfg<T, N, N >= 512 ? 16 : (ONE ? DFT_XCONV1_EM : DFT_XCONV_E
                         !(ONE && N == 128)>;
 
 template <typename T, int N, bool DERIV, bool ONE>
-__global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DFT_XCONV_MINB : DFT_XCONV_MINB64) k_xconv(const MidProg *__restrict__ pgp, int m0, int nl, int ny,
+__global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DFT_XCONV_MINB : DFT_XCONV_MINB64) k_xconv(const MidProg pg, int m0, int nl, int ny,
                                                               int P, int PP, const cplx<T> *__restrict__ g_tw) {
-  const MidProg &pg = *pgp;
   using C = cplx<T>;
   using G = XConvCfg<T, N, ONE>;
   constexpr int E = G::E, TPL = G::TPL, COLS = G::COLS, LP = G::LP;
@@ -577,13 +574,10 @@ __global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DF
 #pragma unroll
     for (int i = 0; i < E; ++i) k[i] = rf::gld<T>((const char *)pg.kern[tm.kern] + i * stR, obR);
     __syncthreads();
-    rf::rfft<T, N, G::EM, -1, rf::BlockSync>(v, X, s_tw, t);
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-      const T sc = (T)tm.scale * k[i];
-      v[i] = cmk<C>(sc * v[i].x, sc * v[i].y);
-    }
-    rf::rfft<T, N, G::EM, +1, rf::BlockSync>(v, X, s_tw, t);
+    rf::rfft_apply<T, N, G::EM, rf::BlockSync>(v, X, s_tw, t, [&](int i, double2 u) {
+      const double sc = tm.scale * (double)k[i];
+      return make_double2(sc * u.x, sc * u.y);
+    });
     if (act)
 #pragma unroll
       for (int i = 0; i < E; ++i) rf::gst<C>((char *)mo.out + i * stC, obC, v[i]);

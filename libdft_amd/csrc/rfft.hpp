@@ -280,8 +280,8 @@ __device__ __forceinline__ void point_fence(int r) {
   if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
 }
 
-// Transform of one line, f(point, value) applied to every Fourier coefficient in
-// FP64, and inverse transform (unnormalised).  The inverse mirrors the forward
+// Transform of one line, f(i, value) applied to every Fourier coefficient (point
+// t + TPL i of thread t) in FP64, and inverse transform (unnormalised).  The inverse mirrors the forward
 // stages, so the last forward stage, f and the first inverse stage work on the
 // same registers of a thread and run in FP64 for every T: a smooth field has few
 // large coefficients, whose rounding is much the same on every call and would
@@ -307,7 +307,7 @@ __device__ __forceinline__ void rfft_apply(Regs<T, N, EM> &v, cplx<T> *X, const 
     fft::dft<R, -1>(u);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      u[r] = f(t + TPL * (b + r * NB), u[r]);
+      u[r] = f(b + r * NB, u[r]);
       point_fence(r);
     }
     fft::dft<R, +1>(u);
