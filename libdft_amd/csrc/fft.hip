@@ -29,15 +29,6 @@ template <typename T> static cplx<T> *make_twiddles(int n) {
   return d;
 }
 
-// sin(2 pi m / n) / h for m in [0, cnt): the symbol of the periodic central difference.
-template <typename T> static T *make_sin(int n, int cnt, double step) {
-  std::vector<T> h(cnt);
-  for (int m = 0; m < cnt; ++m) h[m] = (T)(std::sin(2.0 * M_PI * (double)m / (double)n) / step);
-  auto *d = (T *)dmalloc(sizeof(T) * cnt);
-  DFT_HIP_CHECK(hipMemcpy(d, h.data(), sizeof(T) * cnt, hipMemcpyHostToDevice));
-  return d;
-}
-
 template <typename T> void Plan3D<T>::init(int nx_, int ny_, int nz_, double step_) {
   nx = nx_;
   ny = ny_;
@@ -48,20 +39,13 @@ template <typename T> void Plan3D<T>::init(int nx_, int ny_, int nz_, double ste
   twx = make_twiddles<T>(nx);
   twy = make_twiddles<T>(ny);
   twz = make_twiddles<T>(nz);
-  sinx = make_sin<T>(nx, nx, step);
-  siny = make_sin<T>(ny, ny, step);
-  sinz = make_sin<T>(nz, P, step);
 }
 
 template <typename T> void Plan3D<T>::destroy() {
   dfree(twx);
   dfree(twy);
   dfree(twz);
-  dfree(sinx);
-  dfree(siny);
-  dfree(sinz);
   twx = twy = twz = nullptr;
-  sinx = siny = sinz = nullptr;
 }
 
 namespace {

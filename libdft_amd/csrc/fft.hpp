@@ -196,7 +196,6 @@ struct Combine {
 };
 struct KernTab {
   const void *k[8];    // real half-spectrum arrays [nx][ny][PP]
-  const void *sinx, *siny, *sinz;  // sin(2 pi m / n) / h tables
 };
 
 }  // namespace fft

@@ -19,7 +19,6 @@ template <typename T> struct Plan3D {
   int PP = 0;  // row pitch of the half spectra (half_pitch(nz) >= P)
   double step = 0;
   cplx<T> *twx = nullptr, *twy = nullptr, *twz = nullptr;
-  T *sinx = nullptr, *siny = nullptr, *sinz = nullptr;
   void init(int nx_, int ny_, int nz_, double step_);
   void destroy();
   int64_t n() const { return (int64_t)nx * ny * nz; }

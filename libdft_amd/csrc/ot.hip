@@ -942,10 +942,6 @@ fft::Combine cmb1(int in, int kern, double scale) {
 template <typename T> fft::KernTab kerntab(dft_ot_device *d) {
   fft::KernTab kt{};
   for (int i = 0; i < 4; ++i) kt.k[i] = d->kern[i];
-  Plan3D<T> &p = plan_of<T>(d);
-  kt.sinx = p.sinx;
-  kt.siny = p.siny;
-  kt.sinz = p.sinz;
   return kt;
 }
 
@@ -988,98 +984,32 @@ template <typename T> PW<T> make_pw(dft_ot_functional *otf, double wf_mass, doub
     DFT_PROF_END(lib_stream(), name, (double)(nf) * (double)d->n * sizeof(T));               \
   } while (0)
 
-// x-middle implementation: 0 = all outputs of a column tile in one block
-// (k_xmid), 1 = one output per block (k_xconv) in FP32 for the programs
-// without derivative terms, 2 = k_xconv for every FP32 program, 3 = as 1 in
-// FP64 too (N <= 256)
-#ifndef DFT_XMID_KIND
-#define DFT_XMID_KIND 3
-#endif
-
-// Whether summed outputs without derivative terms take k_xconv (any number of kernels).
-template <typename T> constexpr bool xconv_sums(int nx) {
-  return ((DFT_XMID_KIND == 1 || DFT_XMID_KIND == 2) && sizeof(T) == 4) ||
-         (DFT_XMID_KIND == 3 && (sizeof(T) == 4 || nx <= 256));
-}
-
-template <typename T, int N, int NK, bool DV>
-void launch_xmid1(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T> *tw, hipStream_t s) {
-  using Cfg = fused::MidCfg<T, N>;
-  hipLaunchKernelGGL((fused::k_xmid<T, N, NK, DV>), dim3((unsigned)fused::mid_blocks<Cfg::COLS>(ny, P)),
-                     dim3(Cfg::BS), 0, s, pg, ny, P, PP, tw);
-}
-
+// x-middle pass of program pg, one output per block (k_xconv): leading outputs
+// with a single term take the lean form, the rest the accumulating one.
 template <typename T, int N>
-const char *launch_xconv(const fused::MidProg &pg, bool deriv, int ny, int P, int PP,
-                         const cplx<T> *tw, hipStream_t s) {
-  // leading outputs with a single kernel term take the lean form, the rest
-  // the accumulating one
+void launch_xconv(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T> *tw, hipStream_t s, double bytes) {
   int n1 = 0;
-  while (n1 < pg.nout && pg.o[n1].nterms == 1 && pg.o[n1].t[0].kern >= 0 && pg.o[n1].t[0].deriv < 0) ++n1;
+  while (n1 < pg.nout && pg.o[n1].nterms == 1) ++n1;
   using Cfg1 = fused::XConvCfg<T, N, true>;
   using Cfg = fused::XConvCfg<T, N, false>;
-  if (n1 > 0)
-    hipLaunchKernelGGL((fused::k_xconv<T, N, false, true>), dim3((unsigned)(fused::mid_blocks<Cfg1::COLS>(ny, P) * n1)),
-                       dim3(Cfg1::BS), 0, s, pg, 0, n1, ny, P, PP, tw);
-  if (n1 < pg.nout) {
-    const dim3 grid((unsigned)(fused::mid_blocks<Cfg::COLS>(ny, P) * (pg.nout - n1)));
-    if (deriv)
-      hipLaunchKernelGGL((fused::k_xconv<T, N, true, false>), grid, dim3(Cfg::BS), 0, s, pg, n1, pg.nout - n1, ny, P,
-                         PP, tw);
-    else
-      hipLaunchKernelGGL((fused::k_xconv<T, N, false, false>), grid, dim3(Cfg::BS), 0, s, pg, n1, pg.nout - n1, ny, P,
-                         PP, tw);
-  }
-  return n1 == pg.nout ? "ot_xconv_single" : (n1 == 0 ? "ot_xconv_multi" : "ot_xconv_mixed");
-}
-
-// x-middle pass of program pg (device copy; host copy hp).  Programs without
-// derivative terms run one output per block (k_xconv; FP64 only up to
-// N = 256); the others, and FP64 at N = 512, all outputs of a column tile per
-// block (k_xmid, instantiated per number of distinct kernels): measured at
-// 256^3 FP32, k_xconv takes 337 and 139 us for the first and last programs
-// against 427 and 158, k_xmid 266 us for the derivative program against 380.
-template <typename T, int N>
-void launch_xmid(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T> *tw,
-                 hipStream_t s, double bytes) {
-  bool deriv = false;
-  for (int m = 0; m < pg.nout; ++m)
-    for (int q = 0; q < pg.o[m].nterms; ++q) deriv = deriv || pg.o[m].t[q].deriv >= 0;
   DFT_PROF_BEGIN(s);
-  bool one = true;
-  for (int m = 0; m < pg.nout; ++m) one = one && pg.o[m].nterms == 1;
-  if constexpr (xconv_sums<T>(N)) {
-    // per-output blocks unless the program shares inputs between
-    // multi-term outputs with derivative symbols (J_d and T1 = F sum_d D_d G_d)
-    if (one || !deriv || DFT_XMID_KIND == 2) {
-      const char *label = launch_xconv<T, N>(pg, deriv, ny, P, PP, tw, s);
-      DFT_LAUNCH_CHECK();
-      DFT_PROF_END(s, label, bytes);
-      return;
-    }
-  }
-  {
-    if (deriv && pg.nkern == 1) launch_xmid1<T, N, 1, true>(pg, ny, P, PP, tw, s);
-    else if (!deriv && pg.nkern == 1) launch_xmid1<T, N, 1, false>(pg, ny, P, PP, tw, s);
-    else if (!deriv && pg.nkern == 2) launch_xmid1<T, N, 2, false>(pg, ny, P, PP, tw, s);
-    else if (!deriv && pg.nkern == 3) launch_xmid1<T, N, 3, false>(pg, ny, P, PP, tw, s);
-    else {
-      fprintf(stderr, "libdft: x-middle program with %d kernels%s is not instantiated\n", pg.nkern,
-              deriv ? " and derivative terms" : "");
-      abort();
-    }
-  }
+  if (n1 > 0)
+    hipLaunchKernelGGL((fused::k_xconv<T, N, true>), dim3((unsigned)(fused::mid_blocks<Cfg1::COLS>(ny, P) * n1)),
+                       dim3(Cfg1::BS), 0, s, pg, 0, n1, ny, P, PP, tw);
+  if (n1 < pg.nout)
+    hipLaunchKernelGGL((fused::k_xconv<T, N, false>),
+                       dim3((unsigned)(fused::mid_blocks<Cfg::COLS>(ny, P) * (pg.nout - n1))), dim3(Cfg::BS), 0, s, pg,
+                       n1, pg.nout - n1, ny, P, PP, tw);
   DFT_LAUNCH_CHECK();
-  DFT_PROF_END(s, "ot_xmid_fused", bytes);
+  DFT_PROF_END(s, n1 == pg.nout ? "ot_xconv_single" : (n1 == 0 ? "ot_xconv_multi" : "ot_xconv_mixed"), bytes);
 }
 
 fused::MidProg new_prog() { return fused::MidProg{}; }
 
-fused::MidTerm mterm(int in, int kern, int deriv, double scale) {
+fused::MidTerm mterm(int in, int kern, double scale) {
   fused::MidTerm t{};
   t.in = in;
   t.kern = kern;
-  t.deriv = deriv;
   t.scale = scale;
   return t;
 }
@@ -1104,9 +1034,6 @@ void set_kernels(fused::MidProg &pg, const fft::KernTab &kt) {
       }
       k = slot[k];
     }
-  pg.sinx = kt.sinx;
-  pg.siny = kt.siny;
-  pg.sinz = kt.sinz;
 }
 
 // Convolutions of the unfused paths: inputs are half spectra after the z and y
@@ -1120,19 +1047,15 @@ void convolve(dft_ot_device *d, int nin, const cplx<T> *const *in, int nout, con
   fused::MidProg pg = new_prog();
   pg.nin = nin;
   pg.nout = nout;
-  pg.multi = -1;
   for (int i = 0; i < nin; ++i) pg.in[i] = in[i];
   for (int m = 0; m < nout; ++m) {
     pg.o[m].nterms = c[m].nterms;
     pg.o[m].out = tmp[m];
-    for (int q = 0; q < c[m].nterms; ++q) pg.o[m].t[q] = mterm(c[m].t[q].in, c[m].t[q].kern, -1, c[m].t[q].scale);
+    for (int q = 0; q < c[m].nterms; ++q) pg.o[m].t[q] = mterm(c[m].t[q].in, c[m].t[q].kern, c[m].t[q].scale);
   }
   set_kernels(pg, kerntab<T>(d));
-  DFT_PROF_BEGIN(s);
-  const char *label = "";
-  DFT_DISPATCH_N(d->nx, (label = launch_xconv<T, N_>(pg, false, d->ny, d->P, d->PP, p.twx, s)));
-  DFT_LAUNCH_CHECK();
-  DFT_PROF_END(s, label, mid_bytes<T>(pg, (int64_t)d->nx * d->ny * d->P));
+  DFT_DISPATCH_N(d->nx, (launch_xconv<T, N_>(pg, d->ny, d->P, d->PP, p.twx, s,
+                                             mid_bytes<T>(pg, (int64_t)d->nx * d->ny * d->P))));
   c2r_yz<T>(p, nout, tmp, out, s);
 }
 
@@ -1300,9 +1223,9 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
 // ------------------------------------------------------------ fused path --
 // dft_ot_potential on a wave function and the split-operator steps built on
 // it.  Schedule (stage kernels in ot_fused.hpp):
-//   zA, y, xmid{Pi, F, U products}, y^-1, zAB, y, [xmid{J_d, T1}, y^-1, zBC, y],
-//   xmid{V_LJ + Pi Q + k23 c F H}, y^-1, zC
-// 7 + 5 forward and 7 + 4 + 1 inverse real 3-D transforms for full OT, with
+//   zA, y, xconv{Pi, F, U products}, y^-1, zAB, y, [xconv{J_d}, y^-1, zBC, y],
+//   xconv{V_LJ + Pi Q + k23 c F H}, y^-1, zC
+// 7 + 5 forward and 7 + 3 + 1 inverse real 3-D transforms for full OT, with
 // all pointwise stages inside the z passes.
 struct StepIn {
   const void *vext;   // real field or null
@@ -1372,38 +1295,23 @@ void launch_zBC(bool BF, const fused::ZBCArgs &a, int64_t npairs, int P, const P
   constexpr int LN = rf::LineCfg<T, N, fused::pair_em<N>()>::LINES;
   const dim3 grid((unsigned)((npairs + LN - 1) / LN));
   DFT_PROF_BEGIN(s);
-  constexpr bool SPLIT = sizeof(T) == 8 && DFT_ZBC_SPLIT64;
-  if constexpr (SPLIT) {
-    // FP64: the J_d stages, then T1, the tail and the r2c of H (H and the term-3 sum through memory)
-    if (BF && pw.bfhd) {
-      hipLaunchKernelGGL((fused::k_zBC_bfhd<T, N, 1>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-      hipLaunchKernelGGL((fused::k_zBC_bfhd<T, N, 2>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-    } else if (BF) {
-      hipLaunchKernelGGL((fused::k_zBC<T, N, true, 1>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-      hipLaunchKernelGGL((fused::k_zBC<T, N, true, 2>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-    } else {
-      hipLaunchKernelGGL((fused::k_zBC<T, N, false, 1>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-      hipLaunchKernelGGL((fused::k_zBC<T, N, false, 2>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-    }
-  } else if (BF && pw.bfhd) {
-    hipLaunchKernelGGL((fused::k_zBC_bfhd<T, N>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-  } else if (BF) {
-    hipLaunchKernelGGL((fused::k_zBC<T, N, true>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-  } else {
-    hipLaunchKernelGGL((fused::k_zBC<T, N, false>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-  }
+  if (BF && pw.bfhd) hipLaunchKernelGGL((fused::k_zBC_bfhd<T, N>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
+  else if (BF) hipLaunchKernelGGL((fused::k_zBC<T, N, true>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
+  else hipLaunchKernelGGL((fused::k_zBC<T, N, false>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
   DFT_LAUNCH_CHECK();
   DFT_PROF_END(s, "ot_zBC_c2r_kc_terms_r2c", bytes);
 }
 
 template <typename T, int N>
-void launch_zC(bool step, const fused::ZCArgs &a, int64_t npairs, int P, const cplx<T> *tw, hipStream_t s,
-               double bytes) {
+void launch_zC(bool step, const fused::ZCArgs &a, int64_t npairs, int P, const PW<T> &pw, const cplx<T> *tw,
+               hipStream_t s, double bytes) {
   constexpr int LN = rf::LineCfg<T, N, fused::pair_em<N>()>::LINES;
-  const dim3 grid((unsigned)((npairs + LN - 1) / LN));
+  const dim3 grid((unsigned)((npairs + LN - 1) / LN)), blk(fused::PairBS<T, N>);
   DFT_PROF_BEGIN(s);
-  if (step) hipLaunchKernelGGL((fused::k_zC<T, N, true>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, tw);
-  else hipLaunchKernelGGL((fused::k_zC<T, N, false>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, tw);
+  if (step && a.jx) hipLaunchKernelGGL((fused::k_zC<T, N, true, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  else if (step) hipLaunchKernelGGL((fused::k_zC<T, N, true, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  else if (a.jx) hipLaunchKernelGGL((fused::k_zC<T, N, false, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  else hipLaunchKernelGGL((fused::k_zC<T, N, false, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
   DFT_LAUNCH_CHECK();
   DFT_PROF_END(s, step ? "ot_zC_c2r_phase_z_fwd" : "ot_zC_c2r_accumulate", bytes);
 }
@@ -1429,7 +1337,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
   // step, 4204 -> 4090 FP64).  On small grids the longer chain of the summing
   // pass costs as much as is saved (128^3 FP32: 722 and 724 us; 32x32x64: 92.0 and
   // 92.8).
-  const bool csum = BF && !HB && !pw.clamp_bf && n > ((int64_t)1 << 21) && xconv_sums<T>(d->nx);
+  const bool csum = BF && !HB && !pw.clamp_bf && n > ((int64_t)1 << 21);
   const int nA = BF ? (HB ? 6 : 5) : 1;
   fused::Ptrs8 oA{};
   for (int i = 0; i < nA; ++i) oA.p[i] = d->slot[SP0 + i];
@@ -1445,10 +1353,9 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     fused::MidProg pg = new_prog();
     pg.nin = nA;
     for (int i = 0; i < nA; ++i) pg.in[i] = d->slot[SP0 + i];
-    pg.multi = -1;
     auto add = [&](int in, int kern) {
       pg.o[pg.nout].nterms = 1;
-      pg.o[pg.nout].t[0] = mterm(in, kern, -1, h3N);
+      pg.o[pg.nout].t[0] = mterm(in, kern, h3N);
       pg.o[pg.nout].out = d->slot[TMP0 + pg.nout];
       pg.nout++;
     };
@@ -1460,7 +1367,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     }
     set_kernels(pg, kt);
     nB = pg.nout;
-    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
+    DFT_DISPATCH_N(d->nx, (launch_xconv<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
     cplx<T> *b[8];
     for (int i = 0; i < nB; ++i) b[i] = CS<T>(d, TMP0 + i);
     ypass<T>(p, nB, b, +1, P, PP, s);
@@ -1487,29 +1394,22 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     cplx<T> *b[4] = {CS<T>(d, Q4), CS<T>(d, QX), CS<T>(d, QY), CS<T>(d, QZ)};
     ypass<T>(p, nQ, b, -1, P, PP, s);
   }
-  // ---- KC: J_d = F*G_d, T1 = F*sum_d D_d G_d; then H, terms 1 and 3, BF divergence
+  // ---- KC: J_d = F*G_d; then H, terms 1 (z part) and 3, BF divergence
   if (KC) {
     fused::MidProg pg = new_prog();
-    pg.nin = 3;
-    pg.in[0] = d->slot[QX];
-    pg.in[1] = d->slot[QY];
-    pg.in[2] = d->slot[QZ];
-    pg.nout = 4;
+    pg.nin = pg.nout = 3;
     for (int dd = 0; dd < 3; ++dd) {
+      pg.in[dd] = d->slot[QX + dd];
       pg.o[dd].nterms = 1;
-      pg.o[dd].t[0] = mterm(dd, K_F, -1, h3N);
+      pg.o[dd].t[0] = mterm(dd, K_F, h3N);
       pg.o[dd].out = d->slot[TMP0 + dd];
     }
-    pg.o[3].nterms = 3;
-    for (int dd = 0; dd < 3; ++dd) pg.o[3].t[dd] = mterm(dd, K_F, dd, h3N);
-    pg.o[3].out = d->slot[TMP3];
-    pg.multi = 3;
     set_kernels(pg, kt);
-    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
-    cplx<T> *b[4] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2), CS<T>(d, TMP3)};
-    ypass<T>(p, 4, b, +1, P, PP, s);
+    DFT_DISPATCH_N(d->nx, (launch_xconv<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
+    cplx<T> *b[3] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2)};
+    ypass<T>(p, 3, b, +1, P, PP, s);
     fused::ZBCArgs a{};
-    for (int i = 0; i < 4; ++i) a.in.p[i] = d->slot[TMP0 + i];
+    for (int i = 0; i < 3; ++i) a.in.p[i] = d->slot[TMP0 + i];
     a.out.p[0] = d->slot[SH];
     a.rho = rho;
     a.rhot = d->slot[RT];
@@ -1518,10 +1418,10 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     a.wz = d->slot[WZ];
     a.vre = d->slot[VRE];
     a.vim = d->slot[VIM];
-    // scratch of the split form: the G_d spectra in QX, QY are consumed by the x-middle above
-    a.hbuf = d->slot[QX];
-    a.tbuf = d->slot[QY];
-    const double bytes = 4 * H + 3 * R + (BF ? 4 * R : 0) + H + R + (BF ? R : 0);
+    // the G_d spectra in QX, QY are consumed by the x-middle above
+    a.jx = d->slot[QX];
+    a.jy = d->slot[QY];
+    const double bytes = 3 * H + 3 * R + (BF ? 4 * R : 0) + H + 3 * R + (BF ? R : 0);
     DFT_DISPATCH_N(d->nz, (launch_zBC<T, N_>(BF, a, npairs, PP, pw, p.twz, s, bytes)));
     cplx<T> *hb[1] = {CS<T>(d, SH)};
     ypass<T>(p, 1, hb, -1, P, PP, s);
@@ -1542,12 +1442,11 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     pg.in[0] = d->slot[SP0];
     pg.in[1] = d->slot[Q4];
     pg.nout = 1;
-    pg.multi = 0;
-    pg.o[0].t[0] = mterm(0, K_LJ, -1, h3N);
-    pg.o[0].t[1] = mterm(1, K_SA, -1, h3N);
+    pg.o[0].t[0] = mterm(0, K_LJ, h3N);
+    pg.o[0].t[1] = mterm(1, K_SA, h3N);
     auto add = [&](void *in, int kern, double scale) {
       pg.in[pg.nin] = in;
-      pg.o[0].t[pg.nin] = mterm(pg.nin, kern, -1, scale);
+      pg.o[0].t[pg.nin] = mterm(pg.nin, kern, scale);
       ++pg.nin;
     };
     if (KC) add(d->slot[SH], K_F, h3N * otf->kc_coef23 * otf->alpha_s / (2.0 * otf->mass));
@@ -1555,14 +1454,19 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     pg.o[0].nterms = pg.nin;
     pg.o[0].out = d->slot[TMP4];
     set_kernels(pg, kt);
-    DFT_DISPATCH_N(d->nx, (launch_xmid<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
+    DFT_DISPATCH_N(d->nx, (launch_xconv<T, N_>(pg, d->ny, P, PP, p.twx, s, mid_bytes<T>(pg, nh))));
     cplx<T> *b[1] = {CS<T>(d, TMP4)};
     ypass<T>(p, 1, b, +1, P, PP, s);
     fused::ZCArgs a{};
     a.in.p[0] = d->slot[TMP4];
     a.vre = d->slot[VRE];
     a.vim = BF ? d->slot[VIM] : nullptr;
-    double bytes = H + R + (BF ? R : 0);
+    if (KC) {
+      a.jx = d->slot[QX];
+      a.jy = d->slot[QY];
+      a.rhot = d->slot[RT];
+    }
+    double bytes = H + R + (BF ? R : 0) + (KC ? 3 * R : 0);
     if (!st) {
       a.V = V;
       bytes += 4 * R;
@@ -1578,7 +1482,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
       a.dti = st->dti;
       bytes += (st->vext ? R : 0) + (st->vavg ? 2 * R : 0) + (st->vsave ? 2 * R : 0) + 6 * R;
     }
-    DFT_DISPATCH_N(d->nz, (launch_zC<T, N_>(st != nullptr, a, npairs, PP, p.twz, s, bytes)));
+    DFT_DISPATCH_N(d->nz, (launch_zC<T, N_>(st != nullptr, a, npairs, PP, pw, p.twz, s, bytes)));
   }
 }
 

@@ -14,14 +14,14 @@
 //   zA    psi -> rho (stored) and, with backflow, q_d = rho v_d, q4 = rho |v|^2;
 //         z r2c of {rho, q_x, q_y, q_z, q4} (and of rho~ = G rho, with rho~ in
 //         place of rho in q_d and q4, under the HD / HD2 backflow switch)
-//   xmid  x forward FFT, k-space products with real kernel spectra and the
-//         central-difference symbol i sin(k h)/h, x inverse FFT (a small
-//         program: several outputs per input, one multi-term output)
+//   xconv x forward FFT, k-space products with real kernel spectra and sums
+//         over terms, x inverse FFT (a small program of outputs)
 //   zAB   z c2r of {U*rho, U*q_d, U*q4} -> BF real part, W_d, BF imaginary part;
 //         z c2r of Pi*rho -> local terms, Q, z r2c of Q;
 //         z c2r of F*rho -> rho_st, G_d, z r2c of G_d
-//   zBC   z c2r of {J_d, T1} -> H, KC terms 1 and 3, BF divergence; z r2c of H
-//   zC    z c2r of the summed linear terms; V += (API), or phase = e^{-iV dt/2}
+//   zBC   z c2r of J_d -> J_x, J_y (stored), H, KC term 3 and the z part of
+//         term 1, BF divergence; z r2c of H
+//   zC    x and y parts of KC term 1; z c2r of the summed linear terms; V += (API), or phase = e^{-iV dt/2}
 //         and the first z pass of the propagator (step)
 #pragma once
 #include "fft_kernels.hpp"
@@ -156,6 +156,11 @@ template <typename T, int N> constexpr int PairBS = LineCfg<T, N, pair_em<N>()>:
   rf::load_tw<T, N, G::EM, G::BS>(s_tw, g_tw);                                 \
   __syncthreads();                                                           \
   const PairPos<T, N, TPL> q(p, t, pw)
+
+// Computes x here: arithmetic on registers whose result is needed only after
+// later stages is otherwise sunk past their branches, with its operands (the
+// loaded stencils) kept live in its place.
+template <typename T> __device__ __forceinline__ void settle(T &x) { asm volatile("" : "+v"(x)); }
 
 // r2c of the pair held in v and store of both half spectra to field `out`.
 template <typename T, int N>
@@ -329,9 +334,9 @@ __global__ void __launch_bounds__((PairBS<T, N>), 0)
   zA_body<T, N, true, true>(psi, rho, outs, npairs, P, pw, g_tw);
 }
 
-// ------------------------------------------------------------------ xmid --
+// ------------------------------------------------------------------ xconv --
 struct MidTerm {
-  int in, kern, deriv, pad;  // kern: slot of MidProg::kern (or -1); deriv: axis of i sin(k h)/h (or -1)
+  int in, kern;  // kern: slot of MidProg::kern (or -1)
   double scale;
 };
 struct MidOut {
@@ -341,27 +346,11 @@ struct MidOut {
 };
 constexpr int kMidMaxIn = 6, kMidMaxOut = 8, kMidMaxKern = 4;
 struct MidProg {
-  int nin, nout, multi, nkern;
+  int nin, nout, nkern;
   const void *in[kMidMaxIn];
   MidOut o[kMidMaxOut];
   const void *kern[kMidMaxKern];  // the distinct kernel spectra the terms use
-  const void *sinx, *siny, *sinz;
 };
-
-// x-middle geometry: DFT_XMID_EM points per thread (several spectra are live
-// at once), at least DFT_XMID_COLS columns per block.
-#ifndef DFT_XMID_EM
-#define DFT_XMID_EM 8
-#endif
-#ifndef DFT_XMID_COLS
-#define DFT_XMID_COLS 8
-#endif
-template <typename T, int N> using MidCfg = ColCfg<T, N, DFT_XMID_EM, DFT_XMID_COLS>;
-// minimum resident blocks per CU asked of the register allocator (0: none)
-#ifndef DFT_XMID_MINB
-#define DFT_XMID_MINB 0
-#endif
-template <typename T> constexpr int mid_minb() { return sizeof(T) == 4 ? DFT_XMID_MINB : 0; }
 
 // Blocks of the x-middle pass: ny * ntile tiles of COLS consecutive kz < P-1
 // at one ky, and ceil(ny / COLS) tiles of the Nyquist column kz = P-1 over COLS
@@ -369,7 +358,7 @@ template <typename T> constexpr int mid_minb() { return sizeof(T) == 4 ? DFT_XMI
 // lane, and takes several times as long as the others: these tiles go first,
 // dealt over the XCDs by the plain block order, so that they overlap the rest
 // instead of ending the launch alone (last, at 256^3 FP32: single-term outputs
-// 305 us, accumulating 141, derivative program 216; first: 252, 105, 184).
+// 305 us, accumulating 141; first: 252, 105).
 template <int COLS> __host__ __device__ inline int mid_tiles(int P) { return (P - 1 + COLS - 1) / COLS; }
 template <int COLS> __host__ __device__ inline int mid_blocks(int ny, int P) {
   return ny * mid_tiles<COLS>(P) + (ny + COLS - 1) / COLS;
@@ -396,105 +385,9 @@ template <int COLS> __device__ __forceinline__ MidCol mid_col(int ny, int P, int
 }
 
 // Spectra are [nx][ny][PP] (P values per row) after the y pass; the x line
-// (ky = o, kz) has stride ny*PP.  Each distinct kernel spectrum is read once
-// per point into registers (NK of them) and shared by the terms that use it.
-// The program is a kernel argument, indexed uniformly over the block: scalar loads.
-template <typename T, int N, int NK, bool DERIV>
-__global__ void __launch_bounds__((MidCfg<T, N>::BS), mid_minb<T>()) k_xmid(const MidProg pg, int ny, int P, int PP,
-                                                           const cplx<T> *__restrict__ g_tw) {
-  using C = cplx<T>;
-  using G = MidCfg<T, N>;
-  constexpr int E = G::E, TPL = G::TPL, COLS = G::COLS, LP = G::LP;
-  __shared__ C s_x[G::S > 1 ? COLS * LP : 1];
-  __shared__ C s_tw[rf::tw_len<T, N>()];
-  const int col = threadIdx.x % COLS, t = threadIdx.x / COLS;
-  const MidCol mc = mid_col<COLS>(ny, P, 1, col);
-  const int o = mc.o, kz = mc.kz;
-  const bool act = mc.act;
-  const uint32_t es = (uint32_t)ny * PP;
-  const uint32_t e0 = (uint32_t)o * PP + kz + t * es;  // element index of point t
-  const uint32_t obC = e0 * (uint32_t)sizeof(C), obR = e0 * (uint32_t)sizeof(T);
-  const size_t stC = (size_t)TPL * es * sizeof(C), stR = (size_t)TPL * es * sizeof(T);  // per point i
-  C *X = s_x + col * LP;
-  rf::load_tw<T, N, G::EM, G::BS>(s_tw, g_tw);
-  // the first input and the kernels are in flight while the twiddles land
-  C nxt[E];
-#pragma unroll
-  for (int i = 0; i < E; ++i) nxt[i] = rf::gld<C>((const char *)pg.in[0] + i * stC, obC);
-  T kv[NK][E];
-#pragma unroll
-  for (int k = 0; k < NK; ++k)
-#pragma unroll
-    for (int i = 0; i < E; ++i) kv[k][i] = rf::gld<T>((const char *)pg.kern[k] + i * stR, obR);
-  T sx[DERIV ? E : 1], sy = 0, sz = 0;
-  if constexpr (DERIV) {
-#pragma unroll
-    for (int i = 0; i < E; ++i) sx[i] = ((const T *)pg.sinx)[t + TPL * i];
-    sy = ((const T *)pg.siny)[o];
-    sz = ((const T *)pg.sinz)[kz];
-  }
-  // coefficient scale * K(k) [* i sin(k_d h)/h] times a, point i
-  auto coef = [&](const MidTerm &tm, int i, C a) {
-    T s = (T)tm.scale;
-    if (NK > 0 && tm.kern >= 0) {
-      T k = kv[0][i];
-#pragma unroll
-      for (int j = 1; j < NK; ++j)
-        if (tm.kern == j) k = kv[j][i];
-      s *= k;
-    }
-    if (DERIV && tm.deriv >= 0) {
-      s *= tm.deriv == 0 ? sx[DERIV ? i : 0] : (tm.deriv == 1 ? sy : sz);
-      return cmk<C>(-s * a.y, s * a.x);
-    }
-    return cmk<C>(s * a.x, s * a.y);
-  };
-  __syncthreads();
-  C acc[E];
-  if (pg.multi >= 0)
-#pragma unroll
-    for (int i = 0; i < E; ++i) acc[i] = cmk<C>(0, 0);
-  // the next input is loaded while the current one is transformed
-  for (int ii = 0; ii < pg.nin; ++ii) {
-    C v[E];
-#pragma unroll
-    for (int i = 0; i < E; ++i) v[i] = nxt[i];
-    if (ii + 1 < pg.nin)
-#pragma unroll
-      for (int i = 0; i < E; ++i) nxt[i] = rf::gld<C>((const char *)pg.in[ii + 1] + i * stC, obC);
-    rf::rfft<T, N, G::EM, -1, rf::BlockSync>(v, X, s_tw, t);
-    if (pg.multi >= 0) {
-      const MidOut &mo = pg.o[pg.multi];
-      for (int q = 0; q < mo.nterms; ++q) {
-        if (mo.t[q].in != ii) continue;
-        const MidTerm tm = mo.t[q];
-#pragma unroll
-        for (int i = 0; i < E; ++i) acc[i] = cadd(acc[i], coef(tm, i, v[i]));
-      }
-    }
-    for (int m = 0; m < pg.nout; ++m) {
-      if (m == pg.multi || pg.o[m].t[0].in != ii) continue;
-      const MidTerm tm = pg.o[m].t[0];
-      C u[E];
-#pragma unroll
-      for (int i = 0; i < E; ++i) u[i] = coef(tm, i, v[i]);
-      rf::rfft<T, N, G::EM, +1, rf::BlockSync>(u, X, s_tw, t);
-      if (act)
-#pragma unroll
-        for (int i = 0; i < E; ++i) rf::gst<C>((char *)pg.o[m].out + i * stC, obC, u[i]);
-    }
-  }
-  if (pg.multi >= 0) {
-    rf::rfft<T, N, G::EM, +1, rf::BlockSync>(acc, X, s_tw, t);
-    if (act)
-#pragma unroll
-      for (int i = 0; i < E; ++i) rf::gst<C>((char *)pg.o[pg.multi].out + i * stC, obC, acc[i]);
-  }
-}
-
-// ----------------------------------------------------------------- xconv --
-// The x-middle program one output per block: out_m = F_x^-1 sum_t c_t F_x in_t
-// over the terms of output m.  An input shared by several outputs is read once
+// (ky = o, kz) has stride ny*PP.  The program, a kernel argument, is indexed
+// uniformly over the block (scalar loads) and runs one output per block:
+// out_m = F_x^-1 sum_t c_t F_x in_t over the terms of output m.  An input shared by several outputs is read once
 // per output; the outputs of one column tile are consecutive logical blocks
 // on one XCD, so those re-reads mostly hit that XCD's L2.  Holding one line
 // (16 points per thread) plus an accumulator keeps the register count low
@@ -544,7 +437,7 @@ using XConvCfg = ColCfg<T, N, N >= 512 ? 16 : (ONE ? DFT_XCONV1_EM : DFT_XCONV_E
                                         : (sizeof(T) == 8 && DFT_XCONV_COLS > 32 ? 32 : DFT_XCONV_COLS)),
                         !(ONE && N == 128)>;
 
-template <typename T, int N, bool DERIV, bool ONE>
+template <typename T, int N, bool ONE>
 __global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DFT_XCONV_MINB : DFT_XCONV_MINB64) k_xconv(const MidProg pg, int m0, int nl, int ny,
                                                               int P, int PP, const cplx<T> *__restrict__ g_tw) {
   using C = cplx<T>;
@@ -619,14 +512,8 @@ __global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DF
     rf::rfft<T, N, G::EM, -1, rf::BlockSync>(v, X, s_tw, t);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
-      T sc = (T)tm.scale * k[i];
-      if (DERIV && tm.deriv >= 0) {
-        sc *= tm.deriv == 0 ? ((const T *)pg.sinx)[t + TPL * i]
-                            : (tm.deriv == 1 ? ((const T *)pg.siny)[o] : ((const T *)pg.sinz)[kz]);
-        acc[i] = cadd(acc[i], cmk<C>(-sc * v[i].y, sc * v[i].x));
-      } else {
-        acc[i] = cadd(acc[i], cmk<C>(sc * v[i].x, sc * v[i].y));
-      }
+      const T sc = (T)tm.scale * k[i];
+      acc[i] = cadd(acc[i], cmk<C>(sc * v[i].x, sc * v[i].y));
     }
   }
   rf::rfft<T, N, G::EM, +1, rf::BlockSync>(acc, X, s_tw, t);
@@ -644,30 +531,21 @@ __global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DF
 #ifndef DFT_ZBC_MINB
 #define DFT_ZBC_MINB 2
 #endif
-// the same requests for the single FP64 kernels (0: none), used when the
-// split forms below are off.  FP64 zBC at 2 waves per SIMD spills 240 bytes per
-// lane and still beats 1 wave (256 VGPRs + 56 AGPRs): 192.5 -> 198 steps/s at
-// 256^3; zAB at 2 waves (412 bytes of spills) is slower.
+// the same requests for the single FP64 kernels (0: none); zAB's is used when
+// the split form below is off
 #ifndef DFT_ZAB_MINB64
 #define DFT_ZAB_MINB64 0
 #endif
 #ifndef DFT_ZBC_MINB64
 #define DFT_ZBC_MINB64 2
 #endif
-// FP64 zAB (backflow) and zBC as two kernels each (1) or one (0), and the
-// waves per SIMD asked for the halves (0: none).  In FP64 neither half spills:
-// 200 -> 229 steps/s at 256^3 with both.
+// FP64 zAB (backflow) as two kernels (1) or one (0), and the waves per SIMD
+// asked for the halves (0: none).
 #ifndef DFT_ZAB_SPLIT64
 #define DFT_ZAB_SPLIT64 1
 #endif
-#ifndef DFT_ZBC_SPLIT64
-#define DFT_ZBC_SPLIT64 1
-#endif
 #ifndef DFT_ZAB_SPLIT_MINB64
 #define DFT_ZAB_SPLIT_MINB64 0
-#endif
-#ifndef DFT_ZBC_SPLIT_MINB64
-#define DFT_ZBC_SPLIT_MINB64 0
 #endif
 // (the zAB split in FP32, where neither half gets past 2 waves per SIMD without
 // spills, measured slower: zAB 375 -> 386 us at 256^3)
@@ -937,168 +815,159 @@ __global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZAB_MINB 
 
 // ------------------------------------------------------------------- zBC --
 struct ZBCArgs {
-  Ptrs8 in;   // J_x, J_y, J_z, T1
+  Ptrs8 in;   // J_x, J_y, J_z
   Ptrs8 out;  // H
   const void *rho, *rhot, *wx, *wy, *wz;
   void *vre, *vim;
-  void *hbuf, *tbuf;  // split form: H and the term-3 sum between the two kernels (real fields)
+  void *jx, *jy;  // J_x and J_y as real fields, for the rest of sum_d D_d J_d in zC
 };
 
+// c2r of the J_d; H = sum_d g_d J_d and its r2c, KC term 3, the z part of term 1
+// and the backflow divergence.  KC term 1 is c rst F*(sum_d D_d G_d) = c rst
+// sum_d D_d J_d: J_z's difference comes from the line itself (through LDS), J_x
+// and J_y are stored for the stencils of zC.  Against a fourth transform for
+// the sum, at 256^3 FP32 (us): x-middle 184 -> 116, a y pass of 24 and a z
+// transform less, zC 105 -> 133; 32x32x64 FP32 step 91 -> 83.5.
+// Bound by the loads: 3 spectra and 7 real fields with stencils.  With the sums
+// settled after each axis the kernel takes 114 VGPRs in FP32 (176 without; 4
+// waves per SIMD for 2; zBC 268 -> 225 us at 256^3) and 128 in FP64 (256 and
+// spills, or two kernels with H in memory between them, 547 -> 453 us).
 // Every stage first issues the loads that do not depend on its spectrum (the
 // stencils of rho and rho~, the fields accumulated into), so that their
 // latency overlaps the spectrum's loads and transform.
-// PART 0: the whole stage; PART 1 (the three J_d stages, H and the term-3
-// sum stored) then PART 2 (T1, the tail and the r2c of H): the split form FP64
-// runs with fewer live fields.
 // HB: the backflow density switch of HD / HD2 (the divergence half of Im V_BF
 // is multiplied by G(rho)).
-template <typename T, int N, bool BF, int PART, bool HB>
+template <typename T, int N, bool BF, bool HB>
 __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T> pw,
                                          const cplx<T> *__restrict__ g_tw) {
   FUSED_PAIR_SETUP();
   constexpr int PF = prefetch_bits<T, DFT_ZBC_PF>();
   const void *rho = a.rho, *rhot = a.rhot;
   C v[E];
-  T H[2][PART == 2 ? 1 : E], t3[2][E];
+  T H[2][E], t3[2][E];
   fft::RawPair<T, N, pair_em<N>()> raw;
   auto c2r = [&](const void *cur, const void *next) {
     if constexpr ((PF & 8) != 0) c2r_pipe<T, N>(v, raw, X, s_tw, t, next, p, P);
     else load_c2r<T, N>(v, X, s_tw, t, cur, p, P);
   };
-  if constexpr ((PF & 8) != 0) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[PART == 2 ? 3 : 0], p, P, t);
+  if constexpr ((PF & 8) != 0) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[0], p, P, t);
   auto axis = [&](auto dtag) {
     constexpr int D = decltype(dtag)::value;
     T g[2][E], Pd[2][E];
-    auto stencil = [&] {
+    auto grad_w = [&](int w) {
       const auto qq = q.here();
 #pragma unroll
-      for (int i = 0; i < E; ++i)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          g[w][i] = grad_d<T, D>(rho, qq, w, i, pw);
-          Pd[w][i] = grad_d<T, D>(rhot, qq, w, i, pw);  // (dF_d * rho) = D_d (F * rho)
-        }
+      for (int i = 0; i < E; ++i) g[w][i] = grad_d<T, D>(rho, qq, w, i, pw);
     };
-    if constexpr ((PF & 1) != 0) stencil();
-    c2r(a.in.p[D], a.in.p[D + 1]);
-    if constexpr ((PF & 1) == 0) stencil();
+    auto pd_w = [&](int w) {
+      const auto qq = q.here();
 #pragma unroll
-    for (int i = 0; i < E; ++i) {
+      for (int i = 0; i < E; ++i) Pd[w][i] = grad_d<T, D>(rhot, qq, w, i, pw);  // (dF_d * rho) = D_d (F * rho)
+    };
+    if constexpr ((PF & 1) != 0)
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        const T J = part(v[i], w);
-        if constexpr (D == 0) {
-          H[w][i] = g[w][i] * J;
-          t3[w][i] = Pd[w][i] * J;
-        } else {
-          H[w][i] += g[w][i] * J;
-          t3[w][i] += Pd[w][i] * J;
-        }
-      }
+      for (int w = 0; w < 2; ++w) grad_w(w), pd_w(w);
+    c2r(a.in.p[D], D < 2 ? a.in.p[D + 1] : nullptr);
+    if constexpr (D < 2)
+      if (act)
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) q.template put<T>(D == 0 ? a.jx : a.jy, w, i, part(v[i], w));
+    // without prefetching, the stencils of one line and field at a time
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      if constexpr ((PF & 1) == 0) grad_w(w);
+#pragma unroll
+      for (int i = 0; i < E; ++i) H[w][i] = D == 0 ? g[w][i] * part(v[i], w) : H[w][i] + g[w][i] * part(v[i], w);
     }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      if constexpr ((PF & 1) == 0) pd_w(w);
+#pragma unroll
+      for (int i = 0; i < E; ++i) t3[w][i] = D == 0 ? Pd[w][i] * part(v[i], w) : t3[w][i] + Pd[w][i] * part(v[i], w);
+    }
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int i = 0; i < E; ++i) settle(H[w][i]), settle(t3[w][i]);
   };
-  if constexpr (PART != 2) {
-    axis(std::integral_constant<int, 0>{});
-    axis(std::integral_constant<int, 1>{});
-    axis(std::integral_constant<int, 2>{});
-  }
-  if constexpr (PART == 1) {
-    // first kernel of the split form: H and the term-3 sum to memory
-    if (act) {
-      const auto qs = q.here();
-#pragma unroll
-      for (int i = 0; i < E; ++i)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          qs.template put<T>(a.hbuf, w, i, H[w][i]);
-          qs.template put<T>(a.tbuf, w, i, t3[w][i]);
-        }
-    }
-    return;
-  } else if constexpr (PART == 2) {
-    const auto qs = q.here();
-#pragma unroll
-    for (int i = 0; i < E; ++i)
-#pragma unroll
-      for (int w = 0; w < 2; ++w) t3[w][i] = qs.template at_once<T>(a.tbuf, w, i);
-  }
-  // rho_st, V_re so far, and the backflow imaginary part (which does not
-  // involve T1); with prefetching, all before T1's transform
-  std::remove_const_t<decltype(q)> qt;
-  auto rst_at = [&](int w, int i) { return qt.template at<T>(rhot, w, i) * (-pw.inv_rho0s) + (T)1; };
-  auto vre_at = [&](int w, int i) { return qt.template at_once<T>(a.vre, w, i); };
-  auto kc_at = [&](T J, T rst, int w, int i) { return J * rst * pw.ckc - t3[w][i] * (pw.ckc * pw.k23); };
-  auto bf_im = [&](int w, int i) {
+  // the backflow divergence, and V_re so far and rho_st (both before J_z's
+  // transform with prefetching)
+  auto bf_div = [&](int w) {
     if constexpr (BF) {
-      T im = qt.template at_once<T>(a.vim, w, i);
-      if constexpr (HB) {
-        const T gw = bf_g(qt.template at<T>(rho, w, i), pw);
+      const auto qt = q.here();
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        T im = qt.template at_once<T>(a.vim, w, i);
+        T gw = (T)1;
+        if constexpr (HB) gw = bf_g(qt.template at<T>(rho, w, i), pw);
         im += (T)0.5 * (((qt.template nb<T, 0, 1>(a.wx, w, i) - qt.template nb<T, 0, -1>(a.wx, w, i)) * pw.inv2h) * gw);
         im += (T)0.5 * (((qt.template nb<T, 1, 1>(a.wy, w, i) - qt.template nb<T, 1, -1>(a.wy, w, i)) * pw.inv2h) * gw);
         im += (T)0.5 * (((qt.template nb<T, 2, 1>(a.wz, w, i) - qt.template nb<T, 2, -1>(a.wz, w, i)) * pw.inv2h) * gw);
-      } else {
-        im += (T)0.5 * ((qt.template nb<T, 0, 1>(a.wx, w, i) - qt.template nb<T, 0, -1>(a.wx, w, i)) * pw.inv2h);
-        im += (T)0.5 * ((qt.template nb<T, 1, 1>(a.wy, w, i) - qt.template nb<T, 1, -1>(a.wy, w, i)) * pw.inv2h);
-        im += (T)0.5 * ((qt.template nb<T, 2, 1>(a.wz, w, i) - qt.template nb<T, 2, -1>(a.wz, w, i)) * pw.inv2h);
+        if (pw.clamp_bf) im = clampv(im, pw.bfmax);
+        if (act) qt.template put<T>(a.vim, w, i, im * pw.cbf);
       }
-      if (pw.clamp_bf) im = clampv(im, pw.bfmax);
-      if (act) qt.template put<T>(a.vim, w, i, im * pw.cbf);
     }
   };
-  if constexpr ((PF & 2) != 0) {
-    qt = q.here();
-    T rst[2][E], base[2][E];
+  T rst[2][E], base[2][E];
+  auto base_w = [&](int w) {
+    const auto qt = q.here();
 #pragma unroll
-    for (int i = 0; i < E; ++i)
+    for (int i = 0; i < E; ++i) {
+      rst[w][i] = qt.template at<T>(rhot, w, i) * (-pw.inv_rho0s) + (T)1;
+      base[w][i] = qt.template at_once<T>(a.vre, w, i);
+    }
+  };
+  axis(std::integral_constant<int, 0>{});
+  axis(std::integral_constant<int, 1>{});
+  if constexpr ((PF & 2) != 0)
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        rst[w][i] = rst_at(w, i);
-        base[w][i] = vre_at(w, i);
-        bf_im(w, i);
-      }
-    c2r(a.in.p[3], nullptr);
+    for (int w = 0; w < 2; ++w) bf_div(w), base_w(w);
+  axis(std::integral_constant<int, 2>{});
+  // D_z J_z from the neighbouring points of both lines
+  using LY = rf::LayOf<T, N, pair_em<N>(), PairSync<N>>;
+  C dz[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) X[LY::pad(t + TPL * i)] = v[i];
+  PairSync<N>::sync();
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const int z = t + TPL * i;
+    dz[i] = cscale(csub(X[LY::pad((z + 1) & (N - 1))], X[LY::pad((z - 1) & (N - 1))]), pw.inv2h);
+  }
+  PairSync<N>::sync();
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    if constexpr ((PF & 2) == 0) base_w(w);
     if (act)
 #pragma unroll
       for (int i = 0; i < E; ++i)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) qt.template put<T>(a.vre, w, i, base[w][i] + kc_at(part(v[i], w), rst[w][i], w, i));
-  } else {
-    c2r(a.in.p[3], nullptr);
-    qt = q.here();
-    if (act)
-#pragma unroll
-      for (int i = 0; i < E; ++i)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          qt.template put<T>(a.vre, w, i, vre_at(w, i) + kc_at(part(v[i], w), rst_at(w, i), w, i));
-          bf_im(w, i);
-        }
+        q.template put<T>(a.vre, w, i, base[w][i] + (part(dz[i], w) * rst[w][i] * pw.ckc - t3[w][i] * (pw.ckc * pw.k23)));
   }
-  if constexpr (PART == 2) {
-    const auto qs = q.here();
 #pragma unroll
-    for (int i = 0; i < E; ++i) v[i] = cmk<C>(qs.template at_once<T>(a.hbuf, 0, i), qs.template at_once<T>(a.hbuf, 1, i));
-  } else {
-#pragma unroll
-    for (int i = 0; i < E; ++i) v[i] = cmk<C>(H[0][i], H[1][i]);
-  }
+  for (int i = 0; i < E; ++i) v[i] = cmk<C>(H[0][i], H[1][i]);
   r2c_store<T, N>(v, X, s_tw, t, a.out.p[0], p, P, act);
+  if constexpr ((PF & 2) == 0)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) bf_div(w);
 }
-template <typename T, int N, bool BF, int PART = 0>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZBC_MINB : (PART ? DFT_ZBC_SPLIT_MINB64 : DFT_ZBC_MINB64))
+template <typename T, int N, bool BF>
+__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZBC_MINB : DFT_ZBC_MINB64)
     k_zBC(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
-  zBC_body<T, N, BF, PART, false>(a, npairs, P, pw, g_tw);
+  zBC_body<T, N, BF, false>(a, npairs, P, pw, g_tw);
 }
-template <typename T, int N, int PART = 0>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZBC_MINB : (PART ? DFT_ZBC_SPLIT_MINB64 : DFT_ZBC_MINB64))
+template <typename T, int N>
+__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZBC_MINB : DFT_ZBC_MINB64)
     k_zBC_bfhd(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
-  zBC_body<T, N, true, PART, true>(a, npairs, P, pw, g_tw);
+  zBC_body<T, N, true, true>(a, npairs, P, pw, g_tw);
 }
 
 // -------------------------------------------------------------------- zC --
 struct ZCArgs {
   Ptrs8 in;              // summed linear terms (half spectrum)
   const void *vre, *vim;  // vim null without backflow
+  const void *jx, *jy, *rhot;  // KC: J_x, J_y (the x and y parts of term 1) and F*rho
   void *V;               // API mode: potential accumulated here
   // step mode
   const void *vext;      // real, may be null
@@ -1111,8 +980,9 @@ struct ZCArgs {
   double dtr, dti;
 };
 
-template <typename T, int N, bool STEP>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB : 0) k_zC(ZCArgs a, int64_t npairs, int P, const cplx<T> *__restrict__ g_tw) {
+template <typename T, int N, bool STEP, bool KC>
+__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB : 0)
+    k_zC(ZCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
   using C = cplx<T>;
   using G = LineCfg<T, N, pair_em<N>()>;
   constexpr int E = G::E, TPL = G::TPL, LP = G::LP;
@@ -1129,17 +999,40 @@ __global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB :
   C v[E];
   auto c2r_in = [&] { load_c2r<T, N>(v, X, s_tw, t, a.in.p[0], p, P); };
   const uint32_t cb = p * 2u * N + (uint32_t)t;
+  const PairPos<T, N, TPL> q(p, t, pw);
+  // the x and y parts of KC term 1, c rst (D_x J_x + D_y J_y), in two parts: the
+  // loads of line w, and its value at point i
+  T jd[KC ? 4 : 1][KC ? E : 1], rt[KC ? E : 1];
+  auto t1_fetch = [&](int w) {
+    if constexpr (KC) {
+      const auto qq = q.here();
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        jd[0][i] = qq.template nb<T, 0, 1>(a.jx, w, i);
+        jd[1][i] = qq.template nb<T, 0, -1>(a.jx, w, i);
+        jd[2][i] = qq.template nb<T, 1, 1>(a.jy, w, i);
+        jd[3][i] = qq.template nb<T, 1, -1>(a.jy, w, i);
+        rt[i] = qq.template at_once<T>(a.rhot, w, i);
+      }
+    }
+  };
+  auto t1 = [&](int i) {
+    if constexpr (KC)
+      return ((jd[0][i] - jd[1][i]) + (jd[2][i] - jd[3][i])) * pw.inv2h * (rt[i] * (-pw.inv_rho0s) + (T)1) * pw.ckc;
+    else return (T)0;
+  };
   if constexpr (!STEP) {
     c2r_in();
     const uint32_t c0 = cb + rf::opaque_zero();
-    if (act) {
 #pragma unroll
-      for (int i = 0; i < E; ++i)
+    for (int w = 0; w < 2; ++w) {
+      t1_fetch(w);
+      if (act)
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
+        for (int i = 0; i < E; ++i) {
           const int d = w * N + TPL * i;
           C u = rf::lde<C>(a.V, c0, d);
-          u.x += rf::lde<T>(a.vre, c0, d) + part(v[i], w);
+          u.x += (rf::lde<T>(a.vre, c0, d) + t1(i)) + part(v[i], w);
           u.y += a.vim ? rf::lde<T>(a.vim, c0, d) : (T)0;
           rf::ste<C>(a.V, c0, u, d);
         }
@@ -1150,6 +1043,7 @@ __global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB :
     T bre[E], bim[E], bex[E];
     C bav[E], bps[E];
     auto fetch = [&](int w) {
+      t1_fetch(w);
       const uint32_t c0 = cb + rf::opaque_zero();
 #pragma unroll
       for (int i = 0; i < E; ++i) {
@@ -1170,7 +1064,7 @@ __global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB :
       C u[E], ph[E], vs[E];  // ph: the potential of this half step (re-applied by the inverse z pass)
 #pragma unroll
       for (int i = 0; i < E; ++i) {
-        const T re = bre[i] + part(v[i], w);
+        const T re = (bre[i] + t1(i)) + part(v[i], w);
         const T im = bim[i];
         C ve = cmk<C>(re - (T)a.mu + bex[i], im);
         if (a.vsave) vs[i] = ve;

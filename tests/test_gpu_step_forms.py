@@ -74,6 +74,34 @@ def test_potential_nyquist_tiles(shape, model):
     p.free(), f.free(), w.free()
 
 
+@pytest.mark.parametrize("prec", [L.GRID_FP64, L.GRID_FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("model", [1, 9], ids=["kc", "full"])
+@pytest.mark.parametrize("shape", [(4, 4, 4), (4, 512, 8), (512, 4, 16), (8, 4, 512)], ids=lambda s: "x".join(map(str, s)))
+def test_kc_term1_differences(shape, model, prec):
+    """KC term 1 = c rst sum_d D_d J_d, its z part formed on the line and its x and y
+    parts by stencils of the next stage, where those wrap within a block, across the
+    longest axes and on lines of several wavefronts, against the oracle (which has no
+    potential for a box smaller than the Lennard-Jones core: NaN on both sides)."""
+    step = 0.9
+    o = po.OracleOT(model, shape, step, 2, 4)
+    psi = inputs.smooth_modulated(shape, step, o.p.rho0, 0.3)
+    w = L.Wave(shape, step, prec)
+    w.set(psi)
+    f, p = L.Functional(model, w, 2, 4), L.CField(shape, step, prec)
+    f.potential(p)
+    got, want = p.get(), o.potential(psi)
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), ok) and ok.all() == (min(shape) < max(shape))
+    got, want = got[ok], want[ok]
+    assert np.abs(got - want).max(initial=0) <= (1e-10 if prec == L.GRID_FP64 else 2e-5) * np.abs(want).max(initial=0)
+    p.free(), f.free(), w.free()
+
+
+def test_potential_forms_agree_512():
+    """The k-space sum of U*q4 where an FP64 x line has 512 points."""
+    test_potential_forms_agree((512, 64, 128), 1.0, L.GRID_FP64)
+
+
 def test_reverse_pass_work_space_is_reusable():
     """The reverse passes' kept work space: repeated and interleaved calls of two
     functionals, a sweep with more checkpoints than the one before, and two threads
