@@ -1251,40 +1251,19 @@ template <typename T, int N> void launch_zA(bool BF, const cplx<T> *psi, T *rho,
   DFT_PROF_END(s, "ot_zA_density_r2c", bytes);
 }
 
-// HB: the backflow density switch of HD / HD2 (k_zAB_bfhd)
-template <typename T, int N, bool KC, bool BF, bool HB = false>
-void launch_zAB1(const fused::ZABArgs &a, int64_t npairs, int P, const PW<T> &pw, const cplx<T> *tw, hipStream_t s) {
-  constexpr int LN = rf::LineCfg<T, N, fused::pair_em<N>()>::LINES;
-  const dim3 grid((unsigned)((npairs + LN - 1) / LN));
-  if constexpr (BF && (sizeof(T) == 8 ? DFT_ZAB_SPLIT64 : (HB ? DFT_ZAB_SPLIT32_HB : DFT_ZAB_SPLIT32))) {
-    // the backflow terms, then the local and KC terms (V_re through memory)
-    if constexpr (HB) {
-      hipLaunchKernelGGL((fused::k_zAB_bfhd<T, N, KC, 1>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-      DFT_LAUNCH_CHECK();
-      hipLaunchKernelGGL((fused::k_zAB_bfhd<T, N, KC, 2>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-    } else {
-      hipLaunchKernelGGL((fused::k_zAB<T, N, KC, BF, 1>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-      DFT_LAUNCH_CHECK();
-      hipLaunchKernelGGL((fused::k_zAB<T, N, KC, BF, 2>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-    }
-  } else if constexpr (HB) {
-    hipLaunchKernelGGL((fused::k_zAB_bfhd<T, N, KC>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-  } else {
-    hipLaunchKernelGGL((fused::k_zAB<T, N, KC, BF>), grid, dim3(fused::PairBS<T, N>), 0, s, a, npairs, P, pw, tw);
-  }
-}
-
 template <typename T, int N>
 void launch_zAB(bool KC, bool BF, const fused::ZABArgs &a, int64_t npairs, int P, const PW<T> &pw,
                 const cplx<T> *tw, hipStream_t s, double bytes) {
+  constexpr int LN = rf::LineCfg<T, N, fused::pair_em<N>()>::LINES;
+  const dim3 grid((unsigned)((npairs + LN - 1) / LN)), blk(fused::PairBS<T, N>);
   DFT_PROF_BEGIN(s);
   if (BF && pw.bfhd) {
-    if (KC) launch_zAB1<T, N, true, true, true>(a, npairs, P, pw, tw, s);
-    else launch_zAB1<T, N, false, true, true>(a, npairs, P, pw, tw, s);
-  } else if (KC && BF) launch_zAB1<T, N, true, true>(a, npairs, P, pw, tw, s);
-  else if (KC) launch_zAB1<T, N, true, false>(a, npairs, P, pw, tw, s);
-  else if (BF) launch_zAB1<T, N, false, true>(a, npairs, P, pw, tw, s);
-  else launch_zAB1<T, N, false, false>(a, npairs, P, pw, tw, s);
+    if (KC) hipLaunchKernelGGL((fused::k_zAB_bfhd<T, N, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
+    else hipLaunchKernelGGL((fused::k_zAB_bfhd<T, N, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  } else if (KC && BF) hipLaunchKernelGGL((fused::k_zAB<T, N, true, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  else if (KC) hipLaunchKernelGGL((fused::k_zAB<T, N, true, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  else if (BF) hipLaunchKernelGGL((fused::k_zAB<T, N, false, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  else hipLaunchKernelGGL((fused::k_zAB<T, N, false, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
   DFT_LAUNCH_CHECK();
   DFT_PROF_END(s, "ot_zAB_c2r_local_kc_bf_r2c", bytes);
 }

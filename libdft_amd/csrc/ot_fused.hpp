@@ -57,6 +57,7 @@ template <typename T, int N, int TPL> struct PairPos {
     ym0 = ((uint32_t)ix * pw.ny + ((j - 1) & (pw.ny - 1))) * N + t;
     yp1 = ((uint32_t)ix * pw.ny + ((j + 2) & (pw.ny - 1))) * N + t;
   }
+  static constexpr int kTPL = TPL;
   static constexpr int d(int w, int i) { return w * N + TPL * i; }
   // The same positions with offsets that the loads of the current stage
   // depend on (see rf::opaque_zero).
@@ -110,26 +111,6 @@ __device__ __forceinline__ T velocity_sab(const PW<T> &pw, T f, cplx<T> s, cplx<
   if (pw.clamp_v) v = clampv(v, pw.vmax);
   return v;
 }
-template <typename T, int D, class Q>
-__device__ __forceinline__ T velocity_d(const void *psi, const Q &q, int w, int i, const PW<T> &pw, T f,
-                                        cplx<T> s) {
-  return velocity_sab(pw, f, s, q.template nb<cplx<T>, D, 1>(psi, w, i), q.template nb<cplx<T>, D, -1>(psi, w, i));
-}
-template <typename T, int D, class Q>
-__device__ __forceinline__ T velocity_d(const void *psi, const Q &q, int w, int i, const PW<T> &pw, T f) {
-  return velocity_d<T, D>(psi, q, w, i, pw, f, q.template at<cplx<T>>(psi, w, i));
-}
-
-template <typename T, int D, class Q>
-__device__ __forceinline__ T grad_d(const void *f, const Q &q, int w, int i, const PW<T> &pw) {
-  return (q.template nb<T, D, 1>(f, w, i) - q.template nb<T, D, -1>(f, w, i)) * pw.inv2h;
-}
-// central difference of rho~ = G(rho) rho (backflow density switch)
-template <typename T, int D, class Q>
-__device__ __forceinline__ T grad_rt_d(const void *rho, const Q &q, int w, int i, const PW<T> &pw) {
-  return (bf_rt(q.template nb<T, D, 1>(rho, w, i), pw) - bf_rt(q.template nb<T, D, -1>(rho, w, i), pw)) * pw.inv2h;
-}
-
 // Pair kernels use the plan with the fewest points per thread, 4: a line is
 // one wavefront up to N = 256 and two at N = 512 (exchanges then take the
 // block barrier).
@@ -157,6 +138,43 @@ template <typename T, int N> constexpr int PairBS = LineCfg<T, N, pair_em<N>()>:
   __syncthreads();                                                           \
   const PairPos<T, N, TPL> q(p, t, pw)
 
+template <typename T> __device__ __forceinline__ T dens_of(cplx<T> s) { return s.x * s.x + s.y * s.y; }
+
+// Neighbours a (+) and b (-) along axis D of the kept values s of a pair (X: real
+// or complex).  Along y, line b is line a's neighbour and the other way round;
+// along z the neighbours are other lanes' values (lines within a wavefront):
+// point t + TPL i has z + 1 at lane t + 1 (index i), or at lane 0 (index i + 1)
+// for t = TPL - 1, z - 1 likewise, wrapping around the line.  Only x, and one
+// line each way along y, are loaded.
+__device__ __forceinline__ float lane_of(float x, int l, int w) { return __shfl(x, l, w); }
+__device__ __forceinline__ double lane_of(double x, int l, int w) { return __shfl(x, l, w); }
+__device__ __forceinline__ float2 lane_of(float2 x, int l, int w) { return make_float2(__shfl(x.x, l, w), __shfl(x.y, l, w)); }
+__device__ __forceinline__ double2 lane_of(double2 x, int l, int w) { return make_double2(__shfl(x.x, l, w), __shfl(x.y, l, w)); }
+template <int D, class X, class Q, int E>
+__device__ __forceinline__ void neighbours(const void *f, const Q &q, const X (&s)[2][E], int w, X (&a)[E], X (&b)[E]) {
+  constexpr int TPL = Q::kTPL;
+  if constexpr (D == 2 && TPL <= 64) {
+    const int up = (q.t + 1) & (TPL - 1), dn = (q.t + TPL - 1) & (TPL - 1);
+    X su[E], sd[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      su[i] = lane_of(s[w][i], up, TPL);
+      sd[i] = lane_of(s[w][i], dn, TPL);
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      a[i] = q.t == TPL - 1 ? su[(i + 1) % E] : su[i];
+      b[i] = q.t == 0 ? sd[(i + E - 1) % E] : sd[i];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      a[i] = D == 1 && w == 0 ? s[1][i] : q.template nb<X, D, 1>(f, w, i);
+      b[i] = D == 1 && w == 1 ? s[0][i] : q.template nb<X, D, -1>(f, w, i);
+    }
+  }
+}
+
 // Computes x here: arithmetic on registers whose result is needed only after
 // later stages is otherwise sunk past their branches, with its operands (the
 // loaded stencils) kept live in its place.
@@ -181,55 +199,23 @@ __device__ __forceinline__ void load_c2r(rf::Regs<T, N, pair_em<N>()> &v, cplx<T
 template <typename C> __device__ __forceinline__ auto &part(C &c, int w) { return w ? c.y : c.x; }
 
 // -------------------------------------------------------------------- zA --
-// waves per SIMD asked of the register allocator for the FP32 zA and zC
-// kernels (0: no request)
-#ifndef DFT_ZA_MINB
-#define DFT_ZA_MINB 5
-#endif
-#ifndef DFT_ZC_MINB
-#define DFT_ZC_MINB 0
-#endif
-// FP32 zA with backflow keeps psi of its points in registers for the three
-// velocity axes and q4 instead of reading psi and rho again (zA 158 -> 136 us at
-// 256^3, 5 waves per SIMD either way)
-#ifndef DFT_ZA_KEEP
-#define DFT_ZA_KEEP 1
-#endif
-// ... and takes the z neighbours of those points from the line's other lanes
-// (zA 135 -> 122 us at 256^3, bit-identical; at 4 waves per SIMD, where it
-// needs no spills)
-#ifndef DFT_ZA_ZSHFL
-#define DFT_ZA_ZSHFL 1
-#endif
-#ifndef DFT_ZA_MINB_SH
-#define DFT_ZA_MINB_SH 4
-#endif
-// the same for FP64 (132 -> 192 VGPRs, 3 -> 2 waves per SIMD; zA 257 -> 243 us
-// at 256^3)
-#ifndef DFT_ZA_KEEP64
-#define DFT_ZA_KEEP64 1
-#endif
-template <typename T, int N> constexpr int za_minb() {
-  return sizeof(T) != 4 ? 0 : (DFT_ZA_KEEP && DFT_ZA_ZSHFL && N <= 256 ? DFT_ZA_MINB_SH : DFT_ZA_MINB);
-}
+// Bound by the stores (psi in once, rho and five spectra out) and the loads of
+// the psi stencils: with psi of the points kept and the y neighbours taken from
+// the other line, 2.5 loads of psi per point instead of 5, zA 252 -> 214 us at
+// 256^3 FP64 (192 -> 161 VGPRs, 3 waves per SIMD), 131 -> 129 FP32.
 // HB: the backflow density switch of HD / HD2 (q_d = rho~ v_d, q4 = rho~ |v|^2
 // and a sixth output, the transform of rho~ = G rho)
 template <typename T, int N, bool BF, bool HB>
 __device__ __forceinline__ void zA_body(const cplx<T> *psi, T *rho, Ptrs8 outs, int64_t npairs, int P, PW<T> pw,
                                         const cplx<T> *__restrict__ g_tw) {
   FUSED_PAIR_SETUP();
-  // with backflow, psi of the points is kept for the three axes (KEEP: up to
-  // N = 256; at 512 FP32 it would spill) or read again
-  constexpr bool KEEP = BF && DFT_ZA_KEEP && (sizeof(T) == 4 || DFT_ZA_KEEP64) && N <= 256;
-  C v[E], sp[2][KEEP ? E : 1];
+  // with backflow, psi of the points is kept for the three axes and q4
+  C v[E], sp[2][E];
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    const C sa = q.template at<C>(psi, 0, i), sb = q.template at<C>(psi, 1, i);
-    if constexpr (KEEP) {
-      sp[0][i] = sa;
-      sp[1][i] = sb;
-    }
-    v[i] = cmk<C>(sa.x * sa.x + sa.y * sa.y, sb.x * sb.x + sb.y * sb.y);
+#pragma unroll
+    for (int w = 0; w < 2; ++w) sp[w][i] = q.template at<C>(psi, w, i);
+    v[i] = cmk<C>(dens_of<T>(sp[0][i]), dens_of<T>(sp[1][i]));
   }
   if (act) {
 #pragma unroll
@@ -249,7 +235,9 @@ __device__ __forceinline__ void zA_body(const cplx<T> *psi, T *rho, Ptrs8 outs, 
       if constexpr (HB) {
         rt[0][i] = bf_rt(v[i].x, pw);
         rt[1][i] = bf_rt(v[i].y, pw);
+        settle(rt[0][i]), settle(rt[1][i]);
       }
+      settle(fv[0][i]), settle(fv[1][i]);
     }
     r2c_store<T, N>(v, X, s_tw, t, outs.p[0], p, P, act);
     T v2[2][E];
@@ -257,47 +245,24 @@ __device__ __forceinline__ void zA_body(const cplx<T> *psi, T *rho, Ptrs8 outs, 
     for (int i = 0; i < E; ++i) v2[0][i] = v2[1][i] = 0;
     auto qd = [&](auto dtag) {
       constexpr int D = decltype(dtag)::value;
-      const auto qq = q.here();
-      // z neighbours of the kept points from the line's other lanes: point
-      // t + TPL i has z + 1 at lane t + 1 (index i), or at lane 0 (index i + 1)
-      // for t = TPL - 1; z - 1 likewise (wrapping around the line)
-      constexpr bool ZSH = KEEP && D == 2 && DFT_ZA_ZSHFL && TPL <= 64;
-      C zp[2][ZSH ? E : 1], zm[2][ZSH ? E : 1];
-      if constexpr (ZSH) {
-        const int up = (t + 1) & (TPL - 1), dn = (t + TPL - 1) & (TPL - 1);
+      T vr[2][E];
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          C su[E], sd[E];
+      for (int w = 0; w < 2; ++w) {
+        C na[E], nb[E];
+        neighbours<D>(psi, q.here(), sp, w, na, nb);
 #pragma unroll
-          for (int i = 0; i < E; ++i) {
-            su[i] = cmk<C>(__shfl(sp[w][i].x, up, TPL), __shfl(sp[w][i].y, up, TPL));
-            sd[i] = cmk<C>(__shfl(sp[w][i].x, dn, TPL), __shfl(sp[w][i].y, dn, TPL));
-          }
-#pragma unroll
-          for (int i = 0; i < E; ++i) {
-            zp[w][i] = t == TPL - 1 ? su[(i + 1) % E] : su[i];
-            zm[w][i] = t == 0 ? sd[(i + E - 1) % E] : sd[i];
-          }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < E; ++i) {
-        T o[2];
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          C s;
-          if constexpr (KEEP) s = sp[w][i];
-          else s = qq.template at<C>(psi, w, i);
-          T r = s.x * s.x + s.y * s.y;
-          if constexpr (HB) r = rt[w][i];
-          T vd;
-          if constexpr (ZSH) vd = velocity_sab(pw, fv[w][i], s, zp[w][i], zm[w][i]);
-          else vd = velocity_d<T, D>(psi, qq, w, i, pw, fv[w][i], s);
+        for (int i = 0; i < E; ++i) {
+          const T vd = velocity_sab(pw, fv[w][i], sp[w][i], na[i], nb[i]);
           v2[w][i] += vd * vd;
-          o[w] = vd * r;
+          vr[w][i] = vd * (HB ? rt[w][HB ? i : 0] : dens_of<T>(sp[w][i]));
         }
-        v[i] = cmk<C>(o[0], o[1]);
       }
+#pragma unroll
+      for (int i = 0; i < E; ++i) v[i] = cmk<C>(vr[0][i], vr[1][i]);
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int i = 0; i < E; ++i) settle(v2[w][i]);
       r2c_store<T, N>(v, X, s_tw, t, outs.p[1 + D], p, P, act);
     };
     qd(std::integral_constant<int, 0>{});
@@ -306,10 +271,7 @@ __device__ __forceinline__ void zA_body(const cplx<T> *psi, T *rho, Ptrs8 outs, 
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       if constexpr (HB) v[i] = cmk<C>(v2[0][i] * rt[0][i], v2[1][i] * rt[1][i]);
-      else if constexpr (KEEP)
-        v[i] = cmk<C>(v2[0][i] * (sp[0][i].x * sp[0][i].x + sp[0][i].y * sp[0][i].y),
-                      v2[1][i] * (sp[1][i].x * sp[1][i].x + sp[1][i].y * sp[1][i].y));
-      else v[i] = cmk<C>(v2[0][i] * q.template at<T>(rho, 0, i), v2[1][i] * q.template at<T>(rho, 1, i));
+      else v[i] = cmk<C>(v2[0][i] * dens_of<T>(sp[0][i]), v2[1][i] * dens_of<T>(sp[1][i]));
     }
     r2c_store<T, N>(v, X, s_tw, t, outs.p[4], p, P, act);
     if constexpr (HB) {
@@ -322,7 +284,7 @@ __device__ __forceinline__ void zA_body(const cplx<T> *psi, T *rho, Ptrs8 outs, 
   }
 }
 template <typename T, int N, bool BF>
-__global__ void __launch_bounds__((PairBS<T, N>), (za_minb<T, N>()))
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
     k_zA(const cplx<T> *psi, T *rho, Ptrs8 outs, int64_t npairs, int P, PW<T> pw,
          const cplx<T> *__restrict__ g_tw) {
   zA_body<T, N, BF, false>(psi, rho, outs, npairs, P, pw, g_tw);
@@ -523,61 +485,16 @@ __global__ void __launch_bounds__((XConvCfg<T, N, ONE>::BS), sizeof(T) == 4 ? DF
 }
 
 // ------------------------------------------------------------------- zAB --
-// minimum resident blocks per CU asked of the register allocator for the FP32
-// zAB / zBC kernels (0: none)
-#ifndef DFT_ZAB_MINB
-#define DFT_ZAB_MINB 0
-#endif
-#ifndef DFT_ZBC_MINB
-#define DFT_ZBC_MINB 2
-#endif
-// the same requests for the single FP64 kernels (0: none); zAB's is used when
-// the split form below is off
-#ifndef DFT_ZAB_MINB64
-#define DFT_ZAB_MINB64 0
-#endif
-#ifndef DFT_ZBC_MINB64
-#define DFT_ZBC_MINB64 2
-#endif
-// FP64 zAB (backflow) as two kernels (1) or one (0), and the waves per SIMD
-// asked for the halves (0: none).
-#ifndef DFT_ZAB_SPLIT64
-#define DFT_ZAB_SPLIT64 1
-#endif
-#ifndef DFT_ZAB_SPLIT_MINB64
-#define DFT_ZAB_SPLIT_MINB64 0
-#endif
-// (the zAB split in FP32, where neither half gets past 2 waves per SIMD without
-// spills, measured slower: zAB 375 -> 386 us at 256^3)
-#ifndef DFT_ZAB_SPLIT32
-#define DFT_ZAB_SPLIT32 0
-#endif
-// the same for the FP32 kernels with the HD / HD2 backflow switch (one wave per
-// SIMD in one kernel)
-#ifndef DFT_ZAB_SPLIT32_HB
-#define DFT_ZAB_SPLIT32_HB 1
-#endif
-// Early loads in zAB / zBC, so that memory round trips overlap the transforms
-// (bit masks, FP32; FP64 holds twice the registers and spills at its
-// occupancy, so it uses them only with DFT_PREFETCH64=1):
-//  1  a stage's stencils (velocity, density gradients) before its spectrum's transform;
-//  2  the density (zAB) / the accumulated fields (zBC) before the last transform;
-//  4  zAB: the KC density gradient along the next axis before the current r2c;
-//  8  the next stage's spectrum before the current stage's transform;
-// zC (bit 1): the fields of each line of the step before the preceding transform.
-#ifndef DFT_ZAB_PF
-#define DFT_ZAB_PF 15
-#endif
-#ifndef DFT_ZBC_PF
-#define DFT_ZBC_PF 11
-#endif
-#ifndef DFT_ZC_PF
-#define DFT_ZC_PF 1
-#endif
-#ifndef DFT_PREFETCH64
-#define DFT_PREFETCH64 0
-#endif
-template <typename T, int MASK> constexpr int prefetch_bits() { return (sizeof(T) == 4 || DFT_PREFETCH64) ? MASK : 0; }
+// Early loads in zAB, zBC and zC, so that memory round trips overlap the
+// transforms: the next stage's spectrum before the current stage's transform,
+// the density gradient along the next axis (zAB with KC alone) before the
+// current one, the accumulated fields (zBC) before the last transform, the
+// step's fields of a line (zC) before the preceding one.
+// FP32 only: FP64 holds twice the registers and gains nothing (zBC 433 and 443
+// us at 256^3, zAB with KC alone 68.3 and 70.5 at 128x128x256).  The stencils
+// are taken after the transforms: loaded before, they cost registers for
+// nothing (zAB 297 us at 256^3 FP32 either way, zBC 217 against 213).
+template <typename T> constexpr bool early_loads() { return sizeof(T) == 4; }
 
 // Pipelined c2r stages: the spectrum of the current stage was loaded into
 // `raw` earlier; the next stage's loads (if any) are issued before this
@@ -596,221 +513,215 @@ struct ZABArgs {
   void *rhot, *vre, *vim, *wx, *wy, *wz;
 };
 
-// PART 0: the whole stage; with backflow it may run as two kernels with fewer
-// live fields, PART 1 (the backflow terms, V_re stored) then PART 2 (the local
-// and KC terms, added to the stored V_re).
 // HB: the backflow density switch of HD / HD2 (A, B_d, C come from rho~; Re
 // V_BF is multiplied by d(G rho)/d rho, the gradient half of Im V_BF takes rho~).
-template <typename T, int N, bool KC, bool BF, int PART, bool HB>
+// Bound by its loads and stores: with KC and backflow 7 spectra and psi in, 4
+// spectra and 6 real fields out.  psi of the points is kept, and their density
+// and its neighbours' come from psi, so a point takes 4 loads of psi instead of
+// 9 of psi and 14 of rho; G_d is formed with the axis' velocity, from the same
+// stencil.  With the sums settled after each axis (settle) it takes 160 VGPRs in
+// FP32 (231 before) and, at two waves per SIMD, 247 in FP64 (two kernels of 256 +
+// 72 and 128 before).  Before and after at 256^3 (us): FP32 388 -> 297, FP64
+// 786 -> 516, FP32 with the switch at 256x128x256 261 -> 231.
+template <typename T, int N, bool KC, bool BF, bool HB>
 __device__ __forceinline__ void zAB_body(ZABArgs a, int64_t npairs, int P, PW<T> pw,
                                          const cplx<T> *__restrict__ g_tw) {
-  static_assert(PART == 0 || BF, "only the backflow stage splits");
   FUSED_PAIR_SETUP();
-  // (with the switch the stencils' exponentials would be held across the transform)
-  constexpr int PF = prefetch_bits<T, HB ? (DFT_ZAB_PF & ~1) : DFT_ZAB_PF>();
+  constexpr bool PF = early_loads<T>();
   constexpr int IA = KC ? 2 : 1;  // first backflow input
-  constexpr bool DO_BF = BF && PART != 2, DO_LOCAL = PART != 1;
-  const void *rho = a.rho;
+  const void *rho = a.rho, *psi = a.psi;
   C v[E];
   T vre[2][E];
   fft::RawPair<T, N, pair_em<N>()> raw;
-  // c2r of stage input `cur`, then (with bit 8) the loads of `next`
+  // c2r of stage input `cur`, then (with early loads) those of `next`
   auto c2r = [&](const void *cur, const void *next) {
-    if constexpr ((PF & 8) != 0) c2r_pipe<T, N>(v, raw, X, s_tw, t, next, p, P);
+    if constexpr (PF) c2r_pipe<T, N>(v, raw, X, s_tw, t, next, p, P);
     else load_c2r<T, N>(v, X, s_tw, t, cur, p, P);
   };
-  if constexpr ((PF & 8) != 0) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[DO_BF ? IA : 0], p, P, t);
-  if constexpr (PART == 2) {
-    const auto qv = q.here();
-#pragma unroll
-    for (int i = 0; i < E; ++i)
-#pragma unroll
-      for (int w = 0; w < 2; ++w) vre[w][i] = qv.template at_once<T>(a.vre, w, i);
-  }
-  if constexpr (DO_BF) {
-    // A = U*rho; per axis: B_d = U*q_d -> W_d = v_d A - B_d (stored),
-    // BF real part sum_d (v_d^2 A - 2 v_d B_d) + C, imaginary part sum_d (g_d/(rho+eps)) W_d / 2
-    T A[2][E], tr[2][E], im[2][E];
-    c2r(a.in.p[IA], a.in.p[IA + 1]);
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-      A[0][i] = v[i].x;
-      A[1][i] = v[i].y;
-    }
-    const void *psi = a.psi;
-    // velocity factor and 1 / (rho + eps) per point, kept for the three axes
-    T fv[2][E], fg[2][E], dg[2][HB ? E : 1];
-    {
-      const auto qr = q.here();
-#pragma unroll
-      for (int i = 0; i < E; ++i)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          const T r = qr.template at<T>(rho, w, i);
-          fv[w][i] = velocity_factor(pw, r);
-          fg[w][i] = (T)1 / (r + pw.div_eps);
-          if constexpr (HB) dg[w][i] = bf_dg(r, pw);
-        }
-    }
-    auto axis = [&](auto dtag) {
-      constexpr int D = decltype(dtag)::value;
-      void *wd = D == 0 ? a.wx : (D == 1 ? a.wy : a.wz);
-      // stencil positions taken after the transform unless prefetching, so
-      // that the compiler does not hoist those loads into it
-      std::remove_const_t<decltype(q)> qq;
-      if constexpr ((PF & 1) != 0) qq = q.here();
-      // velocity and (D_d rho)/(rho + eps) at point (w, i)
-      auto vg = [&](int w, int i, T &vd, T &gi) {
-        vd = velocity_d<T, D>(psi, qq, w, i, pw, fv[w][i]);
-        if constexpr (HB) gi = grad_rt_d<T, D>(rho, qq, w, i, pw) * fg[w][i];
-        else gi = grad_d<T, D>(rho, qq, w, i, pw) * fg[w][i];
-      };
-      T vds[2][E], gis[2][E];
-      if constexpr ((PF & 1) != 0)
-#pragma unroll
-        for (int i = 0; i < E; ++i)
-#pragma unroll
-          for (int w = 0; w < 2; ++w) vg(w, i, vds[w][i], gis[w][i]);
-      const void *next = D < 2 || a.in.p[IA + 4] ? a.in.p[D < 2 ? IA + 2 + D : IA + 4] : (DO_LOCAL ? a.in.p[0] : nullptr);
-      c2r(a.in.p[IA + 1 + D], next);
-      if constexpr ((PF & 1) == 0) qq = q.here();
-      T Wv[2][E];
-#pragma unroll
-      for (int i = 0; i < E; ++i) {
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          const T Bd = part(v[i], w);
-          T vd, gi;
-          if constexpr ((PF & 1) != 0) vd = vds[w][i], gi = gis[w][i];
-          else vg(w, i, vd, gi);
-          const T W = vd * A[w][i] - Bd;
-          Wv[w][i] = W;
-          const T ti = vd * vd * A[w][i] + (T)-2 * vd * Bd;
-          const T ii = (T)0.5 * gi * W;
-          if constexpr (D == 0) {
-            tr[w][i] = ti;
-            im[w][i] = ii;
-          } else {
-            tr[w][i] += ti;
-            im[w][i] += ii;
-          }
-        }
-      }
-      if (act)
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-          q.template put<T>(wd, 0, i, Wv[0][i]);
-          q.template put<T>(wd, 1, i, Wv[1][i]);
-        }
-    };
-    axis(std::integral_constant<int, 0>{});
-    axis(std::integral_constant<int, 1>{});
-    axis(std::integral_constant<int, 2>{});
-    const void *C_ = a.in.p[IA + 4];
-    if (C_) c2r(C_, DO_LOCAL ? a.in.p[0] : nullptr);
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-#pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        T re = tr[w][i];
-        if (C_) re += part(v[i], w);
-        if constexpr (HB) re = re * dg[w][i];
-        re = re * ((T)-0.5 * pw.mass);
-        if (pw.clamp_bf) re = clampv(re, pw.bfmax);
-        vre[w][i] = re * pw.cbf;
-      }
-    }
-    if (act)
-#pragma unroll
-      for (int i = 0; i < E; ++i) {
-        q.template put<T>(a.vim, 0, i, im[0][i]);
-        q.template put<T>(a.vim, 1, i, im[1][i]);
-      }
-  }
-  if constexpr (DO_LOCAL) {
-    // local correlation: rhobar = Pi*rho
-    std::remove_const_t<decltype(q)> ql;
-    T rl[2][E];
-    auto dens = [&] {
-      ql = q.here();
-#pragma unroll
-      for (int i = 0; i < E; ++i)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) rl[w][i] = ql.template at<T>(rho, w, i);
-    };
-    if constexpr ((PF & 2) != 0) dens();
-    c2r(a.in.p[0], KC ? a.in.p[1] : nullptr);
-    if constexpr ((PF & 2) == 0) dens();
+  if constexpr (PF) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[BF && KC ? 1 : (BF ? IA : 0)], p, P, t);
+  // local correlation: rhobar = Pi*rho, Q; r: the density at the points
+  auto local = [&](auto &&dens, const void *next) {
+    T r[2][E];
+    if constexpr (PF) dens(r);
+    c2r(a.in.p[0], next);
+    if constexpr (!PF) dens(r);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       T Q[2];
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
-        const T rb = part(v[i], w), r = rl[w][i];
+        const T rb = part(v[i], w);
         T loc = rb * rb * (pw.c2 * (T)0.5) + rb * rb * rb * (pw.c3 / (T)3);
-        if (pw.hdC != (T)0) loc += hd_pot(r, pw);
+        if (pw.hdC != (T)0) loc += hd_pot(r[w][i], pw);
         if constexpr (BF) vre[w][i] += loc;
         else vre[w][i] = loc;
-        Q[w] = (rb * pw.c2 + rb * rb * pw.c3) * r;
+        settle(vre[w][i]);
+        Q[w] = (rb * pw.c2 + rb * rb * pw.c3) * r[w][i];
       }
       v[i] = cmk<C>(Q[0], Q[1]);
     }
     r2c_store<T, N>(v, X, s_tw, t, a.out.p[0], p, P, act);
-    if constexpr (KC) {
-      // rhot = F*rho (stored), rho_st = 1 - rhot/rho_0s, G_d = (D_d rho) rho_st
-      T gn[2][E];
-      auto grad_next = [&](auto dtag) {
-        constexpr int D = decltype(dtag)::value;
-        const auto qq = q.here();
+  };
+  // rhot = F*rho (stored), rho_st = 1 - rhot/rho_0s
+  T rst[2][KC ? E : 1];
+  auto kc_rst = [&](const void *next) {
+    c2r(a.in.p[1], next);
 #pragma unroll
-        for (int i = 0; i < E; ++i)
+    for (int i = 0; i < E; ++i)
 #pragma unroll
-          for (int w = 0; w < 2; ++w) gn[w][i] = grad_d<T, D>(rho, qq, w, i, pw);
-      };
-      if constexpr ((PF & 4) != 0) grad_next(std::integral_constant<int, 0>{});
-      c2r(a.in.p[1], nullptr);
-      T rst[2][E];
-#pragma unroll
-      for (int i = 0; i < E; ++i) {
-#pragma unroll
-        for (int w = 0; w < 2; ++w) rst[w][i] = part(v[i], w) * (-pw.inv_rho0s) + (T)1;
+      for (int w = 0; w < 2; ++w) {
+        rst[w][i] = part(v[i], w) * (-pw.inv_rho0s) + (T)1;
+        if (act) q.template put<T>(a.rhot, w, i, part(v[i], w));
       }
-      if (act)
 #pragma unroll
-        for (int i = 0; i < E; ++i) {
-          q.template put<T>(a.rhot, 0, i, v[i].x);
-          q.template put<T>(a.rhot, 1, i, v[i].y);
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) settle(rst[w][i]);
+  };
+  // G_d = (D_d rho) rho_st
+  auto kc_g = [&](int dd, const T (&g)[2][E]) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) v[i] = cmk<C>(g[0][i] * rst[0][i], g[1][i] * rst[1][i]);
+    r2c_store<T, N>(v, X, s_tw, t, a.out.p[1 + dd], p, P, act);
+  };
+  if constexpr (BF) {
+    // A = U*rho; per axis: B_d = U*q_d -> W_d = v_d A - B_d (stored),
+    // BF real part sum_d (v_d^2 A - 2 v_d B_d) + C, imaginary part sum_d g_d W_d / (2 (rho+eps)).
+    // psi of the points is kept for the three axes; the densities of the
+    // neighbours are those of the psi that the velocities load.
+    C sp[2][E];
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) sp[w][i] = q.template at<C>(psi, w, i);
+    if constexpr (KC) kc_rst(a.in.p[IA]);
+    T A[2][E], tr[2][E], im[2][E];
+    c2r(a.in.p[IA], a.in.p[IA + 1]);
+    // velocity factor per point, kept for the three axes
+    T fv[2][E];
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        A[w][i] = part(v[i], w);
+        fv[w][i] = velocity_factor(pw, dens_of<T>(sp[w][i]));
+        settle(fv[w][i]);
+      }
+    auto axis = [&](auto dtag) {
+      constexpr int D = decltype(dtag)::value;
+      void *wd = D == 0 ? a.wx : (D == 1 ? a.wy : a.wz);
+      // velocity, density gradient (KC) and gradient of the backflow density
+      T vd[2][E], g[2][E], gb[2][HB ? E : 1];
+      auto stencil = [&] {
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          C na[E], nb[E];
+          neighbours<D>(psi, q.here(), sp, w, na, nb);
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            vd[w][i] = velocity_sab(pw, fv[w][i], sp[w][i], na[i], nb[i]);
+            const T ra = dens_of<T>(na[i]), rb = dens_of<T>(nb[i]);
+            g[w][i] = (ra - rb) * pw.inv2h;
+            if constexpr (HB) gb[w][i] = (bf_rt(ra, pw) - bf_rt(rb, pw)) * pw.inv2h;
+            settle(vd[w][i]), settle(g[w][i]);
+            if constexpr (HB) settle(gb[w][i]);
+          }
         }
-      auto gd = [&](auto dtag) {
-        constexpr int D = decltype(dtag)::value;
-        if constexpr ((PF & 4) == 0) grad_next(dtag);
+      };
+      const void *next = D < 2 || a.in.p[IA + 4] ? a.in.p[D < 2 ? IA + 2 + D : IA + 4] : a.in.p[0];
+      c2r(a.in.p[IA + 1 + D], next);
+      stencil();
 #pragma unroll
-        for (int i = 0; i < E; ++i) v[i] = cmk<C>(gn[0][i] * rst[0][i], gn[1][i] * rst[1][i]);
-        if constexpr ((PF & 4) != 0 && D < 2) grad_next(std::integral_constant<int, D + 1>{});
+      for (int i = 0; i < E; ++i)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const T Bd = part(v[i], w), vw = vd[w][i];
+          const T W = vw * A[w][i] - Bd;
+          const T ti = vw * vw * A[w][i] + (T)-2 * vw * Bd;
+          const T ii = (HB ? gb[w][HB ? i : 0] : g[w][i]) * W;
+          tr[w][i] = D == 0 ? ti : tr[w][i] + ti;
+          im[w][i] = D == 0 ? ii : im[w][i] + ii;
+          settle(tr[w][i]), settle(im[w][i]);
+          if (act) q.template put<T>(wd, w, i, W);
+        }
+      if constexpr (KC) kc_g(D, g);
+    };
+    axis(std::integral_constant<int, 0>{});
+    axis(std::integral_constant<int, 1>{});
+    axis(std::integral_constant<int, 2>{});
+    const void *C_ = a.in.p[IA + 4];
+    if (C_) c2r(C_, a.in.p[0]);
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        T re = tr[w][i];
+        if (C_) re += part(v[i], w);
+        const T r = dens_of<T>(sp[w][i]);
+        if constexpr (HB) re = re * bf_dg(r, pw);
+        re = re * ((T)-0.5 * pw.mass);
+        if (pw.clamp_bf) re = clampv(re, pw.bfmax);
+        vre[w][i] = re * pw.cbf;
+        settle(vre[w][i]);
+        if (act) q.template put<T>(a.vim, w, i, im[w][i] * ((T)0.5 / (r + pw.div_eps)));
+      }
+    local([&](T (&r)[2][E]) {
+#pragma unroll
+      for (int i = 0; i < E; ++i)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) r[w][i] = dens_of<T>(sp[w][i]);
+    }, nullptr);
+  } else {
+    T rl[2][E];
+    local([&](T (&r)[2][E]) {
+      const auto ql = q.here();
+#pragma unroll
+      for (int i = 0; i < E; ++i)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) rl[w][i] = r[w][i] = ql.template at<T>(rho, w, i);
+    }, KC ? a.in.p[1] : nullptr);
+    if constexpr (KC) {
+      T g[2][E];
+      auto grad = [&](auto dtag) {
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          T na[E], nb[E];
+          neighbours<decltype(dtag)::value>(rho, q.here(), rl, w, na, nb);
+#pragma unroll
+          for (int i = 0; i < E; ++i) g[w][i] = (na[i] - nb[i]) * pw.inv2h;
+        }
+      };
+      if constexpr (PF) grad(std::integral_constant<int, 0>{});
+      kc_rst(nullptr);
+      auto axis = [&](auto dtag) {
+        constexpr int D = decltype(dtag)::value;
+        if constexpr (!PF) grad(dtag);
+#pragma unroll
+        for (int i = 0; i < E; ++i) v[i] = cmk<C>(g[0][i] * rst[0][i], g[1][i] * rst[1][i]);
+        if constexpr (PF && D < 2) grad(std::integral_constant<int, D + 1>{});
         r2c_store<T, N>(v, X, s_tw, t, a.out.p[1 + D], p, P, act);
       };
-      gd(std::integral_constant<int, 0>{});
-      gd(std::integral_constant<int, 1>{});
-      gd(std::integral_constant<int, 2>{});
+      axis(std::integral_constant<int, 0>{});
+      axis(std::integral_constant<int, 1>{});
+      axis(std::integral_constant<int, 2>{});
     }
   }
-  if (act) {
+  if (act)
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       q.template put<T>(a.vre, 0, i, vre[0][i]);
       q.template put<T>(a.vre, 1, i, vre[1][i]);
     }
-  }
 }
-template <typename T, int N, bool KC, bool BF, int PART = 0>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZAB_MINB : (PART ? DFT_ZAB_SPLIT_MINB64 : DFT_ZAB_MINB64))
+template <typename T, int N, bool KC, bool BF>
+__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? 0 : 2)
     k_zAB(ZABArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
-  zAB_body<T, N, KC, BF, PART, false>(a, npairs, P, pw, g_tw);
+  zAB_body<T, N, KC, BF, false>(a, npairs, P, pw, g_tw);
 }
-template <typename T, int N, bool KC, int PART = 0>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZAB_MINB : (PART ? DFT_ZAB_SPLIT_MINB64 : DFT_ZAB_MINB64))
+template <typename T, int N, bool KC>
+__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? 0 : 2)
     k_zAB_bfhd(ZABArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
-  zAB_body<T, N, KC, true, PART, true>(a, npairs, P, pw, g_tw);
+  zAB_body<T, N, KC, true, true>(a, npairs, P, pw, g_tw);
 }
 
 // ------------------------------------------------------------------- zBC --
@@ -828,45 +739,45 @@ struct ZBCArgs {
 // and J_y are stored for the stencils of zC.  Against a fourth transform for
 // the sum, at 256^3 FP32 (us): x-middle 184 -> 116, a y pass of 24 and a z
 // transform less, zC 105 -> 133; 32x32x64 FP32 step 91 -> 83.5.
-// Bound by the loads: 3 spectra and 7 real fields with stencils.  With the sums
-// settled after each axis the kernel takes 114 VGPRs in FP32 (176 without; 4
-// waves per SIMD for 2; zBC 268 -> 225 us at 256^3) and 128 in FP64 (256 and
-// spills, or two kernels with H in memory between them, 547 -> 453 us).
-// Every stage first issues the loads that do not depend on its spectrum (the
-// stencils of rho and rho~, the fields accumulated into), so that their
-// latency overlaps the spectrum's loads and transform.
+// Bound by the loads: 3 spectra and 7 real fields with stencils (rho and rho~ of
+// the points kept for theirs).  With the sums settled after each axis the kernel
+// takes 109 VGPRs in FP32 (176 without; 4 waves per SIMD for 2; zBC 268 -> 213
+// us at 256^3) and 144 in FP64 (256 and spills, or two kernels with H in memory
+// between them, 547 -> 433 us).
 // HB: the backflow density switch of HD / HD2 (the divergence half of Im V_BF
 // is multiplied by G(rho)).
 template <typename T, int N, bool BF, bool HB>
 __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T> pw,
                                          const cplx<T> *__restrict__ g_tw) {
   FUSED_PAIR_SETUP();
-  constexpr int PF = prefetch_bits<T, DFT_ZBC_PF>();
+  constexpr bool PF = early_loads<T>();
   const void *rho = a.rho, *rhot = a.rhot;
   C v[E];
   T H[2][E], t3[2][E];
   fft::RawPair<T, N, pair_em<N>()> raw;
   auto c2r = [&](const void *cur, const void *next) {
-    if constexpr ((PF & 8) != 0) c2r_pipe<T, N>(v, raw, X, s_tw, t, next, p, P);
+    if constexpr (PF) c2r_pipe<T, N>(v, raw, X, s_tw, t, next, p, P);
     else load_c2r<T, N>(v, X, s_tw, t, cur, p, P);
   };
-  if constexpr ((PF & 8) != 0) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[0], p, P, t);
+  if constexpr (PF) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[0], p, P, t);
+  // rho and rho~ of the points, kept for the stencils of the three axes
+  T sr[2][E], st[2][E];
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      sr[w][i] = q.template at<T>(rho, w, i);
+      st[w][i] = q.template at<T>(rhot, w, i);
+    }
   auto axis = [&](auto dtag) {
     constexpr int D = decltype(dtag)::value;
-    T g[2][E], Pd[2][E];
-    auto grad_w = [&](int w) {
-      const auto qq = q.here();
+    T g[E];
+    auto diff_w = [&](const void *f, const T (&s)[2][E], int w, T (&out)[E]) {
+      T na[E], nb[E];
+      neighbours<D>(f, q.here(), s, w, na, nb);
 #pragma unroll
-      for (int i = 0; i < E; ++i) g[w][i] = grad_d<T, D>(rho, qq, w, i, pw);
+      for (int i = 0; i < E; ++i) out[i] = (na[i] - nb[i]) * pw.inv2h;
     };
-    auto pd_w = [&](int w) {
-      const auto qq = q.here();
-#pragma unroll
-      for (int i = 0; i < E; ++i) Pd[w][i] = grad_d<T, D>(rhot, qq, w, i, pw);  // (dF_d * rho) = D_d (F * rho)
-    };
-    if constexpr ((PF & 1) != 0)
-#pragma unroll
-      for (int w = 0; w < 2; ++w) grad_w(w), pd_w(w);
     c2r(a.in.p[D], D < 2 ? a.in.p[D + 1] : nullptr);
     if constexpr (D < 2)
       if (act)
@@ -874,56 +785,48 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
         for (int i = 0; i < E; ++i)
 #pragma unroll
           for (int w = 0; w < 2; ++w) q.template put<T>(D == 0 ? a.jx : a.jy, w, i, part(v[i], w));
-    // without prefetching, the stencils of one line and field at a time
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-      if constexpr ((PF & 1) == 0) grad_w(w);
+      diff_w(rho, sr, w, g);
 #pragma unroll
-      for (int i = 0; i < E; ++i) H[w][i] = D == 0 ? g[w][i] * part(v[i], w) : H[w][i] + g[w][i] * part(v[i], w);
-    }
+      for (int i = 0; i < E; ++i) H[w][i] = D == 0 ? g[i] * part(v[i], w) : H[w][i] + g[i] * part(v[i], w);
+      diff_w(rhot, st, w, g);  // (dF_d * rho) = D_d (F * rho)
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
-      if constexpr ((PF & 1) == 0) pd_w(w);
-#pragma unroll
-      for (int i = 0; i < E; ++i) t3[w][i] = D == 0 ? Pd[w][i] * part(v[i], w) : t3[w][i] + Pd[w][i] * part(v[i], w);
+      for (int i = 0; i < E; ++i) t3[w][i] = D == 0 ? g[i] * part(v[i], w) : t3[w][i] + g[i] * part(v[i], w);
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w)
 #pragma unroll
       for (int i = 0; i < E; ++i) settle(H[w][i]), settle(t3[w][i]);
   };
-  // the backflow divergence, and V_re so far and rho_st (both before J_z's
-  // transform with prefetching)
-  auto bf_div = [&](int w) {
-    if constexpr (BF) {
-      const auto qt = q.here();
+  // the backflow divergence and V_re so far, with early loads before J_z's transform
+  auto bf_div = [&] {
+    if constexpr (BF)
 #pragma unroll
-      for (int i = 0; i < E; ++i) {
-        T im = qt.template at_once<T>(a.vim, w, i);
-        T gw = (T)1;
-        if constexpr (HB) gw = bf_g(qt.template at<T>(rho, w, i), pw);
-        im += (T)0.5 * (((qt.template nb<T, 0, 1>(a.wx, w, i) - qt.template nb<T, 0, -1>(a.wx, w, i)) * pw.inv2h) * gw);
-        im += (T)0.5 * (((qt.template nb<T, 1, 1>(a.wy, w, i) - qt.template nb<T, 1, -1>(a.wy, w, i)) * pw.inv2h) * gw);
-        im += (T)0.5 * (((qt.template nb<T, 2, 1>(a.wz, w, i) - qt.template nb<T, 2, -1>(a.wz, w, i)) * pw.inv2h) * gw);
-        if (pw.clamp_bf) im = clampv(im, pw.bfmax);
-        if (act) qt.template put<T>(a.vim, w, i, im * pw.cbf);
+      for (int w = 0; w < 2; ++w) {
+        const auto qt = q.here();
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          T im = qt.template at_once<T>(a.vim, w, i);
+          T gw = (T)1;
+          if constexpr (HB) gw = bf_g(sr[w][i], pw);
+          im += (T)0.5 * (((qt.template nb<T, 0, 1>(a.wx, w, i) - qt.template nb<T, 0, -1>(a.wx, w, i)) * pw.inv2h) * gw);
+          im += (T)0.5 * (((qt.template nb<T, 1, 1>(a.wy, w, i) - qt.template nb<T, 1, -1>(a.wy, w, i)) * pw.inv2h) * gw);
+          im += (T)0.5 * (((qt.template nb<T, 2, 1>(a.wz, w, i) - qt.template nb<T, 2, -1>(a.wz, w, i)) * pw.inv2h) * gw);
+          if (pw.clamp_bf) im = clampv(im, pw.bfmax);
+          if (act) qt.template put<T>(a.vim, w, i, im * pw.cbf);
+        }
       }
-    }
   };
-  T rst[2][E], base[2][E];
+  T base[2][E];
   auto base_w = [&](int w) {
     const auto qt = q.here();
 #pragma unroll
-    for (int i = 0; i < E; ++i) {
-      rst[w][i] = qt.template at<T>(rhot, w, i) * (-pw.inv_rho0s) + (T)1;
-      base[w][i] = qt.template at_once<T>(a.vre, w, i);
-    }
+    for (int i = 0; i < E; ++i) base[w][i] = qt.template at_once<T>(a.vre, w, i);
   };
   axis(std::integral_constant<int, 0>{});
   axis(std::integral_constant<int, 1>{});
-  if constexpr ((PF & 2) != 0)
-#pragma unroll
-    for (int w = 0; w < 2; ++w) bf_div(w), base_w(w);
+  if constexpr (PF) bf_div(), base_w(0), base_w(1);
   axis(std::integral_constant<int, 2>{});
   // D_z J_z from the neighbouring points of both lines
   using LY = rf::LayOf<T, N, pair_em<N>(), PairSync<N>>;
@@ -939,26 +842,25 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
   PairSync<N>::sync();
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
-    if constexpr ((PF & 2) == 0) base_w(w);
-    if (act)
+    if constexpr (!PF) base_w(w);
 #pragma unroll
-      for (int i = 0; i < E; ++i)
-        q.template put<T>(a.vre, w, i, base[w][i] + (part(dz[i], w) * rst[w][i] * pw.ckc - t3[w][i] * (pw.ckc * pw.k23)));
+    for (int i = 0; i < E; ++i) {
+      const T rst = st[w][i] * (-pw.inv_rho0s) + (T)1;
+      if (act) q.template put<T>(a.vre, w, i, base[w][i] + (part(dz[i], w) * rst * pw.ckc - t3[w][i] * (pw.ckc * pw.k23)));
+    }
   }
 #pragma unroll
   for (int i = 0; i < E; ++i) v[i] = cmk<C>(H[0][i], H[1][i]);
   r2c_store<T, N>(v, X, s_tw, t, a.out.p[0], p, P, act);
-  if constexpr ((PF & 2) == 0)
-#pragma unroll
-    for (int w = 0; w < 2; ++w) bf_div(w);
+  if constexpr (!PF) bf_div();
 }
 template <typename T, int N, bool BF>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZBC_MINB : DFT_ZBC_MINB64)
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
     k_zBC(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
   zBC_body<T, N, BF, false>(a, npairs, P, pw, g_tw);
 }
 template <typename T, int N>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZBC_MINB : DFT_ZBC_MINB64)
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
     k_zBC_bfhd(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
   zBC_body<T, N, true, true>(a, npairs, P, pw, g_tw);
 }
@@ -981,7 +883,7 @@ struct ZCArgs {
 };
 
 template <typename T, int N, bool STEP, bool KC>
-__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB : 0)
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
     k_zC(ZCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
   using C = cplx<T>;
   using G = LineCfg<T, N, pair_em<N>()>;
@@ -995,7 +897,7 @@ __global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? DFT_ZC_MINB :
   C *X = s_x + ln * LP;
   rf::load_tw<T, N, G::EM, G::BS>(s_tw, g_tw);
   __syncthreads();
-  constexpr bool PF = prefetch_bits<T, DFT_ZC_PF>() != 0;
+  constexpr bool PF = early_loads<T>();
   C v[E];
   auto c2r_in = [&] { load_c2r<T, N>(v, X, s_tw, t, a.in.p[0], p, P); };
   const uint32_t cb = p * 2u * N + (uint32_t)t;
