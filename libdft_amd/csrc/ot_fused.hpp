@@ -995,5 +995,181 @@ __global__ void __launch_bounds__((PairBS<T, N>), 0)
   }
 }
 
+// -------------------------------------------------------------------- zE --
+struct ZEArgs {
+  Ptrs8 in;   // LJ*rho, rhobar, [rhot], [A, B_x, B_y, B_z, C]; k_zE2: J_x, J_y, J_z
+  Ptrs8 out;  // [G_x, G_y, G_z]
+  const void *rho, *psi;
+  void *rhot, *eps;
+};
+
+// The energy density without its KC part, from the convolutions of zA's fields:
+// local terms, backflow -m c_bf/4 (A v^2 + C) rho + m c_bf/2 sum_d B_d rho v_d
+// (rho~ = G rho in place of rho with the switch, HB), and the r2c of G_d =
+// (D_d rho) rho_st.  In this way no convolution, velocity or gradient goes
+// through memory as a real field.  psi (with KC alone: rho) of the points is
+// kept for the stencils, as in zAB; bound by the loads of the spectra.
+template <typename T, int N, bool KC, bool BF, bool HB>
+__device__ __forceinline__ void zE_body(ZEArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
+  FUSED_PAIR_SETUP();
+  constexpr bool PF = early_loads<T>();
+  constexpr int IA = KC ? 3 : 2;  // first backflow input
+  C v[E];
+  fft::RawPair<T, N, pair_em<N>()> raw;
+  auto c2r = [&](const void *cur, const void *next) {
+    if constexpr (PF) c2r_pipe<T, N>(v, raw, X, s_tw, t, next, p, P);
+    else load_c2r<T, N>(v, X, s_tw, t, cur, p, P);
+  };
+  if constexpr (PF) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[KC ? 2 : (BF ? IA + 1 : 0)], p, P, t);
+  // psi of the points (backflow), or their density
+  using S = std::conditional_t<BF, C, T>;
+  const void *src = BF ? a.psi : a.rho;
+  S sp[2][E];
+  T e[2][E], rst[2][KC ? E : 1];
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      sp[w][i] = q.template at<S>(src, w, i);
+      e[w][i] = 0;
+    }
+  auto dens = [&](const S &s) {
+    if constexpr (BF) return dens_of<T>(s);
+    else return s;
+  };
+  if constexpr (KC) {
+    c2r(a.in.p[2], BF ? a.in.p[IA + 1] : a.in.p[0]);
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        rst[w][i] = part(v[i], w) * (-pw.inv_rho0s) + (T)1;
+        settle(rst[w][i]);
+        if (act) q.template put<T>(a.rhot, w, i, part(v[i], w));
+      }
+  }
+  const T mq = pw.cbf * pw.mass * (T)0.25, mh = pw.cbf * pw.mass * (T)0.5;
+  T fv[2][BF ? E : 1], rw[2][BF ? E : 1], v2[2][BF ? E : 1];
+  if constexpr (BF)
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const T r = dens(sp[w][i]);
+        fv[w][i] = velocity_factor(pw, r);
+        rw[w][i] = HB ? bf_rt(r, pw) : r;
+        v2[w][i] = 0;
+        settle(fv[w][i]), settle(rw[w][i]);
+      }
+  auto axis = [&](auto dtag) {
+    constexpr int D = decltype(dtag)::value;
+    if constexpr (BF) c2r(a.in.p[IA + 1 + D], a.in.p[D < 2 ? IA + 2 + D : IA]);
+    T g[2][E];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      S na[E], nb[E];
+      neighbours<D>(src, q.here(), sp, w, na, nb);
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        if constexpr (BF) {
+          const T vd = velocity_sab(pw, fv[w][i], sp[w][i], na[i], nb[i]);
+          v2[w][i] += vd * vd;
+          e[w][i] += mh * (part(v[i], w) * rw[w][i] * vd);
+          settle(v2[w][i]), settle(e[w][i]);
+        }
+        if constexpr (KC) g[w][i] = (dens(na[i]) - dens(nb[i])) * pw.inv2h * rst[w][i];
+      }
+    }
+    if constexpr (KC) {
+#pragma unroll
+      for (int i = 0; i < E; ++i) v[i] = cmk<C>(g[0][i], g[1][i]);
+      r2c_store<T, N>(v, X, s_tw, t, a.out.p[D], p, P, act);
+    }
+  };
+  if constexpr (KC || BF) {
+    axis(std::integral_constant<int, 0>{});
+    axis(std::integral_constant<int, 1>{});
+    axis(std::integral_constant<int, 2>{});
+  }
+  // the remaining convolutions, each weighted with a field at the points
+  auto add = [&](const void *cur, const void *next, auto &&f) {
+    c2r(cur, next);
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        e[w][i] += f(w, i, part(v[i], w));
+        settle(e[w][i]);
+      }
+  };
+  if constexpr (BF) {
+    add(a.in.p[IA], a.in.p[IA + 4], [&](int w, int i, T A) { return -mq * (A * v2[w][i] * rw[w][i]); });
+    add(a.in.p[IA + 4], a.in.p[0], [&](int w, int i, T c) { return -mq * (c * rw[w][i]); });
+  }
+  add(a.in.p[0], a.in.p[1], [&](int w, int i, T lj) { return (T)0.5 * dens(sp[w][i]) * lj; });
+  add(a.in.p[1], nullptr, [&](int w, int i, T rb) {
+    const T r = dens(sp[w][i]);
+    T loc = (pw.c2 * (T)0.5) * (rb * rb * r) + (pw.c3 / (T)3) * (rb * rb * rb * r);
+    if (pw.hdC != (T)0) loc += hd_eps(r, pw);
+    return loc;
+  });
+  if (act)
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) q.template put<T>(a.eps, w, i, e[w][i]);
+}
+template <typename T, int N, bool KC, bool BF, bool HB>
+__global__ void __launch_bounds__((PairBS<T, N>), sizeof(T) == 4 ? 0 : 2)
+    k_zE(ZEArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
+  zE_body<T, N, KC, BF, HB>(a, npairs, P, pw, g_tw);
+}
+
+// KC part of the energy density: eps -= (alpha_s / 4m) rho_st sum_d (D_d rho) J_d
+template <typename T, int N>
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
+    k_zE2(ZEArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
+  FUSED_PAIR_SETUP();
+  constexpr bool PF = early_loads<T>();
+  C v[E];
+  T sr[2][E], H[2][E];
+  fft::RawPair<T, N, pair_em<N>()> raw;
+  if constexpr (PF) fft::load_raw<T, N, pair_em<N>()>(raw, a.in.p[0], p, P, t);
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      sr[w][i] = q.template at<T>(a.rho, w, i);
+      H[w][i] = 0;
+    }
+  auto axis = [&](auto dtag) {
+    constexpr int D = decltype(dtag)::value;
+    if constexpr (PF) c2r_pipe<T, N>(v, raw, X, s_tw, t, D < 2 ? a.in.p[D + 1] : nullptr, p, P);
+    else load_c2r<T, N>(v, X, s_tw, t, a.in.p[D], p, P);
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      T na[E], nb[E];
+      neighbours<D>(a.rho, q.here(), sr, w, na, nb);
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        H[w][i] += (na[i] - nb[i]) * pw.inv2h * part(v[i], w);
+        settle(H[w][i]);
+      }
+    }
+  };
+  axis(std::integral_constant<int, 0>{});
+  axis(std::integral_constant<int, 1>{});
+  axis(std::integral_constant<int, 2>{});
+  const auto qt = q.here();
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const T rst = qt.template at_once<T>(a.rhot, w, i) * (-pw.inv_rho0s) + (T)1;
+      const T e = qt.template at_once<T>(a.eps, w, i) - (T)0.5 * pw.ckc * (rst * H[w][i]);
+      if (act) qt.template put<T>(a.eps, w, i, e);
+    }
+}
+
 }  // namespace fused
 }  // namespace dft

@@ -102,6 +102,24 @@ def test_potential_forms_agree_512():
     test_potential_forms_agree((512, 64, 128), 1.0, L.GRID_FP64)
 
 
+@pytest.mark.parametrize("prec", [L.GRID_FP64, L.GRID_FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("model", [0, 1, 8, 9, 10, 11], ids=["plain", "kc", "bf", "full", "hd-bf", "hd-full"])
+@pytest.mark.parametrize("shape", [(4, 512, 8), (512, 4, 16), (8, 4, 512), (32, 16, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_energy_density_of_a_wave_function(shape, model, prec):
+    """dft_ot_energy_density (stages fused into the z transforms) at short and long
+    axes, lines of part of a wavefront and of several, against the oracle."""
+    step = 0.9
+    o = po.OracleOT(model, shape, step, 2, 4)
+    psi = inputs.smooth_modulated(shape, step, o.p.rho0, 0.3)
+    w, e = L.Wave(shape, step, prec), L.RField(shape, step, prec)
+    w.set(psi)
+    f = L.Functional(model, w, 2, 4)
+    f.energy_density(e)
+    want = o.energy_density(psi)
+    assert np.abs(e.get() - want).max() <= (1e-10 if prec == L.GRID_FP64 else 2e-5) * np.abs(want).max()
+    f.free(), e.free(), w.free()
+
+
 def test_reverse_pass_work_space_is_reusable():
     """The reverse passes' kept work space: repeated and interleaved calls of two
     functionals, a sweep with more checkpoints than the one before, and two threads
