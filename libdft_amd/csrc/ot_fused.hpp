@@ -746,7 +746,9 @@ struct ZBCArgs {
 // between them, 547 -> 433 us).
 // HB: the backflow density switch of HD / HD2 (the divergence half of Im V_BF
 // is multiplied by G(rho)).
-template <typename T, int N, bool BF, bool HB>
+// GRAD: the energy gradient's form, c sum_d D_d (rst J_d) without term 3: rst J_x
+// and rst J_y are stored, the z part added to V_re.
+template <typename T, int N, bool BF, bool HB, bool GRAD>
 __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T> pw,
                                          const cplx<T> *__restrict__ g_tw) {
   FUSED_PAIR_SETUP();
@@ -769,6 +771,7 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
       sr[w][i] = q.template at<T>(rho, w, i);
       st[w][i] = q.template at<T>(rhot, w, i);
     }
+  auto rst = [&](int w, int i) { return st[w][i] * (-pw.inv_rho0s) + (T)1; };
   auto axis = [&](auto dtag) {
     constexpr int D = decltype(dtag)::value;
     T g[E];
@@ -784,20 +787,26 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
 #pragma unroll
         for (int i = 0; i < E; ++i)
 #pragma unroll
-          for (int w = 0; w < 2; ++w) q.template put<T>(D == 0 ? a.jx : a.jy, w, i, part(v[i], w));
+          for (int w = 0; w < 2; ++w)
+            q.template put<T>(D == 0 ? a.jx : a.jy, w, i, GRAD ? rst(w, i) * part(v[i], w) : part(v[i], w));
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
       diff_w(rho, sr, w, g);
 #pragma unroll
       for (int i = 0; i < E; ++i) H[w][i] = D == 0 ? g[i] * part(v[i], w) : H[w][i] + g[i] * part(v[i], w);
-      diff_w(rhot, st, w, g);  // (dF_d * rho) = D_d (F * rho)
+      if constexpr (!GRAD) {
+        diff_w(rhot, st, w, g);  // (dF_d * rho) = D_d (F * rho)
 #pragma unroll
-      for (int i = 0; i < E; ++i) t3[w][i] = D == 0 ? g[i] * part(v[i], w) : t3[w][i] + g[i] * part(v[i], w);
+        for (int i = 0; i < E; ++i) t3[w][i] = D == 0 ? g[i] * part(v[i], w) : t3[w][i] + g[i] * part(v[i], w);
+      }
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w)
 #pragma unroll
-      for (int i = 0; i < E; ++i) settle(H[w][i]), settle(t3[w][i]);
+      for (int i = 0; i < E; ++i) {
+        settle(H[w][i]);
+        if constexpr (!GRAD) settle(t3[w][i]);
+      }
   };
   // the backflow divergence and V_re so far, with early loads before J_z's transform
   auto bf_div = [&] {
@@ -828,11 +837,11 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
   axis(std::integral_constant<int, 1>{});
   if constexpr (PF) bf_div(), base_w(0), base_w(1);
   axis(std::integral_constant<int, 2>{});
-  // D_z J_z from the neighbouring points of both lines
+  // D_z J_z (GRAD: of rst J_z) from the neighbouring points of both lines
   using LY = rf::LayOf<T, N, pair_em<N>(), PairSync<N>>;
   C dz[E];
 #pragma unroll
-  for (int i = 0; i < E; ++i) X[LY::pad(t + TPL * i)] = v[i];
+  for (int i = 0; i < E; ++i) X[LY::pad(t + TPL * i)] = GRAD ? cmk<C>(rst(0, i) * v[i].x, rst(1, i) * v[i].y) : v[i];
   PairSync<N>::sync();
 #pragma unroll
   for (int i = 0; i < E; ++i) {
@@ -845,8 +854,10 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
     if constexpr (!PF) base_w(w);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
-      const T rst = st[w][i] * (-pw.inv_rho0s) + (T)1;
-      if (act) q.template put<T>(a.vre, w, i, base[w][i] + (part(dz[i], w) * rst * pw.ckc - t3[w][i] * (pw.ckc * pw.k23)));
+      T kc;
+      if constexpr (GRAD) kc = part(dz[i], w) * pw.ckc;
+      else kc = part(dz[i], w) * rst(w, i) * pw.ckc - t3[w][i] * (pw.ckc * pw.k23);
+      if (act) q.template put<T>(a.vre, w, i, base[w][i] + kc);
     }
   }
 #pragma unroll
@@ -857,12 +868,41 @@ __device__ __forceinline__ void zBC_body(ZBCArgs a, int64_t npairs, int P, PW<T>
 template <typename T, int N, bool BF>
 __global__ void __launch_bounds__((PairBS<T, N>), 0)
     k_zBC(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
-  zBC_body<T, N, BF, false>(a, npairs, P, pw, g_tw);
+  zBC_body<T, N, BF, false, false>(a, npairs, P, pw, g_tw);
 }
 template <typename T, int N>
 __global__ void __launch_bounds__((PairBS<T, N>), 0)
     k_zBC_bfhd(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
-  zBC_body<T, N, true, true>(a, npairs, P, pw, g_tw);
+  zBC_body<T, N, true, true, false>(a, npairs, P, pw, g_tw);
+}
+
+template <typename T, int N>
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
+    k_zBC_grad(ZBCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
+  zBC_body<T, N, false, false, true>(a, npairs, P, pw, g_tw);
+}
+
+// Last stage of the energy gradient: c2r of the linear terms, V_re and (KC) the
+// differences of M_x = rst J_x and M_y added.
+template <typename T, int N, bool KC>
+__global__ void __launch_bounds__((PairBS<T, N>), 0)
+    k_zG(const void *lin, const void *vre, const void *mx, const void *my, T *grad, int64_t npairs, int P, PW<T> pw,
+         const cplx<T> *__restrict__ g_tw) {
+  FUSED_PAIR_SETUP();
+  C v[E];
+  load_c2r<T, N>(v, X, s_tw, t, lin, p, P);
+  const auto qq = q.here();
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      T g = qq.template at_once<T>(vre, w, i) + part(v[i], w);
+      if constexpr (KC)
+        g += ((qq.template nb<T, 0, 1>(mx, w, i) - qq.template nb<T, 0, -1>(mx, w, i)) +
+              (qq.template nb<T, 1, 1>(my, w, i) - qq.template nb<T, 1, -1>(my, w, i))) *
+             pw.inv2h * pw.ckc;
+      if (act) q.template put<T>(grad, w, i, g);
+    }
 }
 
 // -------------------------------------------------------------------- zC --

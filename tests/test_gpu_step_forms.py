@@ -120,6 +120,26 @@ def test_energy_density_of_a_wave_function(shape, model, prec):
     f.free(), e.free(), w.free()
 
 
+@pytest.mark.parametrize("prec", [L.GRID_FP64, L.GRID_FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("model", [0, 1, 3], ids=["plain", "kc", "hd-kc"])
+@pytest.mark.parametrize("shape", [(4, 512, 8), (512, 4, 16), (8, 4, 512), (32, 16, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_energy_gradient_stages(shape, model, prec):
+    """dft_ot_energy_gradient through the z stages, at short and long axes, against
+    the oracle, with the bounds of the potential, whose stages these are."""
+    step = 0.9
+    o = po.OracleOT(model, shape, step, 2, 4)
+    psi = inputs.smooth_modulated(shape, step, o.p.rho0, 0.3)
+    rho = np.abs(psi) ** 2
+    w, r, g = L.Wave(shape, step, prec), L.RField(shape, step, prec), L.RField(shape, step, prec)
+    r.set(rho)
+    f = L.Functional(model, w, 2, 4)
+    L.lib().dft_ot_energy_gradient(f.h, g.h, r.h)
+    want = o.energy_gradient(rho)
+    assert np.abs(g.get() - want).max() <= (1e-10 if prec == L.GRID_FP64 else 2e-5) * np.abs(want).max()
+    for x in (f, r, g, w):
+        x.free()
+
+
 def test_reverse_pass_work_space_is_reusable():
     """The reverse passes' kept work space: repeated and interleaved calls of two
     functionals, a sweep with more checkpoints than the one before, and two threads
