@@ -1342,7 +1342,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     a.wx = d->slot[WX];
     a.wy = d->slot[WY];
     a.wz = d->slot[WZ];
-    const double bytes = nB * H + R + (BF ? 2 * R : 0) + nQ * H + R + (KC ? R : 0) + (BF ? 4 * R : 0);
+    const double bytes = nB * H + (BF ? 2 : 1) * R + nQ * H + R + (KC ? R : 0) + (BF ? 4 * R : 0);
     DFT_DISPATCH_N(d->nz, (launch_zAB<T, N_>(KC, BF, a, npairs, PP, pw, p.twz, s, bytes)));
     cplx<T> *b[4] = {CS<T>(d, Q4), CS<T>(d, QX), CS<T>(d, QY), CS<T>(d, QZ)};
     ypass<T>(p, nQ, b, -1, P, PP, s);
