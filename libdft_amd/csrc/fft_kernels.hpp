@@ -323,8 +323,9 @@ template <typename T> __global__ void k_scale_psi(cplx<T> *psi, const double *f,
 // (X once per block, in LDS) and applied in FP64 between the FP64 stages of
 // rfft_apply, so that its modulus is exact and one rounding separates the
 // coefficients before it from those after it.
-// Geometry: at least DFT_XKIN_COLS columns per block (N = 512 keeps the
-// column default).
+// Geometry: at least DFT_XKIN_COLS columns per block.  At N = 512 8 columns leave
+// LDS for several blocks per CU (FP32 512^3: 1013 us with 16, 943 with 8; the y
+// pass, whose rows are nearer each other, is faster with 16, 714 and 775).
 #ifndef DFT_XKIN_COLS
 #define DFT_XKIN_COLS 8
 #endif
@@ -339,7 +340,7 @@ template <typename T> __global__ void k_scale_psi(cplx<T> *psi, const double *f,
 #define DFT_XKIN_MINB64 0
 #endif
 template <typename T, int N>
-using KinCfg = typename std::conditional<(N >= 512), ColCfg<T, N>, ColCfg<T, N, 16, DFT_XKIN_COLS>>::type;
+using KinCfg = ColCfg<T, N, 16, DFT_XKIN_COLS>;
 
 template <typename T, int N>
 __global__ void __launch_bounds__((KinCfg<T, N>::BS), sizeof(T) == 4 ? DFT_XKIN_MINB : DFT_XKIN_MINB64)

@@ -386,15 +386,19 @@ template <int COLS> __device__ __forceinline__ MidCol mid_col(int ny, int P, int
 #ifndef DFT_XCONV_MINB64
 #define DFT_XCONV_MINB64 2
 #endif
-// (N = 512 keeps 16 points per thread and 16 columns.  FP64 single-term
-// outputs take DFT_XCONV1_COLS64 columns: 16 measured faster than 32, which
-// fill the LDS with one block per CU; the accumulating form takes at most 32.)
+// (N = 512 takes 16 points per thread and 8 columns: 45 KB of LDS in FP32 and 80
+// in FP64, so that 3 or 2 blocks share a CU and one's barriers overlap another's
+// loads; 16 columns fill it with one.  512^3 FP32 step: single-term outputs 2078
+// -> 1491 us per launch, sums 1012 -> 976; FP64 potential at 512x64x128 955 ->
+// 831 us, 512x32x32 265 -> 209.  FP64 single-term outputs take
+// DFT_XCONV1_COLS64 columns: 16 measured faster than 32, which fill the LDS with
+// one block per CU; the accumulating form takes at most 32.)
 #ifndef DFT_XCONV1_COLS64
 #define DFT_XCONV1_COLS64 16
 #endif
 template <typename T, int N, bool ONE>
 using XConvCfg = ColCfg<T, N, N >= 512 ? 16 : (ONE ? DFT_XCONV1_EM : DFT_XCONV_EM),
-                        N >= 512 ? 16
+                        N >= 512 ? 8
                                  : (ONE ? (sizeof(T) == 8 ? DFT_XCONV1_COLS64 : DFT_XCONV1_COLS)
                                         : (sizeof(T) == 8 && DFT_XCONV_COLS > 32 ? 32 : DFT_XCONV_COLS)),
                         !(ONE && N == 128)>;
