@@ -1878,7 +1878,8 @@ bool check_r(dft_ot_functional *otf, rgrid *g, const char *fn) {
 // sweep's checkpoints and segment.
 template <typename T> struct AdjWork {
   int64_t n = 0, nh = 0;
-  bool bf = false;
+  bool has_bf = false;  // the fields b are there
+  bool bf = false;      // the call at work goes through the backflow terms
   T *r[24] = {};
   T *b[20] = {};
   cplx<T> *c[4] = {};
@@ -1894,7 +1895,7 @@ template <typename T> struct AdjWork {
   bool alloc(int64_t n_, int64_t nh_, bool with_bf) {
     n = n_;
     nh = nh_;
-    bf = with_bf;
+    has_bf = with_bf;
     size_t off = 0;
     // two rounds: sizes, then pointers
     for (int round = 0; round < 2; ++round) {
@@ -1905,7 +1906,7 @@ template <typename T> struct AdjWork {
       };
       off = 0;
       for (auto &x : r) take(x, n);
-      if (bf)
+      if (has_bf)
         for (auto &x : b) take(x, n);
       for (auto &x : c) take(x, n);
       for (auto &x : spec) take(x, nh);
@@ -1937,7 +1938,9 @@ template <typename T> struct AdjWork {
 // 128^3 potential takes 1.3 ms, the allocations and frees of its ~55 fields took
 // 15 ms): up to kAdjKeep bytes, given back by dft_ot_free and when an allocation
 // of the library fails (trim_workspaces).  A call that finds it taken by another
-// thread works with one of its own.
+// thread works with one of its own.  The model may change between calls: whether a
+// call goes through the backflow terms is the call's own, and a work space without
+// their fields is replaced when they are needed.
 constexpr size_t kAdjKeep = (size_t)16 << 30;
 std::mutex g_adj_mu;                    // guards dft_ot_device::adj, adj_busy and g_adj_devs
 std::vector<dft_ot_device *> g_adj_devs;  // functionals that keep a work space
@@ -1957,8 +1960,12 @@ template <typename T> struct AdjLease {
     {
       std::lock_guard<std::mutex> lk(g_adj_mu);
       if (d->adj && !d->adj_busy) {
-        w = (AdjWork<T> *)d->adj;
-        d->adj_busy = true;
+        if (bf && !((AdjWork<T> *)d->adj)->has_bf) {
+          drop_adj<T>(d);
+        } else {
+          w = (AdjWork<T> *)d->adj;
+          d->adj_busy = true;
+        }
       }
     }
     ok = w != nullptr;
@@ -1966,6 +1973,7 @@ template <typename T> struct AdjLease {
       w = new AdjWork<T>();
       ok = w->alloc(d->n, (int64_t)d->nx * d->ny * d->PP, bf);
     }
+    w->bf = bf;
   }
   AdjLease(const AdjLease &) = delete;
   ~AdjLease() {

@@ -177,3 +177,43 @@ def test_reverse_pass_work_space_is_reusable():
     for s in (a, b):
         for x in (s[2], s[3], s[1], s[0]):
             x.free()
+
+
+@pytest.mark.parametrize("prec", [L.GRID_FP64, L.GRID_FP32], ids=["fp64", "fp32"])
+def test_reverse_passes_follow_the_model(prec):
+    """The functional's model flags are read by every call: reverse passes of one
+    functional with the backflow flag cleared and set between them, in both orders,
+    give bit for bit what a functional gives whose first reverse pass they are."""
+    shape, step = (16, 16, 32), 0.9
+    w = L.Wave(shape, step, prec)
+    vb, out = L.CField(shape, step, prec), L.CField(shape, step, prec)
+    vb.set(inputs.smooth_modulated(shape, step, 1.0, 0.5, 6))
+
+    def fresh():
+        f = L.Functional(9, w, 2, 4)
+        w.set(inputs.smooth_modulated(shape, step, f.p.rho0, 0.3, 5))
+        return f
+
+    def vjp(f, model):
+        f.p.model = model
+        assert L.lib().dft_ot_potential_vjp_psi(f.h, out.h, vb.h, w.h) == 0
+        return out.get()
+
+    def sweep(f, model):
+        f.p.model = model
+        return np.array([x for y in f.adjoint_well(-1e-4, 4.0, (0.0, 0.0, 0.0), 0.0, 100.0, 3, 2) for x in np.ravel(y)])
+
+    calls = [(c, m) for m in (9, 1) for c in (vjp, sweep)]
+    want = {}
+    for c, m in calls:
+        f = fresh()
+        want[c, m] = c(f, m)
+        f.free()
+    assert not np.array_equal(want[vjp, 9], want[vjp, 1]) and not np.array_equal(want[sweep, 9], want[sweep, 1])
+    for order in (calls, calls[::-1]):
+        f = fresh()
+        for c, m in order + order:
+            assert np.array_equal(c(f, m), want[c, m]), (c.__name__, m)
+        f.free()
+    for x in (vb, out, w):
+        x.free()
