@@ -273,11 +273,17 @@ __device__ __forceinline__ double2 twmul_d(double2 a, const cplx<T> *tw, int idx
 }
 
 // Keeps the compiler from moving work across every fourth point of an FP64
-// stage: without it the stage's LDS reads are all hoisted, and the FP32 kinetic
-// pass at 256 points spills 132 bytes per lane at 168 VGPRs (95 us at 256^3
-// against 66 with it, 156 VGPRs and no spills).
-__device__ __forceinline__ void point_fence(int r) {
-  if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+// stage of the long FP32 lines, whose FP64 registers otherwise cost waves: the
+// stage's LDS reads are all hoisted.  FP32 at 256 points: the kinetic pass spills
+// 132 bytes per lane (104 us at 256^3 against 76), a single-term x-middle output
+// takes 222 VGPRs instead of 116 (127 us against 103 per launch of 2-3 outputs);
+// at 512 points 112 instead of 73 (512x128x128: 72 against 65).  Not for shorter
+// lines nor for FP64, where as many waves fit either way and the fence only
+// delays the reads: FP64 64^3 single-term output 6.2 -> 5.9 us; FP32 128^3 kinetic pass
+// 11.8 -> 11.2, single-term outputs 24.9 -> 24.2.
+template <typename T, int N> __device__ __forceinline__ void point_fence(int r) {
+  if constexpr (sizeof(T) == 4 && N >= 256)
+    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
 }
 
 // Transform of one line, f(i, value) applied to every Fourier coefficient (point
@@ -302,20 +308,20 @@ __device__ __forceinline__ void rfft_apply(Regs<T, N, EM> &v, cplx<T> *X, const 
     for (int r = 0; r < R; ++r) {
       u[r] = make_double2((double)v[b + r * NB].x, (double)v[b + r * NB].y);
       if (NS > 1 && r > 0) u[r] = twmul_d<T, N, -1>(u[r], tw, tw_entry<N, EM>(NS, r, k));
-      point_fence(r);
+      point_fence<T, N>(r);
     }
     fft::dft<R, -1>(u);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       u[r] = f(b + r * NB, u[r]);
-      point_fence(r);
+      point_fence<T, N>(r);
     }
     fft::dft<R, +1>(u);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (NS > 1 && r > 0) u[r] = twmul_d<T, N, +1>(u[r], tw, tw_entry<N, EM>(NS, r, k));
       v[b + r * NB] = cmk<cplx<T>>((T)u[r].x, (T)u[r].y);
-      point_fence(r);
+      point_fence<T, N>(r);
     }
   }
   if constexpr (P::S == 3) rstage_back<T, N, EM, P::R1, P::R0, false, SYNC>(v, X, tw, t);
