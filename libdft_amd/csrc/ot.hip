@@ -1256,15 +1256,15 @@ void launch_zBC(bool BF, const fused::ZBCArgs &a, int64_t npairs, int P, const P
 }
 
 template <typename T, int N>
-void launch_zC(bool step, const fused::ZCArgs &a, int64_t npairs, int P, const PW<T> &pw, const cplx<T> *tw,
-               hipStream_t s, double bytes) {
+void launch_zC(bool step, const fused::ZCArgs &a, int64_t npairs, int P, const cplx<T> *tw, hipStream_t s,
+               double bytes) {
   constexpr int LN = rf::LineCfg<T, N, fused::pair_em<N>()>::LINES;
   const dim3 grid((unsigned)((npairs + LN - 1) / LN)), blk(fused::PairBS<T, N>);
   DFT_PROF_BEGIN(s);
-  if (step && a.jx) hipLaunchKernelGGL((fused::k_zC<T, N, true, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
-  else if (step) hipLaunchKernelGGL((fused::k_zC<T, N, true, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
-  else if (a.jx) hipLaunchKernelGGL((fused::k_zC<T, N, false, true>), grid, blk, 0, s, a, npairs, P, pw, tw);
-  else hipLaunchKernelGGL((fused::k_zC<T, N, false, false>), grid, blk, 0, s, a, npairs, P, pw, tw);
+  if (step && a.jx) hipLaunchKernelGGL((fused::k_zC<T, N, true, true>), grid, blk, 0, s, tw, npairs, P, a);
+  else if (step) hipLaunchKernelGGL((fused::k_zC<T, N, true, false>), grid, blk, 0, s, tw, npairs, P, a);
+  else if (a.jx) hipLaunchKernelGGL((fused::k_zC<T, N, false, true>), grid, blk, 0, s, tw, npairs, P, a);
+  else hipLaunchKernelGGL((fused::k_zC<T, N, false, false>), grid, blk, 0, s, tw, npairs, P, a);
   DFT_LAUNCH_CHECK();
   DFT_PROF_END(s, step ? "ot_zC_c2r_phase_z_fwd" : "ot_zC_c2r_accumulate", bytes);
 }
@@ -1403,13 +1403,18 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
     cplx<T> *b[1] = {CS<T>(d, TMP4)};
     ypass<T>(p, 1, b, +1, P, PP, s);
     fused::ZCArgs a{};
-    a.in.p[0] = d->slot[TMP4];
+    a.in = d->slot[TMP4];
+    a.nx = d->nx;
+    a.ny = d->ny;
     a.vre = d->slot[VRE];
     a.vim = BF ? d->slot[VIM] : nullptr;
     if (KC) {
       a.jx = d->slot[QX];
       a.jy = d->slot[QY];
       a.rhot = d->slot[RT];
+      a.inv2h = pw.inv2h;
+      a.inv_rho0s = pw.inv_rho0s;
+      a.ckc = pw.ckc;
     }
     double bytes = H + R + (BF ? R : 0) + (KC ? 3 * R : 0);
     if (!st) {
@@ -1427,7 +1432,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
       a.dti = st->dti;
       bytes += (st->vext ? R : 0) + (st->vavg ? 2 * R : 0) + (st->vsave ? 2 * R : 0) + 6 * R;
     }
-    DFT_DISPATCH_N(d->nz, (launch_zC<T, N_>(st != nullptr, a, npairs, PP, pw, p.twz, s, bytes)));
+    DFT_DISPATCH_N(d->nz, (launch_zC<T, N_>(st != nullptr, a, npairs, PP, p.twz, s, bytes)));
   }
 }
 

@@ -48,14 +48,14 @@ template <typename T, int N, int TPL> struct PairPos {
   uint32_t ym0, yp1;   // point t of lines (ix, j - 1) and (ix, j + 2)
   int t;
   PairPos() = default;
-  __device__ PairPos(uint32_t p, int t_, const PW<T> &pw) : t(t_) {
+  __device__ PairPos(uint32_t p, int t_, int nx, int ny) : t(t_) {
     const uint32_t l = 2 * p;
-    const int j = (int)(l & (uint32_t)(pw.ny - 1)), ix = (int)(l >> __builtin_ctz(pw.ny));
+    const int j = (int)(l & (uint32_t)(ny - 1)), ix = (int)(l >> __builtin_ctz(ny));
     a0 = l * N + t;
-    xp0 = ((uint32_t)((ix + 1) & (pw.nx - 1)) * pw.ny + j) * N + t;
-    xm0 = ((uint32_t)((ix - 1) & (pw.nx - 1)) * pw.ny + j) * N + t;
-    ym0 = ((uint32_t)ix * pw.ny + ((j - 1) & (pw.ny - 1))) * N + t;
-    yp1 = ((uint32_t)ix * pw.ny + ((j + 2) & (pw.ny - 1))) * N + t;
+    xp0 = ((uint32_t)((ix + 1) & (nx - 1)) * ny + j) * N + t;
+    xm0 = ((uint32_t)((ix - 1) & (nx - 1)) * ny + j) * N + t;
+    ym0 = ((uint32_t)ix * ny + ((j - 1) & (ny - 1))) * N + t;
+    yp1 = ((uint32_t)ix * ny + ((j + 2) & (ny - 1))) * N + t;
   }
   static constexpr int kTPL = TPL;
   static constexpr int d(int w, int i) { return w * N + TPL * i; }
@@ -136,7 +136,7 @@ template <typename T, int N> constexpr int PairBS = LineCfg<T, N, pair_em<N>()>:
   C *X = s_x + ln * LP;                                                      \
   rf::load_tw<T, N, G::EM, G::BS>(s_tw, g_tw);                                 \
   __syncthreads();                                                           \
-  const PairPos<T, N, TPL> q(p, t, pw)
+  const PairPos<T, N, TPL> q(p, t, pw.nx, pw.ny)
 
 template <typename T> __device__ __forceinline__ T dens_of(cplx<T> s) { return s.x * s.x + s.y * s.y; }
 
@@ -910,11 +910,13 @@ __global__ void __launch_bounds__((PairBS<T, N>), 0)
 }
 
 // -------------------------------------------------------------------- zC --
+// Kernel arguments are fetched when a wavefront starts, and on small grids that is
+// part of a launch's time: kept to what the kernel reads, most used first (plain
+// step at 64^3 FP64: zC 9.5 us with the whole PW, 384 bytes of arguments, 8.6 with
+// these 184).
 struct ZCArgs {
-  Ptrs8 in;              // summed linear terms (half spectrum)
+  const void *in;         // summed linear terms (half spectrum)
   const void *vre, *vim;  // vim null without backflow
-  const void *jx, *jy, *rhot;  // KC: J_x, J_y (the x and y parts of term 1) and F*rho
-  void *V;               // API mode: potential accumulated here
   // step mode
   const void *vext;      // real, may be null
   double mu;
@@ -924,11 +926,15 @@ struct ZCArgs {
   const void *psi_src;
   void *psi_dst;         // z forward transform of psi_src * phase
   double dtr, dti;
+  void *V;               // API mode: potential accumulated here
+  const void *jx, *jy, *rhot;  // KC: J_x, J_y (the x and y parts of term 1) and F*rho
+  int nx, ny;                  // and the values of PW that it takes
+  double inv2h, inv_rho0s, ckc;
 };
 
 template <typename T, int N, bool STEP, bool KC>
 __global__ void __launch_bounds__((PairBS<T, N>), 0)
-    k_zC(ZCArgs a, int64_t npairs, int P, PW<T> pw, const cplx<T> *__restrict__ g_tw) {
+    k_zC(const cplx<T> *__restrict__ g_tw, int64_t npairs, int P, ZCArgs a) {
   using C = cplx<T>;
   using G = LineCfg<T, N, pair_em<N>()>;
   constexpr int E = G::E, TPL = G::TPL, LP = G::LP;
@@ -943,9 +949,9 @@ __global__ void __launch_bounds__((PairBS<T, N>), 0)
   __syncthreads();
   constexpr bool PF = early_loads<T>();
   C v[E];
-  auto c2r_in = [&] { load_c2r<T, N>(v, X, s_tw, t, a.in.p[0], p, P); };
+  auto c2r_in = [&] { load_c2r<T, N>(v, X, s_tw, t, a.in, p, P); };
   const uint32_t cb = p * 2u * N + (uint32_t)t;
-  const PairPos<T, N, TPL> q(p, t, pw);
+  const PairPos<T, N, TPL> q(p, t, a.nx, a.ny);
   // the x and y parts of KC term 1, c rst (D_x J_x + D_y J_y), in two parts: the
   // loads of line w, and its value at point i
   T jd[KC ? 4 : 1][KC ? E : 1], rt[KC ? E : 1];
@@ -964,7 +970,7 @@ __global__ void __launch_bounds__((PairBS<T, N>), 0)
   };
   auto t1 = [&](int i) {
     if constexpr (KC)
-      return ((jd[0][i] - jd[1][i]) + (jd[2][i] - jd[3][i])) * pw.inv2h * (rt[i] * (-pw.inv_rho0s) + (T)1) * pw.ckc;
+      return ((jd[0][i] - jd[1][i]) + (jd[2][i] - jd[3][i])) * (T)a.inv2h * (rt[i] * (T)-a.inv_rho0s + (T)1) * (T)a.ckc;
     else return (T)0;
   };
   if constexpr (!STEP) {
