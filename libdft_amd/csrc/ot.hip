@@ -944,22 +944,36 @@ template <typename T> PW<T> make_pw(dft_ot_functional *otf, double wf_mass, doub
     DFT_PROF_END(lib_stream(), name, (double)(nf) * (double)d->n * sizeof(T));               \
   } while (0)
 
-// x-middle pass of program pg, one output per block (k_xconv): leading outputs
-// with a single term take the lean form, the rest the accumulating one.
+// x-middle pass of program pg, one output per block (k_xconv): its single-term
+// outputs as one launch of the lean form, the others a launch each of the
+// accumulating one.
 template <typename T, int N>
 void launch_xconv(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T> *tw, hipStream_t s, double bytes) {
-  int n1 = 0;
-  while (n1 < pg.nout && pg.o[n1].nterms == 1) ++n1;
   using Cfg1 = fused::XConvCfg<T, N, true>;
   using Cfg = fused::XConvCfg<T, N, false>;
+  fused::XOnes ones{};
+  int n1 = 0;
+  for (int m = 0; m < pg.nout; ++m)
+    if (pg.o[m].nterms == 1) {
+      const fused::MidTerm &t = pg.o[m].t[0];
+      ones.o[n1++] = {pg.in[t.in], pg.kern[t.kern], pg.o[m].out, t.scale};
+    }
   DFT_PROF_BEGIN(s);
   if (n1 > 0)
     hipLaunchKernelGGL((fused::k_xconv<T, N, true>), dim3((unsigned)(fused::mid_blocks<Cfg1::COLS>(ny, P) * n1)),
-                       dim3(Cfg1::BS), 0, s, pg, 0, n1, ny, P, PP, tw);
-  if (n1 < pg.nout)
-    hipLaunchKernelGGL((fused::k_xconv<T, N, false>),
-                       dim3((unsigned)(fused::mid_blocks<Cfg::COLS>(ny, P) * (pg.nout - n1))), dim3(Cfg::BS), 0, s, pg,
-                       n1, pg.nout - n1, ny, P, PP, tw);
+                       dim3(Cfg1::BS), 0, s, tw, n1, ny, P, PP, ones);
+  for (int m = 0; m < pg.nout; ++m)
+    if (pg.o[m].nterms > 1) {
+      fused::XSum sum{};
+      sum.out = pg.o[m].out;
+      sum.nterms = pg.o[m].nterms;
+      for (int q = 0; q < sum.nterms; ++q) {
+        const fused::MidTerm &t = pg.o[m].t[q];
+        sum.t[q] = {pg.in[t.in], pg.kern[t.kern], t.scale};
+      }
+      hipLaunchKernelGGL((fused::k_xconv<T, N, false>), dim3((unsigned)fused::mid_blocks<Cfg::COLS>(ny, P)),
+                         dim3(Cfg::BS), 0, s, tw, 1, ny, P, PP, sum);
+    }
   DFT_LAUNCH_CHECK();
   DFT_PROF_END(s, n1 == pg.nout ? "ot_xconv_single" : (n1 == 0 ? "ot_xconv_multi" : "ot_xconv_mixed"), bytes);
 }
