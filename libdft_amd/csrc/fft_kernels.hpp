@@ -342,8 +342,14 @@ template <typename T> __global__ void k_scale_psi(cplx<T> *psi, const double *f,
 template <typename T, int N>
 using KinCfg = ColCfg<T, N, 16, DFT_XKIN_COLS>;
 
+// (A 16-point line is one thread's, transformed in FP64 both ways: at 3 waves it
+// spills 220 bytes per lane, 16^3 FP32 6.8 us; at 2, 4.5.)
+template <typename T, int N> constexpr int xkin_minb() {
+  return sizeof(T) == 8 ? DFT_XKIN_MINB64 : (N == 16 ? 2 : DFT_XKIN_MINB);
+}
+
 template <typename T, int N>
-__global__ void __launch_bounds__((KinCfg<T, N>::BS), sizeof(T) == 4 ? DFT_XKIN_MINB : DFT_XKIN_MINB64)
+__global__ void __launch_bounds__((KinCfg<T, N>::BS), (xkin_minb<T, N>()))
     k_xkin(cplx<T> *psi, int ny, int nz, int ntile, const cplx<T> *__restrict__ g_tw, double cx, double cy, double cz,
            double dtr, double dti, double ox, double oy, double oz) {
   using C = cplx<T>;
