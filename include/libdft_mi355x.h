@@ -472,6 +472,11 @@ int dft_ot_adjoint_well(dft_ot_functional *otf, wf *gwf, REAL amp, REAL width, R
    or -1 (message on stderr) for invalid arguments or lack of device memory. */
 int dft_ot_adjoint_cavity(dft_ot_functional *otf, wf *gwf, REAL rho0, REAL radius, REAL width, REAL mu,
                           REAL_COMPLEX time, INT nsteps, INT every, REAL *bubble_radius, REAL *grad);
+/* The reverse passes above keep their work space with the functional for the next
+   call: at most 16 GiB over all functionals, the least recently used given back
+   first, a functional's own by dft_ot_free.  dft_ot_trim gives back all of it that
+   no call is using. */
+void dft_ot_trim(void);
 /* Progress lines of the adjoint sweeps on stderr (level > 0), one per checkpoint. */
 void dft_set_verbose(int level);
 

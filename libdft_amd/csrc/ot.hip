@@ -1892,9 +1892,9 @@ bool check_r(dft_ot_functional *otf, rgrid *g, const char *fn) {
 
 // -------------------------------------------------------- adjoint sweep --
 // Work space of the reverse pass: real fields, complex fields and half spectra,
-// for backflow models the fields of the backflow transpose, and the sweep's
-// adjoint state, running state and well; one allocation.  `states` holds a
-// sweep's checkpoints and segment.
+// and for backflow models the fields of the backflow transpose, one allocation
+// (slab); for a sweep its adjoint state, running state, well, checkpoints and
+// segment, another (sweep).
 template <typename T> struct AdjWork {
   int64_t n = 0, nh = 0;
   bool has_bf = false;  // the fields b are there
@@ -1903,14 +1903,14 @@ template <typename T> struct AdjWork {
   T *b[20] = {};
   cplx<T> *c[4] = {};
   cplx<T> *spec[10] = {};
-  cplx<T> *psib = nullptr, *cur = nullptr;
-  T *well = nullptr;
   double *pa = nullptr, *pw = nullptr;
   void *slab = nullptr;
-  cplx<T> *states = nullptr;
+  cplx<T> *psib = nullptr, *cur = nullptr, *states = nullptr;
+  T *well = nullptr;
+  void *sweep = nullptr;
   int64_t nstates = 0;
-  size_t slab_bytes = 0;
-  size_t bytes() const { return slab_bytes + sizeof(cplx<T>) * (size_t)n * nstates; }
+  size_t slab_bytes = 0, sweep_bytes = 0;
+  size_t bytes() const { return slab_bytes + sweep_bytes; }
   bool alloc(int64_t n_, int64_t nh_, bool with_bf) {
     n = n_;
     nh = nh_;
@@ -1929,58 +1929,95 @@ template <typename T> struct AdjWork {
         for (auto &x : b) take(x, n);
       for (auto &x : c) take(x, n);
       for (auto &x : spec) take(x, nh);
-      take(psib, n);
-      take(cur, n);
-      take(well, n);
       take(pa, red_blocks(n));
       take(pw, red_blocks(n));
       if (!round && !(slab = dmalloc(slab_bytes = off))) return false;
     }
     return true;
   }
-  bool alloc_states(int64_t k) {
+  // fields of a sweep with k checkpoints and segment states
+  bool alloc_sweep(int64_t k) {
     if (k <= nstates) return true;
-    dfree(states);
+    dfree(sweep);
     nstates = 0;
-    if (!(states = (cplx<T> *)dmalloc(sizeof(cplx<T>) * n * k))) return false;
+    sweep_bytes = (sizeof(cplx<T>) * (k + 2) + sizeof(T)) * (size_t)n;
+    if (!(sweep = dmalloc(sweep_bytes))) {
+      sweep_bytes = 0;
+      return false;
+    }
+    psib = (cplx<T> *)sweep;
+    cur = psib + n;
+    states = cur + n;
+    well = (T *)(states + k * n);
     nstates = k;
     return true;
   }
   void release() {
     dfree(slab);
-    dfree(states);
+    dfree(sweep);
     *this = AdjWork<T>();
   }
 };
 
 // The work space stays with its functional between calls (a reverse pass of a
-// 128^3 potential takes 1.3 ms, the allocations and frees of its ~55 fields took
-// 15 ms): up to kAdjKeep bytes, given back by dft_ot_free and when an allocation
-// of the library fails (trim_workspaces).  A call that finds it taken by another
-// thread works with one of its own.  The model may change between calls: whether a
-// call goes through the backflow terms is the call's own, and a work space without
-// their fields is replaced when they are needed.
+// 128^3 potential takes 1.0 ms, the allocations and frees of its ~55 fields took
+// 15 ms).  All functionals together keep at most kAdjKeep bytes, the spaces used
+// least recently going first; dft_ot_free gives back a functional's own,
+// dft_ot_trim all that no call is using, as does an allocation of the library that
+// fails.  The model may change between calls: whether a call goes through the
+// backflow terms is the call's own, and a work space without their fields is
+// replaced when they are needed.  (Two calls at once on one functional share its
+// other fields and are not supported; the second one still gets memory of its own.)
 constexpr size_t kAdjKeep = (size_t)16 << 30;
-std::mutex g_adj_mu;                    // guards dft_ot_device::adj, adj_busy and g_adj_devs
-std::vector<dft_ot_device *> g_adj_devs;  // functionals that keep a work space
+struct AdjKept {
+  dft_ot_device *d;
+  size_t bytes;
+};
+std::mutex g_adj_mu;               // guards dft_ot_device::adj, adj_busy and g_adj_kept
+std::vector<AdjKept> g_adj_kept;  // functionals that keep a work space, the last used last
 
-template <typename T> void drop_adj(dft_ot_device *d) {  // g_adj_mu held
-  ((AdjWork<T> *)d->adj)->release();
-  delete (AdjWork<T> *)d->adj;
-  d->adj = nullptr;
-  g_adj_devs.erase(std::find(g_adj_devs.begin(), g_adj_devs.end(), d));
+auto find_adj(dft_ot_device *d) {  // g_adj_mu held, as in the next two
+  return std::find_if(g_adj_kept.begin(), g_adj_kept.end(), [d](const AdjKept &k) { return k.d == d; });
 }
 
+void drop_adj(dft_ot_device *d) {
+  DFT_BY_PREC(d->prec, {
+    ((AdjWork<T> *)d->adj)->release();
+    delete (AdjWork<T> *)d->adj;
+  });
+  d->adj = nullptr;
+  g_adj_kept.erase(find_adj(d));
+}
+
+// Drops idle work spaces, the least recently used first, until `bytes` are kept.
+bool shrink_adj(size_t bytes) {
+  size_t total = 0;
+  for (const AdjKept &k : g_adj_kept) total += k.bytes;
+  bool any = false;
+  for (size_t i = 0; i < g_adj_kept.size() && total > bytes;) {
+    const AdjKept k = g_adj_kept[i];
+    if (k.d->adj_busy) {
+      ++i;
+      continue;
+    }
+    total -= k.bytes;
+    drop_adj(k.d);
+    any = true;
+  }
+  return any;
+}
+
+// A call's work space, with the fields of a sweep if it has `states` of them.
 template <typename T> struct AdjLease {
   dft_ot_device *d;
   AdjWork<T> *w;
   bool ok;
-  AdjLease(dft_ot_device *d_, bool bf) : d(d_), w(nullptr) {
+  AdjLease(dft_ot_device *d_, bool bf, int64_t states = 0) : d(d_), w(nullptr) {
     {
       std::lock_guard<std::mutex> lk(g_adj_mu);
       if (d->adj && !d->adj_busy) {
         if (bf && !((AdjWork<T> *)d->adj)->has_bf) {
-          drop_adj<T>(d);
+          drop_adj(d);
         } else {
           w = (AdjWork<T> *)d->adj;
           d->adj_busy = true;
@@ -1993,30 +2030,31 @@ template <typename T> struct AdjLease {
       ok = w->alloc(d->n, (int64_t)d->nx * d->ny * d->PP, bf);
     }
     w->bf = bf;
+    if (ok && states) ok = w->alloc_sweep(states);
   }
   AdjLease(const AdjLease &) = delete;
   ~AdjLease() {
     DFT_HIP_CHECK(hipStreamSynchronize(lib_stream()));
     std::lock_guard<std::mutex> lk(g_adj_mu);
-    const bool keep = ok && w->bytes() <= kAdjKeep;
     if (d->adj == w) {
       d->adj_busy = false;
-      if (!keep) drop_adj<T>(d);
-    } else if (keep && !d->adj) {
+      g_adj_kept.erase(find_adj(d));
+    } else if (!d->adj) {
       d->adj = w;
-      g_adj_devs.push_back(d);
     } else {
       w->release();
       delete w;
+      return;
     }
+    g_adj_kept.push_back({d, w->bytes()});
+    if (!ok || w->bytes() > kAdjKeep) drop_adj(d);
+    shrink_adj(kAdjKeep);
   }
 };
 
 void free_adj(dft_ot_device *d) {
   std::lock_guard<std::mutex> lk(g_adj_mu);
-  if (!d->adj) return;
-  if (d->prec == GRID_FP32) drop_adj<float>(d);
-  else drop_adj<double>(d);
+  if (d->adj) drop_adj(d);
 }
 
 // Real fields of the work space.
@@ -2255,6 +2293,8 @@ void adj_step(dft_ot_functional *otf, const cplx<T> *psi, cplx<T> *psib, double 
 // Progress lines of the long-running sweeps on stderr (dft_set_verbose).
 int g_verbose = 0;
 
+int64_t checkpoints(int64_t K, int64_t every) { return (K + every - 1) / every; }
+
 // Checkpointed adjoint of K single steps of dft_ot_propagate from the state in
 // gwf (left unchanged), with the well wl as V_ext.  The forward pass keeps every
 // `every`-th state; the reverse pass recomputes each segment from its
@@ -2262,14 +2302,13 @@ int g_verbose = 0;
 // dJ = Re sum conj(psib) dpsi) and may start th; on return psib holds dJ/dpsi_0
 // and th[0..1] has accumulated dJ/d(amp, width) through V_ext.
 template <typename T, class Seed>
-int adjoint_sweep(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu, double dtr, double dti, int64_t K,
+void adjoint_sweep(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu, double dtr, double dti, int64_t K,
                   int64_t every, AdjWork<T> &w, cplx<T> *psib, double th[2], Seed seed) {
   dft_ot_device *d = otf->device;
   hipStream_t s = lib_stream();
   const int64_t n = d->n;
   const size_t bytes = sizeof(cplx<T>) * n;
-  const int64_t ncp = (K + every - 1) / every;
-  if (!w.alloc_states(ncp + every)) return -1;
+  const int64_t ncp = checkpoints(K, every);
   auto cp = [&](int64_t i) { return w.states + i * n; };
   auto seg = [&](int64_t i) { return w.states + (ncp + i) * n; };
   // the running state and the well, on the work space's fields
@@ -2312,7 +2351,6 @@ int adjoint_sweep(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu, do
       adj_step<T>(otf, seg(it - n0), psib, mass, wl, mu, dtr, dti, k0, w, th);
     if (g_verbose) fprintf(stderr, "libdft: adjoint reverse segment %lld / %lld done\n", (long long)(ncp - j), (long long)ncp);
   }
-  return 0;
 }
 
 // J = E_kin + E_OT + E_ext of psi_K and dJ/d(amp, width) of the well.
@@ -2323,10 +2361,9 @@ int adjoint_well_impl(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu
   hipStream_t s = lib_stream();
   const int64_t n = d->n;
   const bool BF = (otf->model & DFT_OT_BACKFLOW) != 0;
-  AdjLease<T> lease(d, BF);
+  AdjLease<T> lease(d, BF, checkpoints(K, every) + every);
   AdjWork<T> &w = *lease.w;
   cplx<T> *psib = w.psib;
-  const bool ok = lease.ok;
   double th[2] = {0.0, 0.0};
   auto seed = [&](wf *cur, cplx<T> *pb, double t2[2]) {
     // the gradient of the total energy with respect to psi_K
@@ -2354,11 +2391,11 @@ int adjoint_well_impl(dft_ot_functional *otf, wf *gwf, const Well &wl, double mu
     if (BF) seed_bf<T>(otf, psiK, gwf->mass, pb, w);
     *E = grid_wf_energy(cur, nullptr) + dft_ot_energy(otf, cur) + wl.amp * t2[0];
   };
-  const int rc = ok ? adjoint_sweep<T>(otf, gwf, wl, mu, dtr, dti, K, every, w, psib, th, seed) : -1;
-  if (rc) fprintf(stderr, "libdft: dft_ot_adjoint_well: out of device memory\n");
+  if (lease.ok) adjoint_sweep<T>(otf, gwf, wl, mu, dtr, dti, K, every, w, psib, th, seed);
+  else fprintf(stderr, "libdft: dft_ot_adjoint_well: out of device memory\n");
   grad[0] = th[0];
   grad[1] = th[1];
-  return rc;
+  return lease.ok ? 0 : -1;
 }
 
 // psi_0 = sqrt(rho0 (1 + tanh((r - R0)/w)) / 2): bulk with a spherical cavity.
@@ -2438,10 +2475,9 @@ int adjoint_cavity_impl(dft_ot_functional *otf, wf *gwf, double rho0, double R0,
   hipLaunchKernelGGL(k_cavity<T>, dim3(grid_for(n)), dim3(kBlock), 0, s, (cplx<T> *)gwf->grid->dev, geo, rho0, R0, wd,
                      n);
   DFT_LAUNCH_CHECK();
-  AdjLease<T> lease(d, (otf->model & DFT_OT_BACKFLOW) != 0);
+  AdjLease<T> lease(d, (otf->model & DFT_OT_BACKFLOW) != 0, checkpoints(K, every) + every);
   AdjWork<T> &w = *lease.w;
   cplx<T> *psib = w.psib;
-  const bool ok = lease.ok;
   double th[2] = {0.0, 0.0}, explicit_term = 0.0;
   auto seed = [&](wf *cur, cplx<T> *pb, double *) {
     const cplx<T> *psiK = (const cplx<T> *)cur->grid->dev;
@@ -2457,8 +2493,8 @@ int adjoint_cavity_impl(dft_ot_functional *otf, wf *gwf, double rho0, double R0,
                        (*J / (3.0 * V)) * (-2.0 * h3 / rho0), n);
     DFT_LAUNCH_CHECK();
   };
-  int rc = ok ? adjoint_sweep<T>(otf, gwf, geo, mu, dtr, dti, K, every, w, psib, th, seed) : -1;
-  if (rc) {
+  if (lease.ok) adjoint_sweep<T>(otf, gwf, geo, mu, dtr, dti, K, every, w, psib, th, seed);
+  if (!lease.ok) {
     fprintf(stderr, "libdft: dft_ot_adjoint_cavity: out of device memory\n");
   } else {
     hipLaunchKernelGGL(k_cavity_grad<T>, dim3((unsigned)red_blocks(n)), dim3(kBlock), 0, s, (const cplx<T> *)psib, geo,
@@ -2466,7 +2502,7 @@ int adjoint_cavity_impl(dft_ot_functional *otf, wf *gwf, double rho0, double R0,
     DFT_LAUNCH_CHECK();
     *grad = sum_partials(w.pa, red_blocks(n), s) + explicit_term;
   }
-  return rc;
+  return lease.ok ? 0 : -1;
 }
 
 // Standalone reverse pass of V_OT at the density of gwf (for tests): rho_bar = (dV/drho)^T v_bar.
@@ -2521,15 +2557,7 @@ template <typename T> bool potential_vjp_psi_impl(dft_ot_functional *otf, cplx<T
 
 bool dft::trim_workspaces() {
   std::lock_guard<std::mutex> lk(g_adj_mu);
-  bool any = false;
-  for (size_t i = g_adj_devs.size(); i-- > 0;) {
-    dft_ot_device *d = g_adj_devs[i];
-    if (d->adj_busy) continue;
-    if (d->prec == GRID_FP32) drop_adj<float>(d);
-    else drop_adj<double>(d);
-    any = true;
-  }
-  return any;
+  return shrink_adj(0);
 }
 
 // ================================================================== C ABI ==
@@ -2961,6 +2989,8 @@ int dft_ot_adjoint_well(dft_ot_functional *otf, wf *gwf, REAL amp, REAL width, R
   grad[1] = g[1];
   return rc;
 }
+
+void dft_ot_trim(void) { dft::trim_workspaces(); }
 
 void dft_set_verbose(int level) { g_verbose = level; }
 

@@ -217,3 +217,47 @@ def test_reverse_passes_follow_the_model(prec):
         f.free()
     for x in (vb, out, w):
         x.free()
+
+
+def test_kept_work_spaces_are_bounded():
+    """The work spaces that reverse passes leave with their functionals: 16 GiB in all
+    (19 of 1 GiB each here), the last used among them, results as before; dft_ot_trim
+    gives all of it back, and the next call does without."""
+    import ctypes
+
+    shape, step, lib = (128, 128, 128), 0.9, L.lib()
+    GiB, slack = 1 << 30, 1 << 28
+
+    def free():
+        a, b = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert lib.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0  # of the HIP runtime the library is linked with
+        return a.value
+
+    w = L.Wave(shape, step, L.GRID_FP64)
+    vb, out = L.CField(shape, step, L.GRID_FP64), L.CField(shape, step, L.GRID_FP64)
+    fs = [L.Functional(9, w, 1, 1) for _ in range(19)]
+    w.set(inputs.smooth_modulated(shape, step, fs[0].p.rho0, 0.3, 5))
+    vb.set(inputs.smooth_modulated(shape, step, 1.0, 0.5, 6))
+
+    def vjp(f):
+        assert lib.dft_ot_potential_vjp_psi(f.h, out.h, vb.h, w.h) == 0
+        return out.get()
+
+    want = vjp(fs[0])
+    lib.dft_ot_trim()
+    base = free()
+    vjp(fs[0])
+    one = base - free()
+    assert one > GiB - slack
+    for f in fs:
+        vjp(f)
+        assert base - free() <= 16 * GiB + slack
+    kept = base - free()
+    assert kept > 16 * GiB - one - slack
+    assert np.array_equal(vjp(fs[-1]), want) and abs(base - free() - kept) <= slack
+    assert np.array_equal(vjp(fs[0]), want) and base - free() <= 16 * GiB + slack
+    lib.dft_ot_trim()
+    assert abs(base - free()) <= slack
+    assert np.array_equal(vjp(fs[1]), want)
+    for x in (*fs, vb, out, w):
+        x.free()
