@@ -1016,6 +1016,10 @@ void set_kernels(fused::MidProg &pg, const fft::KernTab &kt) {
 template <typename T>
 void convolve(dft_ot_device *d, int nin, const cplx<T> *const *in, int nout, const fft::Combine *c,
               cplx<T> *const *tmp, T *const *out) {
+  if (nin > fused::kMidMaxIn || nout > fused::kMidMaxOut) {
+    fprintf(stderr, "libdft: convolve: too many inputs or outputs\n");
+    abort();
+  }
   Plan3D<T> &p = plan_of<T>(d);
   hipStream_t s = lib_stream();
   fused::MidProg pg = new_prog();
