@@ -978,8 +978,6 @@ void launch_xconv(const fused::MidProg &pg, int ny, int P, int PP, const cplx<T>
   DFT_PROF_END(s, n1 == pg.nout ? "ot_xconv_single" : (n1 == 0 ? "ot_xconv_multi" : "ot_xconv_mixed"), bytes);
 }
 
-fused::MidProg new_prog() { return fused::MidProg{}; }
-
 fused::MidTerm mterm(int in, int kern, double scale) {
   fused::MidTerm t{};
   t.in = in;
@@ -1001,7 +999,6 @@ void set_kernels(fused::MidProg &pg, const fft::KernTab &kt) {
   for (int m = 0; m < pg.nout; ++m)
     for (int q = 0; q < pg.o[m].nterms; ++q) {
       int &k = pg.o[m].t[q].kern;
-      if (k < 0) continue;
       if (slot[k] < 0) {
         slot[k] = pg.nkern;
         pg.kern[pg.nkern++] = kt.k[k];
@@ -1022,7 +1019,7 @@ void convolve(dft_ot_device *d, int nin, const cplx<T> *const *in, int nout, con
   }
   Plan3D<T> &p = plan_of<T>(d);
   hipStream_t s = lib_stream();
-  fused::MidProg pg = new_prog();
+  fused::MidProg pg{};
   pg.nin = nin;
   pg.nout = nout;
   for (int i = 0; i < nin; ++i) pg.in[i] = in[i];
@@ -1200,7 +1197,7 @@ void potential_impl(dft_ot_functional *otf, cgrid *V, const cplx<T> *psi, double
 
 // J_d = F*G_d for the three axes
 template <typename C> fused::MidProg j_program(C *const *g, C *const *j, double scale, const fft::KernTab &kt) {
-  fused::MidProg pg = new_prog();
+  fused::MidProg pg{};
   pg.nin = pg.nout = 3;
   for (int dd = 0; dd < 3; ++dd) {
     pg.in[dd] = g[dd];
@@ -1321,7 +1318,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
   // x middle: Pi*rho, [F*rho], [U*rho (U*rho~ with the switch), U*q_x, U*q_y, U*q_z, U*q4]
   int nB = 0;
   {
-    fused::MidProg pg = new_prog();
+    fused::MidProg pg{};
     pg.nin = nA;
     for (int i = 0; i < nA; ++i) pg.in[i] = d->slot[SP0 + i];
     auto add = [&](int in, int kern) {
@@ -1400,7 +1397,7 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
   }
   // ---- stage C: linear terms summed in k space, z^-1, accumulate or start the step
   {
-    fused::MidProg pg = new_prog();
+    fused::MidProg pg{};
     pg.nin = 2;
     pg.in[0] = d->slot[SP0];
     pg.in[1] = d->slot[Q4];
@@ -1505,7 +1502,7 @@ void fused_energy(dft_ot_functional *otf, T *eps, const cplx<T> *psi, double wf_
   for (int i = 0; i < nA; ++i) oA.p[i] = sp[i] = CS<T>(d, SP0 + i);
   DFT_DISPATCH_N(d->nz, (launch_zA<T, N_>(BF, psi, rho, oA, npairs, PP, pw, p.twz, s, 3 * R + nA * H)));
   ypass<T>(p, nA, sp, -1, P, PP, s);
-  fused::MidProg pg = new_prog();
+  fused::MidProg pg{};
   pg.nin = nA;
   for (int i = 0; i < nA; ++i) pg.in[i] = sp[i];
   auto add = [&](int in, int kern) {
@@ -1693,7 +1690,7 @@ template <typename T> void gradient_impl(dft_ot_functional *otf, T *grad, const 
   };
   cplx<T> *tmp[3] = {CS<T>(d, TMP0), CS<T>(d, TMP1), CS<T>(d, TMP2)};
   {
-    fused::MidProg pg = new_prog();
+    fused::MidProg pg{};
     pg.nin = 1;
     pg.in[0] = d->slot[SP0];
     pg.nout = KC ? 2 : 1;
@@ -1731,7 +1728,7 @@ template <typename T> void gradient_impl(dft_ot_functional *otf, T *grad, const 
     ypass<T>(p, 1, hb, -1, P, PP, s);
   }
   {
-    fused::MidProg pg = new_prog();
+    fused::MidProg pg{};
     pg.nin = KC ? 3 : 2;
     pg.in[0] = d->slot[SP0];
     pg.in[1] = d->slot[Q4];

@@ -298,11 +298,11 @@ __global__ void __launch_bounds__((PairBS<T, N>), 0)
 
 // ------------------------------------------------------------------ xconv --
 struct MidTerm {
-  int in, kern;  // kern: slot of MidProg::kern (or -1)
+  int in, kern;  // of MidProg::in, MidProg::kern
   double scale;
 };
 struct MidOut {
-  int nterms, pad;
+  int nterms;
   MidTerm t[4];
   void *out;
 };

@@ -228,25 +228,23 @@ __device__ __forceinline__ void rfft(Regs<T, N, EM> &v, cplx<T> *X, const cplx<T
   }
 }
 
-// Inverse of one forward stage, mirrored: exchange back (not for the last
-// stage, whose outputs are in place), radix-R inverse DFT, conjugate twiddles.
-template <typename T, int N, int EM, int R, int NS, bool LAST, class SYNC>
+// Inverse of one forward stage before the last, mirrored: exchange back, radix-R
+// inverse DFT, conjugate twiddles.
+template <typename T, int N, int EM, int R, int NS, class SYNC>
 __device__ __forceinline__ void rstage_back(Regs<T, N, EM> &v, cplx<T> *X, const cplx<T> *tw, int t) {
   using C = cplx<T>;
   constexpr int E = RP<N, EM>::E, TPL = RP<N, EM>::TPL, NB = E / R;
-  if constexpr (!LAST) {
 #pragma unroll
-    for (int i = 0; i < E; ++i) X[LayOf<T, N, EM, SYNC>::pad(t + TPL * i)] = v[i];
-    SYNC::sync();
-  }
+  for (int i = 0; i < E; ++i) X[LayOf<T, N, EM, SYNC>::pad(t + TPL * i)] = v[i];
+  SYNC::sync();
   C w[NB][R];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int j = t + TPL * b, d = (j / NS) * NS * R + (j & (NS - 1));
 #pragma unroll
-    for (int r = 0; r < R; ++r) w[b][r] = LAST ? v[b + r * NB] : X[LayOf<T, N, EM, SYNC>::pad(d + r * NS)];
+    for (int r = 0; r < R; ++r) w[b][r] = X[LayOf<T, N, EM, SYNC>::pad(d + r * NS)];
   }
-  if constexpr (!LAST) SYNC::sync();
+  SYNC::sync();
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int k = (t + TPL * b) & (NS - 1);
@@ -324,8 +322,8 @@ __device__ __forceinline__ void rfft_apply(Regs<T, N, EM> &v, cplx<T> *X, const 
       point_fence<T, N>(r);
     }
   }
-  if constexpr (P::S == 3) rstage_back<T, N, EM, P::R1, P::R0, false, SYNC>(v, X, tw, t);
-  if constexpr (P::S >= 2) rstage_back<T, N, EM, P::R0, 1, false, SYNC>(v, X, tw, t);
+  if constexpr (P::S == 3) rstage_back<T, N, EM, P::R1, P::R0, SYNC>(v, X, tw, t);
+  if constexpr (P::S >= 2) rstage_back<T, N, EM, P::R0, 1, SYNC>(v, X, tw, t);
 }
 
 // LDS entries of a twiddle table: the N - R0 stage-ordered twiddles, and for
@@ -391,15 +389,6 @@ template <typename X> __device__ __forceinline__ void gst(void *base, uint32_t o
   } else {
     *p = v;
   }
-}
-
-// Logical block index with consecutive indices on one XCD: blocks are
-// dispatched round-robin over the 8 XCDs, each with its own L2, so with this
-// order the column tiles of one transform line (consecutive indices) share an
-// L2.  Identity when the grid is not a multiple of 8.
-__device__ __forceinline__ int xcd_block() {
-  const int b = blockIdx.x, n = gridDim.x;
-  return (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b;
 }
 
 // Element-indexed forms: element `e` (per thread) plus constant element delta `d`.
