@@ -261,3 +261,20 @@ def test_kept_work_spaces_are_bounded():
     assert np.array_equal(vjp(fs[1]), want)
     for x in (*fs, vb, out, w):
         x.free()
+
+
+@pytest.mark.parametrize("model", [0, 1, 9], ids=["plain", "kc", "full"])
+@pytest.mark.parametrize("shape", [(8, 4, 16), (16, 8, 4), (64, 16, 32), (32, 64, 128)], ids=lambda s: "x".join(map(str, s)))
+def test_potential_nyquist_tiles_fp32(shape, model):
+    """test_potential_nyquist_tiles in FP32, whose tiles have column counts of their
+    own, with the bound of the FP32 potential tests."""
+    step = 1.1
+    o = po.OracleOT(model, shape, step, 2, 4)
+    psi = inputs.smooth_modulated(shape, step, o.p.rho0, 0.3)
+    w = L.Wave(shape, step, L.GRID_FP32)
+    w.set(psi)
+    f, p = L.Functional(model, w, 2, 4), L.CField(shape, step, L.GRID_FP32)
+    f.potential(p)
+    want = o.potential(psi)
+    assert np.abs(p.get() - want).max() <= 2e-5 * np.abs(want).max()
+    p.free(), f.free(), w.free()
