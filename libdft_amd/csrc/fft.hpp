@@ -12,9 +12,8 @@
 //  * y / x passes work on column tiles of the half spectrum
 //    [nx][ny][nz/2+1] (or of a full complex field for the propagator).
 //  * The x pass of a convolution transforms forward, forms
-//    out(k) = sum_t s_t K_t(k) D_t(k) in_t(k), with K_t a real kernel
-//    spectrum and D_t = i sin(k_d h)/h, the symbol of the periodic central
-//    difference, and transforms back (the x-middle pass of ot_fused.hpp).
+//    out(k) = sum_t s_t K_t(k) in_t(k), with K_t a real kernel spectrum, and
+//    transforms back (the x-middle pass of ot_fused.hpp).
 // Twiddles are computed in FP64 on the host; FP32 carries each as a rounded
 // value plus its residual.  Forward transforms are unnormalised (e^{-i}).
 #pragma once

@@ -4,19 +4,20 @@
 // Schedule of one full-OT potential (PLAIN|KC|BACKFLOW), src/ot.c:314-991:
 //   P1   psi -> rho, v_d, q_d = rho v_d, q4 = rho v^2           (one stencil pass)
 //   F1   r2c {rho, q_x, q_y, q_z, q4}
-//   I1   c2r {Pi*rho, F*rho, dF_d*rho (3), U*rho, U*q_d (3), U*q4}
+//   I1   c2r {Pi*rho, F*rho, U*rho, U*q_d (3), U*q4}
 //   P2   local terms, Q = (c2 rhobar + c3 rhobar^2) rho, G_d = d_d rho (1 - F*rho/rho_0s),
 //        BF real part, W_d = v_d A - B_d, (d_d rho/(rho+eps)) W_d
 //   F2   r2c {Q, G_x, G_y, G_z}
-//   I2   c2r {J_d = F*G_d (3)} (unfused; fused: and T1 = F*sum_d d_d G_d = sum_d d_d J_d)
-//   P3   H = sum_d d_d rho J_d, KC terms 1 and 3, BF sum_d d_d W_d
+//   I2   c2r {J_d = F*G_d (3)}
+//   P3   H = sum_d d_d rho J_d, KC term 1 (F*sum_d d_d G_d = sum_d d_d J_d) and
+//        term 3 (dF_d*rho = d_d (F*rho)), BF sum_d d_d W_d
 //   F3   r2c {H}
 //   I3   c2r {V_LJ*rho + Pi*Q + k23 c F*H}  (all linear terms summed in k space)
 //   P4   V += ...
-// i.e. 10 forward + 15 inverse real 3-D transforms, against 34 in the
-// reference.  The derivative kernels dF_d are never stored: their spectra
-// are F^ * i sin(k_d h)/h, the symbol of the periodic central difference
-// the reference applies to F before transforming (src/ot.c:196).
+// i.e. 10 forward + 11 inverse real 3-D transforms, against 34 in the
+// reference.  The derivative kernels dF_d are not built: the reference applies the
+// periodic central difference to F before transforming (src/ot.c:196), so a
+// convolution with dF_d is that difference of the convolution with F.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -1214,8 +1215,9 @@ template <typename C> fused::MidProg j_program(C *const *g, C *const *j, double 
 // it.  Schedule (stage kernels in ot_fused.hpp):
 //   zA, y, xconv{Pi, F, U products}, y^-1, zAB, y, [xconv{J_d}, y^-1, zBC, y],
 //   xconv{V_LJ + Pi Q + k23 c F H}, y^-1, zC
-// 7 + 5 forward and 7 + 3 + 1 inverse real 3-D transforms for full OT, with
-// all pointwise stages inside the z passes.
+// 5 + 4 + 1 forward and 7 + 3 + 1 inverse real 3-D transforms for full OT (6 + 3 + 1
+// inverse where U*q4 is summed with the linear terms), with all pointwise stages
+// inside the z passes.
 struct StepIn {
   const void *vext;   // real field or null
   double mu;
@@ -1301,10 +1303,12 @@ void fused_impl(dft_ot_functional *otf, const cplx<T> *psi, double wf_mass, T *r
   const bool HB = BF && pw.bfhd;
   // Re V_BF holds C = U*q4 linearly, -m/2 c_bf C, unless it is clamped or multiplied
   // by the switch's d(G rho)/d rho: then C joins the linear terms that stage C sums
-  // in k space and its inverse transform is saved (256^3: 2135 -> 2122 us per FP32
-  // step, 4204 -> 4090 FP64).  On small grids the longer chain of the summing
-  // pass costs as much as is saved (128^3 FP32: 722 and 724 us; 32x32x64: 92.0 and
-  // 92.8).
+  // in k space and its inverse transform is saved.  On small grids the longer chain
+  // of the summing pass costs as much as is saved.  Time of a step without the sum over
+  // that with it, full model (backflow alone is alike), FP32 and FP64: up to 2^21
+  // points 0.975 to 1.010, 0.994 in the mean (64^3 1.005, 0.992; 128^3 1.009, 1.002;
+  // 256x128x64 0.992, 0.986); at 2^22 1.006, 1.014 (128x128x256) and 0.993, 1.004
+  // (256x128x128); at 2^23 1.008-1.021, 1.011-1.021; 256^3 1.027, 1.023.
   const bool csum = BF && !HB && !pw.clamp_bf && n > ((int64_t)1 << 21);
   const int nA = BF ? (HB ? 6 : 5) : 1;
   fused::Ptrs8 oA{};
@@ -2692,8 +2696,7 @@ dft_ot_functional *dft_ot_alloc(INT model, wf *gwf, INT min_substeps, INT max_su
   bool ok = true;
   for (int i = 0; i < NSLOT && ok; ++i) ok = (d->slot[i] = dmalloc(es * d->slot_elems)) != nullptr;
   for (int i = 0; i < 4 && ok; ++i) ok = (d->kern[i] = dmalloc(es * nh)) != nullptr;
-  // the step's potential and the predictor's potential (complex fields), and
-  // the x-middle programs of the fused schedule
+  // the step's potential and the predictor's potential (complex fields)
   if (ok) ok = (d->phase = dmalloc(2 * es * d->n)) != nullptr;
   if (ok) ok = (d->vsave = dmalloc(2 * es * d->n)) != nullptr;
   if (ok)
@@ -2729,7 +2732,7 @@ dft_ot_functional *dft_ot_alloc(INT model, wf *gwf, INT min_substeps, INT max_su
   otf->spherical_avg = spectral_handle(otf, K_SA, "OT Sph. average");
   if (model & DFT_OT_KC) otf->gaussian_tf = spectral_handle(otf, K_F, "OT KC Gauss TF");
   if (model & DFT_OT_BACKFLOW) otf->backflow_pot = spectral_handle(otf, K_U, "OT Backflow");
-  // x/y/z derivatives of F are applied in k space (i sin(k h)/h F^), not stored
+  // convolutions with the x/y/z derivatives of F are differences of those with F
   otf->gaussian_x_tf = otf->gaussian_y_tf = otf->gaussian_z_tf = nullptr;
 
   int save = grid_get_precision();

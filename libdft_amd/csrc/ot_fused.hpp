@@ -368,14 +368,18 @@ template <int COLS> __device__ __forceinline__ MidCol mid_col(int ny, int P, int
 }
 
 // Spectra are [nx][ny][PP] (P values per row) after the y pass; the x line
-// (ky = o, kz) has stride ny*PP.  The program, a kernel argument, is indexed
-// uniformly over the block (scalar loads) and runs one output per block:
-// out_m = F_x^-1 sum_t c_t F_x in_t over the terms of output m.  An input shared by several outputs is read once
-// per output; the outputs of one column tile are consecutive logical blocks
-// on one XCD, so those re-reads mostly hit that XCD's L2.  Holding one line
-// (16 points per thread) plus an accumulator keeps the register count low
-// enough for four waves per SIMD.  Single-term outputs take 32 columns per
-// block (256-byte row segments in FP32), the accumulating form 16.
+// (ky = o, kz) has stride ny*PP.  The arguments are indexed uniformly over the
+// block (scalar loads); one output per block:
+// out_m = F_x^-1 sum_t c_t F_x in_t over the terms of output m.  An input shared by
+// several outputs is read once per output; the outputs of one column tile are
+// consecutive logical blocks on one XCD, so those re-reads mostly hit that XCD's
+// L2.  Bound by the movement of the x columns: without the transform the
+// single-term FP32 outputs take 29 us per launch for 31 at 128^3, 170 for 183 at
+// 256^3, 1565 for 1593 at 512^3 (profiler's times).  A block holds its lines, up
+// to 16 points per thread: 4 waves per SIMD at 256 points FP32; the
+// accumulating form adds an accumulator and the next term and runs at 2.
+// Single-term outputs take 32 columns per block (256-byte row segments in FP32),
+// the accumulating form 16.
 // DFT_XCONV1_EM / DFT_XCONV1_COLS set that geometry for the single-term form,
 // DFT_XCONV_EM / DFT_XCONV_COLS for the accumulating one; DFT_XCONV_MINB asks
 // the register allocator for that many waves per SIMD (0: no request).
@@ -407,7 +411,7 @@ template <int COLS> __device__ __forceinline__ MidCol mid_col(int ny, int P, int
 #ifndef DFT_XCONV_MINB64
 #define DFT_XCONV_MINB64 2
 #endif
-// (N = 512 takes 16 points per thread and 8 columns: 45 KB of LDS in FP32 and 80
+// (N = 512 takes 8 columns: 45 KB of LDS in FP32 and 80
 // in FP64, so that 3 or 2 blocks share a CU and one's barriers overlap another's
 // loads; 16 columns fill it with one.  512^3 FP32 step: single-term outputs 2078
 // -> 1491 us per launch, sums 1012 -> 976; FP64 potential at 512x64x128 955 ->
