@@ -845,8 +845,8 @@ enum Kern { K_LJ = 0, K_SA = 1, K_F = 2, K_U = 3 };
 enum Slot {
   SP0, SP1, SP2, SP3, SP4, SP5,             // spectra (SP5: rho~ of the HD / HD2 backflow switch)
   VX, VY, VZ, QX, QY, QZ, Q4,               // velocities, products
-  RB, RT, PX, SA_, SBX, SBY, SBZ, SC,       // first inverse batch (PX: LJ*rho of the energy)
-  TMP0, TMP1, TMP2, TMP3, TMP4, TMP5, TMP6, TMP7,
+  RB, RT, PX, PY, PZ, SA_, SBX, SBY, SBZ, SC,  // first inverse batch
+  TMP0, TMP1, TMP2, TMP3, TMP4, TMP5, TMP6, TMP7, TMP8, TMP9,
   VRE, VIM, WX, WY, WZ, SH,
   NSLOT
 };
