@@ -274,7 +274,7 @@ __device__ __forceinline__ double2 twmul_d(double2 a, const cplx<T> *tw, int idx
 // stage of the long FP32 lines, whose FP64 registers otherwise cost waves: the
 // stage's LDS reads are all hoisted.  FP32 at 256 points: the kinetic pass spills
 // 132 bytes per lane (104 us at 256^3 against 76), a single-term x-middle output
-// takes 222 VGPRs instead of 116 (127 us against 103 per launch of 2-3 outputs);
+// takes 222 VGPRs instead of 118 (127 us against 103 per launch of 2-3 outputs);
 // at 512 points 112 instead of 73 (512x128x128: 72 against 65).  Not for shorter
 // lines nor for FP64, where as many waves fit either way and the fence only
 // delays the reads: FP64 64^3 single-term output 6.2 -> 5.9 us; FP32 128^3 kinetic pass
